@@ -1,0 +1,789 @@
+/*
+ * uocr_gemm_tile.hip - the large-tile MFMA GEMM of the prompt prefill, the
+ * operator API and the vision linears on gfx950 (replaces the reference's
+ * tiled GEMMs gemm_q4.metal / gemm_q8.metal where a grid of large tiles fills
+ * the chip).
+ */
+#include "uocr_gemm.h"
+
+#define NA 3u  /* activation tiles in LDS: two steps of loads in flight */
+
+namespace {
+
+/* Waits until at most N of the wavefront's vector memory operations are in
+ * flight and its LDS reads are done, then for the block's other wavefronts. */
+template <int N>
+__device__ __forceinline__ void wait_barrier() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
+__device__ __forceinline__ u32 uni(u32 v) {
+    return (u32)__builtin_amdgcn_readfirstlane((int)v);
+}
+
+template <typename T>
+__device__ __forceinline__ T *uni(T *p) {
+    const uint64_t v = (uint64_t)p;
+    return (T *)(((uint64_t)uni((u32)(v >> 32)) << 32) | uni((u32)v));
+}
+
+/* 16 bytes per lane from base + voff straight into LDS at lds + 16 lane.  In
+ * inline assembly because the compiler's own LDS-direct load makes every later
+ * LDS read wait for all of them; wait_barrier counts them instead. */
+__device__ __forceinline__ void lds_load16(const void *base, u32 voff, u32 lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                 :
+                 : "v"(voff), "s"(uni(base)), "s"(lds)
+                 : "memory");
+}
+
+/* The block's tile.  Blocks go to the 8 XCDs in turn; with by_row or by_col
+ * each XCD takes a contiguous run of row tiles (of column tiles) instead, so
+ * that its L2 fetches only its share of the activations (of the weights). */
+__device__ __forceinline__ bool tile_of(u32 order, u32 nx, u32 ny, u32 &bx, u32 &by) {
+    const u32 id = blockIdx.x;
+    if (order == GO_PLAIN) {
+        bx = id % nx;
+        by = id / nx;
+        return by < ny;
+    }
+    const u32 total = nx * ny, q = total / 8u, rem = total % 8u, x = id % 8u, slot = id / 8u;
+    if (slot >= q + (x < rem ? 1u : 0u)) return false;
+    const u32 l = x * q + min(x, rem) + slot;
+    if (order == GO_BY_ROW) {
+        bx = l / ny;
+        by = l % ny;
+    } else {
+        bx = l % nx;
+        by = l / nx;
+    }
+    return true;
+}
+
+/* Groups of 64 columns in the 128 bytes of a weight row. */
+template <int QT>
+constexpr int groups_per_line() {
+    return QT == 4 ? 4 : (QT == 3 ? 2 : 1);
+}
+
+__device__ __forceinline__ float vision_act(float v, u32 act) {
+    return act == UOCR_VISION_ACT_QUICKGELU ? quick_gelu(v) : (act == UOCR_VISION_ACT_GELU_ERF ? gelu_erf_as(v) : v);
+}
+
+/* LDS of one K group: the activation tiles and its wavefronts' weight lines. */
+template <int RT, int WN>
+constexpr u32 group_lds_bytes() {
+    return NA * 32u * RT * 128u + WN * 8192u;
+}
+
+template <int RT, int WN, int WK>
+constexpr u32 tile_lds_bytes(bool rope) {
+    constexpr u32 main = WK * group_lds_bytes<RT, WN>(), stage = 32u * RT * (64u * WN + 8u) * 2u;
+    return rope && stage > main ? stage : main;
+}
+
+template <int QT, int EPI, bool GROUPED, bool PACKED, int RT, int WN, int WK>
+__device__ __forceinline__ void tile_body(const GemmArgs &p, u32 bx, u32 by, uint8_t *sm, const RopeDst &rd) {
+    constexpr int NG = groups_per_line<QT>();
+    constexpr bool SW = EPI == GE_SWIGLU;
+    constexpr u32 CW = SW ? 32u : 64u; /* output columns of a wavefront */
+    constexpr u32 ROWS = 32u * RT, ABUF = ROWS * 128u, TT = 64u * WN * WK;
+    constexpr int AL = RT * 4 / WN; /* activation loads of a wavefront per step */
+    static_assert(AL * WN == RT * 4, "activation rows");
+    constexpr u32 RB = QT == 4 ? 32u : 64u; /* packed: bytes of a row's group */
+    const u32 t = threadIdx.x, lane = t & 63u, r = lane & 31u, h = lane >> 5;
+    const u32 wave = uni(t >> 6) % WN, kg = uni(t >> 6) / WN; /* column group, K group */
+    u32 e = 0, s0 = bx * ROWS, rows;
+    if (GROUPED) {
+        e = uni((u32)p.tile_e[bx]);
+        s0 = uni((u32)p.tile_s0[bx]);
+        rows = uni((u32)p.tile_s1[bx]) - s0;
+    } else {
+        rows = min(ROWS, p.M - s0);
+    }
+    const u32 K = p.K;
+    /* K group kg takes steps [ks, ks + NT) of its matrix; all groups run the
+     * same number of steps (NS) for the block's barriers */
+    const u32 NTA = K / 64u, NS = (NTA + WK - 1u) / WK, ks = min(kg * NS, NTA - 1u), NT = kg * NS < NTA ? min(NS, NTA - ks) : 0u;
+    const u32 NCH = (NS + NG - 1u) / NG;
+    const u32 rowb = QT == 4 ? K / 2u : (QT == 3 ? K : 2u * K);
+    const u32 n0 = by * WN * CW;
+    const uocr_qmat *W0 = &p.W[0];
+    u32 nbase = 0, nmax = p.N;
+    if (p.nseg != 0u) {
+        const u32 sg = n0 / p.nseg;
+        W0 = &p.W[sg];
+        nbase = sg * p.nseg;
+        nmax = p.nseg;
+    }
+    const uint8_t *w[2];
+    const unsigned short *sc[2];
+    u32 cb[2]; /* first weight row of the wavefront's two column groups */
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const uocr_qmat &m = SW ? p.W[j] : *W0;
+        w[j] = (const uint8_t *)m.w + (GROUPED ? e * p.w_stride : 0);
+        sc[j] = (const unsigned short *)m.s + (GROUPED ? e * p.s_stride : 0);
+        cb[j] = n0 - nbase + CW * wave + (SW ? 0u : 32u * j);
+    }
+
+    /* activation staging: this lane's rows, 16-byte piece (lane % 8) ^ (row /
+     * 2 % 8) of the row's 128 bytes; two rows span the 64 banks, so this
+     * swizzle keeps the reads free of bank conflicts (16 reads by 4 wavefronts
+     * 118 ns; by row % 8, two rows to a bank, 230 ns).  The wavefront loads RT
+     * groups of 8 rows; pc(i): the piece's offset in group i */
+    auto pc = [&](u32 i) { return 16u * ((lane & 7u) ^ (lane >> 4)) ^ (64u * (i & 1u)); };
+    u32 va[AL];
+#pragma unroll
+    for (int q = 0; q < AL; ++q) {
+        const u32 rr = min(8u * (AL * wave + q) + (lane >> 3), rows - 1u);
+        const u32 ar = GROUPED ? (u32)p.a_idx[s0 + rr] : s0 + rr;
+        va[q] = ar * p.lda * 2u + pc(AL * wave + q);
+    }
+    const u32 lds0 = uni((u32)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)sm);
+    uint8_t *gsm = sm + kg * group_lds_bytes<RT, WN>();
+    const u32 ldsg = lds0 + kg * group_lds_bytes<RT, WN>(), lds_a = ldsg + wave * AL * 1024u, lds_b = ldsg + NA * ABUF + wave * 8192u;
+    const uint8_t *Ab = (const uint8_t *)p.A + (size_t)ks * 128u;
+    auto issue_a = [&](u32 s, u32 buf, int q) { lds_load16(Ab + (size_t)s * 128u, va[q], lds_a + buf + 1024u * q); };
+    /* weight staging: the wavefront's own 64 rows, a line of 128 bytes (NG
+     * groups) of each; pieces past the row's end re-read its last 16 bytes */
+    u32 vb[PACKED ? 1 : 8];
+    const uint8_t *pb[2];
+    const u32 room = rowb - ks * (rowb / NTA) - 16u; /* a row's last 16 bytes, from the group's first */
+    if constexpr (PACKED) {
+        vb[0] = 16u * lane;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) pb[j] = w[j] + (size_t)min(cb[j] / 32u, nmax / 32u - 1u) * NTA * (32u * RB) + (size_t)ks * (32u * RB);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) vb[i] = min(cb[i >> 2] + 8u * (i & 3) + (lane >> 3), nmax - 1u) * rowb;
+        pb[0] = w[0] + ks * (rowb / NTA);
+        pb[1] = w[1] + ks * (rowb / NTA);
+    }
+    auto issue_b = [&](u32 c, int i) {
+        if constexpr (PACKED) {
+            const u32 cc = min(c, (NTA - ks - 1u) / NG), left = (NTA - ks - cc * NG) * 32u * RB, o = 1024u * (i & 3); /* left: bytes to the run's end */
+            lds_load16(pb[i >> 2] + (size_t)cc * 4096u + (o < left ? o : 0u), vb[0], lds_b + 1024u * i);
+        } else {
+            lds_load16(pb[i >> 2], vb[i] + min(c * 128u + pc(i & 1), room), lds_b + 1024u * i);
+        }
+    };
+    u32 sn[2][NG];
+    const unsigned short *srow[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        srow[j] = sc[j] + (size_t)min(cb[j] + r, nmax - 1u) * NTA + ks;
+#pragma unroll
+        for (int g = 0; g < NG; ++g) sn[j][g] = 0u;
+    }
+    auto load_s = [&](u32 c) {
+        if constexpr (QT != 1) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int g = 0; g < NG; ++g) sn[j][g] = srow[j][min(c * NG + g, NTA - ks - 1u)];
+        }
+    };
+
+    f32x16 acc[RT][2];
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int k = 0; k < 16; ++k) acc[i][j][k] = 0.0f;
+
+    /* LDS offsets of this lane's activation operand of substep i (row r of a
+     * 32-row tile) */
+    u32 ao[4];
+#pragma unroll
+    for (u32 i = 0; i < 4; ++i) ao[i] = r * 128u + 16u * ((b_koff<QT>(i, h) / 8u) ^ ((r >> 1) & 7u));
+    const uint8_t *bsm = gsm + NA * ABUF + wave * 8192u;
+
+    load_s(0);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) issue_b(0, i);
+#pragma unroll
+    for (int q = 0; q < AL; ++q) issue_a(0, 0u, q);
+    const u32 sl = max(NT, 1u) - 1u; /* the group's last step */
+#pragma unroll
+    for (int q = 0; q < AL; ++q) issue_a(min(1u, sl), ABUF, q);
+    u32 cur = 0, nxt = 2u * ABUF; /* LDS offsets of step s's activations and of step s + 2's */
+    u32 br[2][16], sv[2][NG];
+    for (u32 c = 0; c < NCH; ++c) {
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            const u32 s = c * NG + g;
+            if (g > 0 && s >= NS) break;
+            /* A step issues its share of line c + 1, then the activations of
+             * step s + 2.  Needed here: the activations of step s, issued in
+             * step s - 2, and at g = 0 line c, older than step s - 1's
+             * activations; in flight may stay all of step s - 1's loads (at g
+             * = 0 only its activations). */
+            constexpr int NB = NG == 4 ? 4 : 8, BS = 8 / NB; /* loads of a line per step, in the line's first BS steps */
+            if (g >= 1 && g <= BS && c + 1u < NCH) wait_barrier<AL + NB>();
+            else wait_barrier<AL>();
+            if (g == 0) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int q = 0; q < NG; ++q) {
+                        asm volatile("" : "+v"(sn[j][q])); /* the scales' wait belongs here, before later loads */
+                        sv[j][q] = sn[j][q];
+                    }
+                load_s(min(c + 1u, NCH - 1u));
+            }
+            if (g == 0) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        u32 o;
+                        if constexpr (PACKED) {
+                            o = QT == 4 ? 1024u * q + 16u * lane : 2048u * (q >> 1) + 32u * lane + 16u * (q & 1);
+                        } else {
+                            const u32 ch = QT == 4 ? 2u * q + h : (QT == 3 ? 4u * (q >> 1) + 2u * h + (q & 1) : 4u * h + q);
+                            o = r * 128u + 16u * (ch ^ ((r >> 1) & 7u));
+                        }
+                        const uint4 x = *(const uint4 *)(bsm + 4096u * j + o);
+                        br[j][4 * q] = x.x;
+                        br[j][4 * q + 1] = x.y;
+                        br[j][4 * q + 2] = x.z;
+                        br[j][4 * q + 3] = x.w;
+                    }
+            }
+            if (WK == 1 || s < NT) {
+            const uint8_t *abuf = gsm + cur;
+            U4H8 a[2][RT]; /* substep i's operands and the next one's */
+#pragma unroll
+            for (int k = 0; k < RT; ++k) a[0][k].u = *(const uint4 *)(abuf + ao[0] + 4096u * k);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (i < 3) {
+#pragma unroll
+                    for (int k = 0; k < RT; ++k) a[(i + 1) & 1][k].u = *(const uint4 *)(abuf + ao[i < 3 ? i + 1 : 3] + 4096u * k);
+                }
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    h16x8 wv;
+                    if (QT == 4) wv = dequant_q4(br[j][4 * g + 2 * (i & 1)], br[j][4 * g + 2 * (i & 1) + 1], (i & 2) != 0, sv[j][g]);
+                    else if (QT == 3) wv = dequant_q8(br[j][(8 * g + 2 * i) & 15], br[j][(8 * g + 2 * i + 1) & 15], sv[j][g]);
+                    else wv = operand_f16(br[j][4 * i], br[j][4 * i + 1], br[j][4 * i + 2], br[j][4 * i + 3]);
+#pragma unroll
+                    for (int k = 0; k < RT; ++k) acc[k][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wv, a[i & 1][k].v, acc[k][j], 0, 0, 0);
+                    /* the loads spread over the step, between its MFMAs: issued
+                     * together they fill the memory pipe's queue and the
+                     * wavefront's MFMAs wait behind them */
+                    const int slot = 2 * i + j;
+                    if (g < BS && slot >= 1 && slot <= 4 && c + 1u < NCH) {
+                        /* the line is in registers: its LDS takes the next one */
+                        if (slot == 1) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+                        for (int x = 0; x < NB / 4; ++x) issue_b(c + 1u, NB * g + NB / 4 * (slot - 1) + x);
+                    }
+                    /* (past the end the last step again, which nothing reads:
+                     * the count of loads in flight stays the same) */
+                    if (slot >= 4) {
+#pragma unroll
+                        for (int q = 0; q < AL; ++q)
+                            if (4 + q * 4 / AL == slot) issue_a(min(s + 2u, sl), nxt, q);
+                    }
+                }
+            }
+            }
+            nxt = cur;
+            cur = cur + ABUF == NA * ABUF ? 0u : cur + ABUF;
+        }
+    }
+
+    if constexpr (WK > 1) {
+        /* the K groups' sums, added in order by group 0 */
+        wait_barrier<0>();
+        if (kg > 0) {
+            uint8_t *dst = sm + ((kg - 1u) * WN + wave) * (RT * 8192u) + 16u * lane;
+#pragma unroll
+            for (int k = 0; k < RT; ++k)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        *(float4 *)(dst + ((k * 2 + j) * 4 + q) * 1024u) =
+                            make_float4(acc[k][j][4 * q], acc[k][j][4 * q + 1], acc[k][j][4 * q + 2], acc[k][j][4 * q + 3]);
+        }
+        __syncthreads();
+        if (kg == 0) {
+            for (u32 g = 1; g < WK; ++g) {
+                const uint8_t *src = sm + ((g - 1u) * WN + wave) * (RT * 8192u) + 16u * lane;
+#pragma unroll
+                for (int k = 0; k < RT; ++k)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            const float4 v = *(const float4 *)(src + ((k * 2 + j) * 4 + q) * 1024u);
+                            acc[k][j][4 * q] += v.x;
+                            acc[k][j][4 * q + 1] += v.y;
+                            acc[k][j][4 * q + 2] += v.z;
+                            acc[k][j][4 * q + 3] += v.w;
+                        }
+            }
+        }
+    }
+    /* Lane l holds row l % 32 of each 32-row tile and, of column group j,
+     * columns 8q + 4 (l / 32) + 0..3 in elements 4q..4q+3. */
+    if constexpr (EPI == GE_ROPE) {
+        constexpr u32 LD = 64u * WN + 8u; /* padded row (halves) */
+        h16 *tile = (h16 *)sm;
+        wait_barrier<0>();
+#pragma unroll
+        for (int k = 0; k < RT; ++k)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    union {
+                        h16 x[4];
+                        uint2 u;
+                    } o;
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) o.x[x] = (h16)acc[k][j][4 * q + x];
+                    *(uint2 *)(tile + (32u * k + r) * LD + 64u * wave + 32u * j + 8u * q + 4u * h) = o.u;
+                }
+        __syncthreads();
+        const u32 seg = n0 / p.nseg, h0 = (n0 - seg * p.nseg) / 128u;
+        /* 8 pairs (d, d + 64) of one head and row per thread and turn */
+        for (u32 it = t; it < rows * 4u * WN; it += TT) {
+            const u32 row = it / (4u * WN), hd = (it / 8u) % (WN / 2u), d = 8u * (it % 8u), tok = s0 + row;
+            U4H8 a, b;
+            a.u = *(const uint4 *)(tile + row * LD + 128u * hd + d);
+            b.u = *(const uint4 *)(tile + row * LD + 128u * hd + d + 64u);
+            h16 *dst = seg == 0u ? rd.q + (size_t)tok * UOCR_K_HIDDEN + (h0 + hd) * 128u + d
+                                 : (seg == 1u ? rd.k : rd.v) + ((size_t)(h0 + hd) * rd.cap + tok) * 128u + d;
+            if (seg != 2u) {
+                const float4 *cs = (const float4 *)(rd.cs + (size_t)tok * 64u + d);
+                U4H8 x, y;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const float4 f = cs[q];
+                    const float a0 = (float)a.h[2 * q], b0 = (float)b.h[2 * q], a1 = (float)a.h[2 * q + 1], b1 = (float)b.h[2 * q + 1];
+                    x.h[2 * q] = (h16)(a0 * f.x - b0 * f.y);
+                    y.h[2 * q] = (h16)(a0 * f.y + b0 * f.x);
+                    x.h[2 * q + 1] = (h16)(a1 * f.z - b1 * f.w);
+                    y.h[2 * q + 1] = (h16)(a1 * f.w + b1 * f.z);
+                }
+                a = x;
+                b = y;
+            }
+            *(uint4 *)dst = a.u;
+            *(uint4 *)(dst + 64) = b.u;
+        }
+        return;
+    }
+    /* Through LDS, so that the stores (and the residual's loads) cover whole
+     * rows of the tile: 16-byte pieces, swizzled by row.  Stored from the
+     * registers, 8 bytes of 32 rows at a time, every piece was a write request
+     * of its own. */
+    constexpr bool F32O = EPI == GE_F32;
+    constexpr u32 CPP = F32O ? 4u : 8u;        /* columns per piece */
+    constexpr u32 CH = WN * CW / CPP;          /* pieces per row */
+    constexpr int PASS_RT = F32O && RT > 2 ? 2 : RT; /* 32-row tiles per pass */
+    static_assert(PASS_RT * 32u * CH * 16u <= tile_lds_bytes<RT, WN, WK>(false), "staging fits");
+    const u32 ch = t % CH, col = n0 + CPP * ch; /* the piece this thread moves, in rows t / CH, + TT / CH, .. */
+#pragma unroll
+    for (int k0 = 0; k0 < RT; k0 += PASS_RT) {
+        wait_barrier<0>();
+        if (EPI == GE_F16 && p.res != nullptr) {
+            /* the residual's tile into the pieces' places; columns past N and
+             * rows past the tile re-read valid ones */
+            constexpr u32 RPL = 64u / CH; /* rows per load */
+#pragma unroll 4
+            for (u32 q = uni(t >> 6); q < ROWS / RPL; q += WN * WK) {
+                const u32 row = q * RPL + lane / CH;
+                const u32 c = min(n0 + CPP * ((lane % CH) ^ (row % CH)), p.N - CPP);
+                const u32 rr = min(row, rows - 1u);
+                const size_t orow = GROUPED ? (size_t)p.o_idx[s0 + rr] : (size_t)(s0 + rr);
+                lds_load16(p.res, (u32)((orow * p.ldr + c) * 2u), lds0 + q * 1024u);
+            }
+            wait_barrier<0>();
+        }
+        if (WK == 1 || kg == 0) {
+#pragma unroll
+        for (int j = 0; j < (SW ? 1 : 2); ++j) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                float bias[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+                if constexpr (EPI == GE_VISION) {
+                    union {
+                        h16 x[4];
+                        uint2 u;
+                    } b;
+                    b.u = *(const uint2 *)(p.bias + min(n0 + CW * wave + 32u * j + 8u * q + 4u * h, p.N - 4u));
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) bias[x] = (float)b.x[x];
+                }
+                const u32 pcs = F32O ? 16u * wave + 8u * j + 2u * q + h : (SW ? 4u * wave + q : 8u * wave + 4u * j + q);
+#pragma unroll
+                for (int k = 0; k < PASS_RT; ++k) {
+                    uint8_t *at = sm + ((32u * k + r) * CH + (pcs ^ (r % CH))) * 16u + (F32O ? 0u : 8u * h);
+                    float v[4];
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) {
+                        v[x] = acc[k0 + k][j][4 * q + x];
+                        if (SW) v[x] = silu_p(v[x]) * acc[k0 + k][1][4 * q + x];
+                        if constexpr (EPI == GE_VISION) v[x] = vision_act(v[x] + bias[x], p.act);
+                    }
+                    if constexpr (F32O) {
+                        *(float4 *)at = make_float4(v[0], v[1], v[2], v[3]);
+                    } else {
+                        union {
+                            h16 x[4];
+                            uint2 u;
+                        } o;
+                        if (EPI == GE_F16 && p.res != nullptr) {
+                            o.u = *(const uint2 *)at;
+#pragma unroll
+                            for (int x = 0; x < 4; ++x) v[x] += (float)o.x[x];
+                        }
+#pragma unroll
+                        for (int x = 0; x < 4; ++x) o.x[x] = (h16)v[x];
+                        *(uint2 *)at = o.u;
+                    }
+                }
+            }
+        }
+        }
+        __syncthreads();
+        if (col < p.N) {
+            uint8_t *out = (uint8_t *)p.out;
+            u32 c = col, ld = p.ldo;
+            if (EPI == GE_VISION && p.split != 0u) {
+                const u32 pj = col / p.split;
+                out = (uint8_t *)(pj == 0u ? p.out : (pj == 1u ? p.out1 : p.out2));
+                c = col - pj * p.split;
+                ld = p.split;
+            }
+#pragma unroll 4
+            for (u32 row = t / CH; row < PASS_RT * 32u; row += TT / CH) {
+                const u32 rr = 32u * k0 + row;
+                if (rr >= rows) break;
+                const size_t orow = GROUPED ? (size_t)p.o_idx[s0 + rr] : (size_t)(s0 + rr);
+                const uint4 v = *(const uint4 *)(sm + (row * CH + (ch ^ (row % CH % 32u))) * 16u);
+                *(uint4 *)(out + (orow * ld + c) * (F32O ? 4u : 2u)) = v;
+            }
+        }
+    }
+}
+
+template <int QT, int EPI, bool GROUPED, bool PACKED, int RT, int WN, int WK>
+__global__ __launch_bounds__(64 * WN * WK, 2) void k_gemm_tile(GemmArgs p) {
+    __shared__ __attribute__((aligned(1024))) uint8_t sm[tile_lds_bytes<RT, WN, WK>(false)];
+    u32 bx, by;
+    if (!tile_of(p.order, GROUPED ? (u32)*p.ntiles : p.nx, p.ny, bx, by)) return;
+    tile_body<QT, EPI, GROUPED, PACKED, RT, WN, WK>(p, bx, by, sm, RopeDst{});
+}
+
+/* ---- narrow tiles, K split over the block's wavefronts ---------------------- */
+
+#define KS_WAVES 8u                     /* wavefronts of a block at most */
+#define KS_PLANE (8u * 1040u)           /* bytes of a wavefront's 32 x 64 partials: 8 pieces of 64 float4, padded */
+
+template <int QT, int EPI, bool GROUPED, bool PACKED>
+__global__ __launch_bounds__(64u * KS_WAVES) void k_gemm_ksplit(GemmArgs p) {
+    constexpr int NG = groups_per_line<QT>();
+    constexpr bool SW = EPI == GE_SWIGLU;
+    constexpr int RT = 1; /* 32-row tiles (2 measured slower at 32 to 4096 rows) */
+    constexpr u32 CW = SW ? 32u : 64u, ROWS = 32u * RT, RB = QT == 4 ? 32u : 64u;
+    extern __shared__ __attribute__((aligned(16))) uint8_t ksm[];
+    const u32 t = threadIdx.x, lane = t & 63u, wave = uni(t >> 6), r = lane & 31u, h = lane >> 5, nw = blockDim.x / 64u;
+    u32 bx, by;
+    if (!tile_of(p.order, GROUPED ? (u32)*p.ntiles : p.nx, p.ny, bx, by)) return;
+    const u32 n0 = by * CW;
+    u32 e = 0, s0 = bx * ROWS, rows;
+    if (GROUPED) {
+        e = uni((u32)p.tile_e[bx]);
+        s0 = uni((u32)p.tile_s0[bx]);
+        rows = uni((u32)p.tile_s1[bx]) - s0;
+    } else {
+        rows = min(ROWS, p.M - s0);
+    }
+    const u32 K = p.K, NT = K / 64u, NCH = (NT + NG - 1u) / NG;
+    const u32 rowb = QT == 4 ? K / 2u : (QT == 3 ? K : 2u * K);
+    const uint8_t *pb[2];
+    const unsigned short *srow[2];
+    u32 vb[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const uocr_qmat &m = SW ? p.W[j] : p.W[0];
+        const u32 cb = n0 + (SW ? 0u : 32u * j), row = min(cb + r, p.N - 1u);
+        pb[j] = (const uint8_t *)m.w + (GROUPED ? e * p.w_stride : 0);
+        if (PACKED) pb[j] += (size_t)min(cb / 32u, p.N / 32u - 1u) * NT * (32u * RB);
+        vb[j] = PACKED ? 0u : row * rowb;
+        srow[j] = (const unsigned short *)m.s + (GROUPED ? e * p.s_stride : 0) + (size_t)row * NT;
+    }
+    u32 va[RT];
+#pragma unroll
+    for (int k = 0; k < RT; ++k) {
+        const u32 rr = min(32u * k + r, rows - 1u), ar = GROUPED ? (u32)p.a_idx[s0 + rr] : s0 + rr;
+        va[k] = ar * p.lda * 2u + 2u * b_koff<QT>(0u, h);
+    }
+    u32 bn[2][16], sn[2][NG], bc[2][16], sc[2][NG];
+    U4H8 an[4][RT], ac[4][RT];
+    /* line c of the lane's two weight rows: its half of every group (past the
+     * row's end the last piece again) */
+    auto load_b = [&](u32 c) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+#pragma unroll
+            for (u32 q = 0; q < 4; ++q) {
+                uint4 x;
+                if constexpr (PACKED) {
+                    const u32 left = (NT - c * NG) * 32u * RB, o = QT == 4 ? 1024u * q : 2048u * (q >> 1);
+                    x = *(const uint4 *)(pb[j] + (size_t)c * 4096u + (o < left ? o : 0u) + (QT == 4 ? 16u * lane : 32u * lane + 16u * (q & 1u)));
+                } else {
+                    const u32 ch = QT == 4 ? 2u * q + h : (QT == 3 ? 4u * (q >> 1) + 2u * h + (q & 1) : 4u * h + q);
+                    x = *(const uint4 *)(pb[j] + (vb[j] + min(c * 128u + 16u * ch, rowb - 16u)));
+                }
+                bn[j][4 * q] = x.x;
+                bn[j][4 * q + 1] = x.y;
+                bn[j][4 * q + 2] = x.z;
+                bn[j][4 * q + 3] = x.w;
+            }
+            if constexpr (QT != 1) {
+#pragma unroll
+                for (int g = 0; g < NG; ++g) sn[j][g] = srow[j][min(c * NG + g, NT - 1u)];
+            }
+        }
+    };
+    auto load_a = [&](u32 s) {
+        const uint8_t *base = (const uint8_t *)p.A + (size_t)s * 128u;
+#pragma unroll
+        for (u32 i = 0; i < 4; ++i)
+#pragma unroll
+            for (int k = 0; k < RT; ++k) an[i][k].u = *(const uint4 *)(base + (va[k] + 2u * b_koff<QT>(i, 0u)));
+    };
+    f32x16 acc[RT][2];
+#pragma unroll
+    for (int k = 0; k < RT; ++k)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int x = 0; x < 16; ++x) acc[k][j][x] = 0.0f;
+
+    if (wave < NCH) {
+        load_b(wave);
+        load_a(wave * NG);
+    }
+    for (u32 c = wave; c < NCH; c += nw) {
+        const bool more = c + nw < NCH;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+#pragma unroll
+            for (int x = 0; x < 16; ++x) bc[j][x] = bn[j][x];
+#pragma unroll
+            for (int g = 0; g < NG; ++g) sc[j][g] = sn[j][g];
+        }
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            const u32 s = c * NG + g;
+            if (g > 0 && s >= NT) break;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int k = 0; k < RT; ++k) ac[i][k] = an[i][k];
+            if (g + 1 < NG) load_a(min(s + 1u, NT - 1u));
+            if (g == 0 && more) load_b(c + nw);
+            if (g + 1 == NG && more) load_a((c + nw) * NG);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    h16x8 wv;
+                    if (QT == 4) wv = dequant_q4(bc[j][4 * g + 2 * (i & 1)], bc[j][4 * g + 2 * (i & 1) + 1], (i & 2) != 0, sc[j][g]);
+                    else if (QT == 3) wv = dequant_q8(bc[j][(8 * g + 2 * i) & 15], bc[j][(8 * g + 2 * i + 1) & 15], sc[j][g]);
+                    else wv = operand_f16(bc[j][4 * i], bc[j][4 * i + 1], bc[j][4 * i + 2], bc[j][4 * i + 3]);
+#pragma unroll
+                    for (int k = 0; k < RT; ++k) acc[k][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wv, ac[i][k].v, acc[k][j], 0, 0, 0);
+                }
+            }
+        }
+    }
+
+    /* The wavefronts' partials are added in order, 8 columns of a row per
+     * thread and turn; 32 rows at a time.  Piece (j, q) of a plane: the four
+     * values of row r and half h at 16 (32 h + r). */
+    constexpr u32 CH = CW / 8u;
+#pragma unroll
+    for (int k = 0; k < RT; ++k) {
+        if (k > 0 && 32u * k >= rows) break;
+        if (k > 0) __syncthreads();
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                *(float4 *)(ksm + wave * KS_PLANE + (4u * j + q) * 1040u + 16u * lane) =
+                    make_float4(acc[k][j][4 * q], acc[k][j][4 * q + 1], acc[k][j][4 * q + 2], acc[k][j][4 * q + 3]);
+        __syncthreads();
+        for (u32 it = t; it < 32u * CH; it += blockDim.x) {
+            const u32 row = it / CH, pc = it % CH, rr = 32u * k + row, col = n0 + 8u * pc;
+            if (rr >= rows || col >= p.N) continue;
+            const size_t orow = GROUPED ? (size_t)p.o_idx[s0 + rr] : (size_t)(s0 + rr);
+            U4H8 rs;
+            if (EPI == GE_F16 && p.res != nullptr) rs.u = *(const uint4 *)(p.res + orow * p.ldr + col);
+            if (EPI == GE_VISION) rs.u = *(const uint4 *)(p.bias + col);
+            float v[8], u[8];
+            auto sum = [&](u32 piece, float (&o)[8]) {
+                const uint8_t *src = ksm + piece * 1040u + 16u * row;
+#pragma unroll
+                for (int x = 0; x < 8; ++x) o[x] = 0.0f;
+                for (u32 w = 0; w < nw; ++w) {
+                    const float4 a = *(const float4 *)(src + w * KS_PLANE), b = *(const float4 *)(src + w * KS_PLANE + 512u);
+                    o[0] += a.x;
+                    o[1] += a.y;
+                    o[2] += a.z;
+                    o[3] += a.w;
+                    o[4] += b.x;
+                    o[5] += b.y;
+                    o[6] += b.z;
+                    o[7] += b.w;
+                }
+            };
+            sum(pc, v);
+            if constexpr (SW) {
+                sum(pc + 4u, u);
+#pragma unroll
+                for (int x = 0; x < 8; ++x) v[x] = silu_p(v[x]) * u[x];
+            }
+            if constexpr (EPI == GE_F32) {
+                float4 *o = (float4 *)((float *)p.out + orow * p.ldo + col);
+                o[0] = make_float4(v[0], v[1], v[2], v[3]);
+                o[1] = make_float4(v[4], v[5], v[6], v[7]);
+                continue;
+            }
+            h16 *dst = (h16 *)p.out + orow * p.ldo + col;
+            if (EPI == GE_VISION && p.split != 0u) {
+                const u32 pj = col / p.split;
+                dst = (h16 *)(pj == 0u ? p.out : (pj == 1u ? p.out1 : p.out2)) + orow * p.split + (col - pj * p.split);
+            }
+            U4H8 o;
+#pragma unroll
+            for (int x = 0; x < 8; ++x) {
+                if (EPI == GE_F16 && p.res != nullptr) v[x] += (float)rs.h[x];
+                if (EPI == GE_VISION) v[x] = vision_act(v[x] + (float)rs.h[x], p.act);
+                o.h[x] = (h16)v[x];
+            }
+            *(uint4 *)dst = o.u;
+        }
+    }
+}
+
+/* The launch's blocks and the order of its tiles. */
+dim3 tile_grid(GemmArgs &a, u32 row_tiles, u32 col_tiles, u32 qt, bool grouped) {
+    a.nx = row_tiles;
+    a.ny = col_tiles;
+    const uint64_t wb = (uint64_t)a.N * a.K * (qt == UOCR_QT_F16 ? 4u : (qt == UOCR_QT_Q8 ? 2u : 1u)), ab = (uint64_t)a.M * a.K * 4u;
+    a.order = grouped || ab > wb ? GO_BY_ROW : GO_BY_COL;
+    return dim3((row_tiles * col_tiles + 7u) / 8u * 8u);
+}
+
+/* Wavefronts per block: as many lines of 128 bytes each, at most KS_WAVES. */
+u32 ksplit_waves(u32 qt, u32 K) {
+    const u32 ng = qt == UOCR_QT_Q4 ? 4u : (qt == UOCR_QT_Q8 ? 2u : 1u), nch = (K / 64u + ng - 1u) / ng;
+    const u32 per = (nch + KS_WAVES - 1u) / KS_WAVES;
+    return (nch + per - 1u) / per;
+}
+
+template <int EPI, bool GROUPED>
+hipError_t launch_ksplit(hipStream_t st, u32 qt, GemmArgs a, u32 row_tiles) {
+    const u32 nw = ksplit_waves(qt, a.K), cw = EPI == GE_SWIGLU ? 32u : 64u;
+    const dim3 grid = tile_grid(a, row_tiles, (a.N + cw - 1u) / cw, qt, GROUPED);
+#define GO(Q, PK) hipLaunchKernelGGL((k_gemm_ksplit<Q, EPI, GROUPED, PK>), grid, dim3(64u * nw), nw * KS_PLANE, st, a)
+    if (qt == UOCR_QT_F16) GO(1, false);
+    else if (qt == UOCR_QT_Q8 && a.packed) GO(3, true);
+    else if (qt == UOCR_QT_Q8) GO(3, false);
+    else if (a.packed) GO(4, true);
+    else GO(4, false);
+#undef GO
+    return hipGetLastError();
+}
+
+template <int EPI, bool GROUPED, int RT, int WN, int WK>
+hipError_t launch(hipStream_t st, u32 qt, GemmArgs a, u32 row_tiles) {
+    const u32 cw = (EPI == GE_SWIGLU ? 32u : 64u) * WN;
+    const dim3 grid = tile_grid(a, row_tiles, (a.N + cw - 1u) / cw, qt, GROUPED);
+#define GO(Q, PK) hipLaunchKernelGGL((k_gemm_tile<Q, EPI, GROUPED, PK, RT, WN, WK>), grid, dim3(64 * WN * WK), 0, st, a)
+    if (qt == UOCR_QT_F16) GO(1, false);
+    else if (qt == UOCR_QT_Q8 && a.packed) GO(3, true);
+    else if (qt == UOCR_QT_Q8) GO(3, false);
+    else if (a.packed) GO(4, true);
+    else GO(4, false);
+#undef GO
+    return hipGetLastError();
+}
+
+template <int RT, int WN, int WK>
+hipError_t plain(hipStream_t st, int epi, u32 qt, const GemmArgs &a) {
+    const u32 tiles = (a.M + 32u * RT - 1u) / (32u * RT);
+    switch (epi) {
+        case GE_F16: return launch<GE_F16, false, RT, WN, WK>(st, qt, a, tiles);
+        case GE_F32: return launch<GE_F32, false, RT, WN, WK>(st, qt, a, tiles);
+        case GE_VISION: return launch<GE_VISION, false, RT, WN, WK>(st, qt, a, tiles);
+        case GE_SWIGLU: return launch<GE_SWIGLU, false, RT, WN, WK>(st, qt, a, tiles);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+hipError_t plain_lines(hipStream_t st, int epi, u32 qt, const GemmArgs &a) {
+    const u32 tiles = (a.M + 31u) / 32u;
+    switch (epi) {
+        case GE_F16: return launch_ksplit<GE_F16, false>(st, qt, a, tiles);
+        case GE_F32: return launch_ksplit<GE_F32, false>(st, qt, a, tiles);
+        case GE_VISION: return launch_ksplit<GE_VISION, false>(st, qt, a, tiles);
+        case GE_SWIGLU: return launch_ksplit<GE_SWIGLU, false>(st, qt, a, tiles);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+/* Which kernel a plain GEMM of M x N (SwiGLU: N pairs) x K takes.  A K step of
+ * a block takes 0.6-0.9 us whatever it computes (its loads' latency), so the
+ * large tile, the cheapest per output, is taken once its grid gives two thirds
+ * of the CUs a block, and smaller grids split K over the wavefronts instead.
+ * Measured (us, Q8, old kernel / large / 64 x 128, K in 2 / 32 x 64, K in 8 /
+ * 32 x 64, K by lines):
+ *   4001 x 1280 x 1280   34.9 / 27.7 / 28.9 / 78  / 62    160 large tiles
+ *   4096 x 768 x 768     15.0 / 20.8 / 15.1 / 43  / 27     96
+ *   932 x 1280 x 1280    25.2 / 25.6 / 13.6 / 25  / 22     40
+ *   257 x 3072 x 1024    14.6 / 24.4 / 12.6 / 17  / 13.4   432 narrow tiles
+ *   196 x 3072 x 768     13.2 / 23.2 / 13.0 / 17  / 10.0   336
+ *   257 x 1024 x 4096    18.0 / 69   / 33   / 17  / 22     144
+ *   300 x 1280 x 6848    68.2 / 109  / 47   / 23.5 / 28    200
+ *   77 x 1280 x 896      13.4 / 17.0 / 9.2  / 6.8 / 6.2     60 */
+enum { CFG_LARGE, CFG_MID, CFG_MID_K4, CFG_NARROW_K8, CFG_LINES };
+
+int choose(bool sw, u32 M, u32 N, u32 K) {
+    const u32 n2 = sw ? 2u * N : N, large = ((M + 127u) / 128u) * ((n2 + 255u) / 256u), narrow = ((M + 31u) / 32u) * ((n2 + 63u) / 64u);
+    if (large >= 160u) return CFG_LARGE;
+    if (K >= 3072u && narrow <= 256u) return CFG_NARROW_K8;
+    if (narrow <= 384u) return CFG_LINES;
+    /* 932 x 1280 x 6848: 65.1 (old), 47.3 (K in 2), 41.1 (K in 4); 1600 x 768
+     * x 3072: 32.4, 26.4, 26.0 */
+    return K >= 4096u ? CFG_MID_K4 : CFG_MID;
+}
+
+}  // namespace
+
+bool uocr_gemm_tile_fits(int epi, u32 qt, const GemmArgs &a) {
+    const uint64_t rowb = qt == UOCR_QT_Q4 ? a.K / 2u : (qt == UOCR_QT_Q8 ? a.K : 2ull * a.K), lim = 1ull << 32;
+    uintptr_t al = (uintptr_t)a.A | (uintptr_t)a.W[0].w | (epi == GE_SWIGLU ? (uintptr_t)a.W[1].w : 0u);
+    return a.vec != 0u && (epi == GE_F16 || epi == GE_F32 || epi == GE_SWIGLU || epi == GE_VISION) && a.nseg == 0u && al % 16u == 0u &&
+           (uint64_t)a.M * a.lda * 2u < lim && (uint64_t)a.M * a.ldr * 2u < lim && a.N * rowb < lim && (!a.packed || a.N % 32u == 0u);
+}
+
+hipError_t uocr_gemm_tile_plain(hipStream_t st, int epi, u32 qt, const GemmArgs &a) {
+    switch (choose(epi == GE_SWIGLU, a.M, a.N, a.K)) {
+        case CFG_LARGE: return plain<4, 4, 1>(st, epi, qt, a);
+        case CFG_MID: return plain<2, 2, 2>(st, epi, qt, a);
+        case CFG_MID_K4: return plain<2, 2, 4>(st, epi, qt, a);
+        case CFG_NARROW_K8: return plain<1, 1, 8>(st, epi, qt, a);
+        default: return plain_lines(st, epi, qt, a);
+    }
+}

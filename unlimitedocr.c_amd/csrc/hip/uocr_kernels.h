@@ -259,6 +259,9 @@ typedef struct uocr_gemm_desc {
 } uocr_gemm_desc;
 
 hipError_t uocr_launch_gemm(hipStream_t st, int epi, const uocr_gemm_desc *d);
+/* 1 when uocr_launch_gemm runs d in one launch that needs no partials (ksplit
+ * and part are then ignored). */
+int uocr_gemm_splits_itself(int epi, const uocr_gemm_desc *d);
 /* Two independent GEMMs in one launch (blocks split between their tile
  * grids): A plain SwiGLU with B the fp16 router (F32), or A plain F16 with B
  * grouped SwiGLU or grouped F32 of the same qtype; neither split-K, fused

@@ -394,7 +394,7 @@ extern "C" int uocr_op_vision_linear(uint32_t qtype, const void *w, const void *
     d.split = split;
     d.out1 = dst1;
     d.out2 = dst2;
-    d.ksplit = vision_ksplit(m, n, k);
+    if (!uocr_gemm_splits_itself(UOCR_GEMM_VISION, &d)) d.ksplit = vision_ksplit(m, n, k);
     lazy_lock lk;
     if (d.ksplit > 1u) {
         const size_t need = (size_t)d.ksplit * m * n * sizeof(float);

@@ -23,16 +23,9 @@
  * fp16 rounding happens where the decode path rounds (norm, q/k/v, RoPE,
  * attention output, O + residual, SwiGLU mids, shared output, layer output).
  */
-#include "uocr_kernels.h"
+#include "uocr_gemm.h"
 
 #include <math.h>
-
-#include <type_traits>
-
-typedef _Float16 h16;
-typedef _Float16 h16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef uint32_t u32;
 
 #define PB 256 /* threads per prefill block */
 #define TM 64  /* GEMM tile rows */
@@ -51,55 +44,9 @@ typedef uint32_t u32;
 #define GDEPTH_SWIGLU 1
 #endif
 
-__device__ __forceinline__ float silu_p(float g) {
-    return g / (1.0f + expf(-g));
-}
-
-union U4H8 {
-    uint4 u;
-    h16x8 v;
-    h16 h[8];
-};
-
-/* exact fp16 of bytes b0,b1 (each < 256) + 1024 */
-__device__ __forceinline__ u32 magic2(u32 v, u32 sel) {
-    return __builtin_amdgcn_perm(0x64646464u, v, sel);
-}
-
 /* ------------------------------------------------------------------------ */
 /* GEMM                                                                      */
 /* ------------------------------------------------------------------------ */
-
-/* f(integral_constant<int, i>) for i = 0..N-1, in order, unrolled at compile
- * time (register-ring slots need constant indices). */
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F &&f) {
-    if constexpr (N > 0) {
-        static_for<N - 1>(f);
-        f(std::integral_constant<int, N - 1>{});
-    }
-}
-
-enum { GE_F16 = 0, GE_F32 = 1, GE_SWIGLU = 2, GE_VISION = 3, GE_PART = 4, GE_ROPE = 5 };
-
-/* QuickGELU of the CLIP MLP: x * sigmoid(1.702 x) (dense.metal:63-66). */
-__device__ __forceinline__ float quick_gelu(float x) {
-    /* hardware exp2 and reciprocal (about 1 ulp each in fp32; the result is
-     * rounded to fp16) instead of the full-precision expf and divide */
-    return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.702f * 1.4426950408889634f * x));
-}
-
-/* GELU of the SAM MLP, 0.5 x (1 + erf(x / sqrt 2)), with erf from
- * Abramowitz & Stegun 7.1.26 (|error| <= 1.5e-7), the approximation the
- * reference's SAM kernels use (sam.metal:78-91). */
-__device__ __forceinline__ float gelu_erf_as(float x) {
-    const float z = x * 0.70710678118654752f;
-    const float az = fabsf(z);
-    const float t = __builtin_amdgcn_rcpf(1.0f + 0.3275911f * az);
-    const float poly = ((((1.061405429f * t - 1.453152027f) * t + 1.421413741f) * t - 0.284496736f) * t + 0.254829592f) * t;
-    const float e = 1.0f - poly * __builtin_amdgcn_exp2f(-1.4426950408889634f * az * az);
-    return 0.5f * x * (1.0f + (z < 0.0f ? -e : e));
-}
 
 /* Weight piece of one K step (one 64-column quantisation group) for the
  * weight row n = the output column of this lane, lane half h = lane / 32:
@@ -116,11 +63,6 @@ struct BPiece {
     static constexpr int NV = QT == 4 ? 1 : (QT == 3 ? 2 : 4); /* uint4 loads */
     static constexpr int NW = 4 * NV;                          /* words */
 };
-
-template <int QT>
-__device__ __forceinline__ u32 b_koff(u32 i, u32 h) {
-    return QT == 4 ? ((i & 2u) << 4) + 16u * h + ((i & 1u) << 3) : 32u * h + 8u * i;
-}
 
 /* The piece is kept as plain words (no struct or vector copies), so the
  * register ring stays in registers. */
@@ -147,81 +89,16 @@ __device__ __forceinline__ void b_load(u32 (&w)[BPiece<QT>::NW], u32 &sc, const 
     if (QT != 1 && with_scale) sc = ((const unsigned short *)S)[(size_t)n * (K / 64u) + g];
 }
 
-/* The four B operands (8 fp16 each) of a loaded piece: fp16(q * scale), the
- * product of two fp16 values rounded once, as half(float(q) * scale) in
- * gemm_q4.metal:55 (the integer q is exact after the bias subtraction);
- * f16: the values. */
+/* The four B operands (8 fp16 each) of a loaded piece: fp16(q * scale). */
 template <int QT>
 __device__ __forceinline__ void b_dequant(const u32 (&w)[BPiece<QT>::NW], u32 sc, h16x8 (&b)[4]) {
-    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-    const h16 sv = __builtin_bit_cast(h16, (unsigned short)sc);
-    const h2 sc2 = {sv, sv};
-    union {
-        h16x8 v;
-        u32 d[4];
-    } o;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        if (QT == 4) {
-            const h2 bb = __builtin_bit_cast(h2, 0x64086408u); /* (1032, 1032) */
-#pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                const u32 x = w[2 * (i & 1) + q];
-                const u32 nb = (i & 2) ? (x >> 4) & 0x0F0F0F0Fu : x & 0x0F0F0F0Fu;
-                o.d[2 * q] = __builtin_bit_cast(u32, (__builtin_bit_cast(h2, magic2(nb, 0x04010400u)) - bb) * sc2);
-                o.d[2 * q + 1] = __builtin_bit_cast(u32, (__builtin_bit_cast(h2, magic2(nb, 0x04030402u)) - bb) * sc2);
-            }
-        } else if (QT == 3) {
-            const h2 bb = __builtin_bit_cast(h2, 0x64806480u); /* (1152, 1152) */
-#pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                const u32 u = w[2 * i + q] ^ 0x80808080u;
-                o.d[2 * q] = __builtin_bit_cast(u32, (__builtin_bit_cast(h2, magic2(u, 0x04010400u)) - bb) * sc2);
-                o.d[2 * q + 1] = __builtin_bit_cast(u32, (__builtin_bit_cast(h2, magic2(u, 0x04030402u)) - bb) * sc2);
-            }
-        } else {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) o.d[q] = w[4 * i + q];
-        }
-        b[i] = o.v;
+        if (QT == 4) b[i] = dequant_q4(w[2 * (i & 1)], w[2 * (i & 1) + 1], (i & 2) != 0, sc);
+        else if (QT == 3) b[i] = dequant_q8(w[2 * i], w[2 * i + 1], sc);
+        else b[i] = operand_f16(w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]);
     }
 }
-
-struct RopeTabP {
-    float f[UOCR_K_HEAD_DIM / 2];
-};
-
-/* GE_ROPE destinations: q rows [P][1280], the layer's K / V caches
- * [head][cap][128]; cs holds (cos, sin) of token t's angle t * f[d] at
- * cs[64 t + d]. */
-struct RopeDst {
-    const float2 *cs;
-    h16 *q, *k, *v;
-    u32 cap;
-};
-
-struct GemmArgs {
-    const h16 *A;        /* activations, row stride lda (halves) */
-    u32 lda;
-    const int32_t *a_idx;  /* grouped: A row of each slot */
-    const int32_t *o_idx;  /* grouped: output row of each slot */
-    u32 M, N, K;
-    uocr_qmat W[3];      /* W[0] (and W[1] for SwiGLU; W[seg] when nseg) */
-    u32 nseg;            /* when nonzero, columns [s*nseg, (s+1)*nseg) use W[s] */
-    uint64_t w_stride, s_stride; /* grouped: per-expert strides (bytes / halves) */
-    const int32_t *tile_e, *tile_s0, *tile_s1, *ntiles; /* grouped tile table */
-    void *out;
-    u32 ldo;
-    const h16 *res;      /* GE_F16: optional residual, row stride ldr */
-    u32 ldr;
-    const h16 *bias;     /* GE_VISION: per-column bias */
-    u32 act;             /* GE_VISION: UOCR_VISION_ACT_* */
-    u32 split;           /* GE_VISION: 0, or the width of each of out/out1/out2 */
-    void *out1, *out2;
-    u32 kst;             /* split-K: K steps per blockIdx.z (0: all of K in one block) */
-    u32 sc_lds;          /* the block's scale rows are preloaded into dynamic LDS */
-    u32 packed;          /* Q4/Q8 payloads in the GEMM-packed layout */
-};
 
 /* Scale rows in LDS: a block's 128 weight rows x K/64 groups are one
  * contiguous region of the scale tensor, loaded once with wide loads instead
@@ -1393,6 +1270,13 @@ static bool gemm_desc_ok(int epi, const uocr_gemm_desc *d) {
     return true;
 }
 
+/* 16-byte accesses of the epilogues: every row of the outputs, the residual
+ * and the bias starts on such a boundary. */
+static bool gemm_vec(const uocr_gemm_desc *d) {
+    const uintptr_t p = (uintptr_t)d->out | (uintptr_t)d->out1 | (uintptr_t)d->out2 | (uintptr_t)d->bias | (uintptr_t)d->res;
+    return d->N % 8u == 0u && d->ldo % 8u == 0u && d->split % 8u == 0u && (d->res == nullptr || d->ldr % 8u == 0u) && p % 16u == 0u;
+}
+
 static GemmArgs gemm_args(const uocr_gemm_desc *d) {
     GemmArgs a;
     a.A = (const h16 *)d->A;
@@ -1422,7 +1306,12 @@ static GemmArgs gemm_args(const uocr_gemm_desc *d) {
     a.kst = 0u;
     a.packed = d->packed != 0u && d->W[0].qtype != UOCR_QT_F16 ? 1u : 0u;
     a.sc_lds = 0u;
+    a.vec = gemm_vec(d) ? 1u : 0u;
     return a;
+}
+
+extern "C" int uocr_gemm_splits_itself(int epi, const uocr_gemm_desc *d) {
+    return d->tile_e == nullptr && uocr_gemm_tile_fits(epi, d->W[0].qtype, gemm_args(d));
 }
 
 extern "C" hipError_t uocr_launch_gemm(hipStream_t st, int epi, const uocr_gemm_desc *d) {
@@ -1450,6 +1339,13 @@ extern "C" hipError_t uocr_launch_gemm(hipStream_t st, int epi, const uocr_gemm_
         return hipErrorInvalidValue;
     }
     const bool fuse_norm = want_norm && splittable;
+    if (!grouped && uocr_gemm_tile_fits(epi, qt, a)) {
+        const hipError_t e = uocr_gemm_tile_plain(st, epi, qt, a);
+        if (e != hipSuccess || !want_norm) return e;
+        hipLaunchKernelGGL(k_rows_rmsnorm, dim3((d->M + 3u) / 4u), dim3(PB), 0, st, (const h16 *)d->out,
+                           (const h16 *)d->norm_w, d->M, (h16 *)d->norm_out);
+        return hipGetLastError();
+    }
     if (splittable) {
         /* split-K: blockIdx.z takes K steps [z*kst, (z+1)*kst) into an fp32
          * partial plane of part, then one ordered reduce applies the
