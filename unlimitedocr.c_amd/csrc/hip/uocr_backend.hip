@@ -97,7 +97,6 @@ struct uocr_hip_ctx {
     uint32_t *route_ids;
     /* MFMA prefill scratch, sized for prompt_cap rows */
     uint16_t *p_xn, *p_q, *p_ctx, *p_a, *p_mid, *p_smid, *p_sout, *p_rmid;
-    float *p_fa_ws; /* prefill attention key-split partials */
     float *p_rope;  /* prefill RoPE (cos, sin) per token and pair */
     float *p_kpart; /* prefill GEMM split-K partials */
     float *p_logits, *p_wts;
@@ -687,7 +686,6 @@ extern "C" int uocr_hip_context_allocate_runtime(uocr_hip_ctx *ctx, uint32_t pro
     const uint64_t o_poff = p.take(64u * 4u);
     const uint64_t o_pte = p.take(max_tiles * 4u), o_pts0 = p.take(max_tiles * 4u), o_pts1 = p.take(max_tiles * 4u);
     const uint64_t o_pnt = p.take(4u), o_plt = p.take(PK * 4u), o_plp = p.take(PK * 4u);
-    const uint64_t o_pfa = p.take(uocr_flash_attn_ws_bytes());
     /* split-K partials of the O projection and the dense down (UOCR_PREFILL_KSPLIT_MAX splits x
      * P x 1280, fp32) */
     const uint64_t o_pkp = p.take(Pc * H_SIZE * UOCR_PREFILL_KSPLIT_MAX * 4u);
@@ -739,7 +737,6 @@ extern "C" int uocr_hip_context_allocate_runtime(uocr_hip_ctx *ctx, uint32_t pro
     ctx->p_ntiles = (int32_t *)(b + o_pnt);
     ctx->p_list_tok = (int32_t *)(b + o_plt);
     ctx->p_list_pair = (int32_t *)(b + o_plp);
-    ctx->p_fa_ws = (float *)(b + o_pfa);
     ctx->p_rope = (float *)(b + o_prope);
     ctx->p_kpart = (float *)(b + o_pkp);
     ctx->run_arena = b + o_run;
@@ -988,7 +985,7 @@ static hipError_t enqueue_prefill_mfma(uocr_hip_ctx *c, uint32_t P) {
         }
         d.nseg = H_SIZE;
         ENQ(uocr_launch_gemm_qkv_rope(s, &d, c->p_rope, c->p_q, kc, vc, c->cache_cap));
-        ENQ(uocr_launch_flash_attn(s, c->p_q, kc, vc, c->cache_cap, P, c->p_ctx, c->p_fa_ws));
+        ENQ(uocr_launch_flash_attn(s, c->p_q, kc, vc, c->cache_cap, P, c->p_ctx));
         d = gdesc(c->p_ctx, H_SIZE, P, H_SIZE, H_SIZE, c->p_a, H_SIZE);
         d.W[0] = packed_of(L.o, L.po);
         d.packed = L.po != nullptr;

@@ -4,38 +4,12 @@
  * tiled GEMMs gemm_q4.metal / gemm_q8.metal where a grid of large tiles fills
  * the chip).
  */
+#include "uocr_async.h"
 #include "uocr_gemm.h"
 
 #define NA 3u  /* activation tiles in LDS: two steps of loads in flight */
 
 namespace {
-
-/* Waits until at most N of the wavefront's vector memory operations are in
- * flight and its LDS reads are done, then for the block's other wavefronts. */
-template <int N>
-__device__ __forceinline__ void wait_barrier() {
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
-}
-
-__device__ __forceinline__ u32 uni(u32 v) {
-    return (u32)__builtin_amdgcn_readfirstlane((int)v);
-}
-
-template <typename T>
-__device__ __forceinline__ T *uni(T *p) {
-    const uint64_t v = (uint64_t)p;
-    return (T *)(((uint64_t)uni((u32)(v >> 32)) << 32) | uni((u32)v));
-}
-
-/* 16 bytes per lane from base + voff straight into LDS at lds + 16 lane.  In
- * inline assembly because the compiler's own LDS-direct load makes every later
- * LDS read wait for all of them; wait_barrier counts them instead. */
-__device__ __forceinline__ void lds_load16(const void *base, u32 voff, u32 lds) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                 :
-                 : "v"(voff), "s"(uni(base)), "s"(lds)
-                 : "memory");
-}
 
 /* The block's tile.  Blocks go to the 8 XCDs in turn; with by_row or by_col
  * each XCD takes a contiguous run of row tiles (of column tiles) instead, so

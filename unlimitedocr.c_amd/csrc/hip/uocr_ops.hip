@@ -351,9 +351,8 @@ extern "C" int uocr_op_gemm(uint32_t qtype, const void *w, const void *s, uint32
  * 14-20 us unsplit). */
 static float *g_vision_part = nullptr;
 static size_t g_vision_part_bytes = 0;
-/* Guards the lazily allocated operator buffers (g_vision_part, the prefill
- * attention partials): held from the size check through the launch, so two
- * threads never allocate twice or launch into a buffer being replaced; the
+/* Guards the lazily allocated operator buffer (g_vision_part): held from the
+ * size check through the launch, so two threads never allocate twice or launch into a buffer being replaced; the
  * launches then serialise on the operator stream. */
 static pthread_mutex_t g_lazy_mu = PTHREAD_MUTEX_INITIALIZER;
 struct lazy_lock {
@@ -425,20 +424,8 @@ extern "C" int uocr_op_prefill_attention(const void *q, const void *k_cache, con
         return op_fail(UOCR_ERROR_INVALID_ARGUMENT, "invalid prefill_attention arguments");
     }
     STREAM_OR_RETURN(st);
-    /* key-split partials: allocated on first need outside graph capture and
-     * kept (calls must not overlap); without them the unsplit kernel runs */
-    static float *fa_ws = nullptr;
-    lazy_lock lk;
-    if (fa_ws == nullptr) {
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(st, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone) {
-            void *p = nullptr;
-            if (hipMalloc(&p, uocr_flash_attn_ws_bytes()) == hipSuccess) fa_ws = (float *)p;
-        }
-    }
     return hip_status(uocr_launch_flash_attn(st, (const uint16_t *)q, (const uint16_t *)k_cache,
-                                             (const uint16_t *)v_cache, cache_capacity, prompt_length, (uint16_t *)ctx,
-                                             fa_ws),
+                                             (const uint16_t *)v_cache, cache_capacity, prompt_length, (uint16_t *)ctx),
                       "prefill_attention");
 }
 

@@ -15,9 +15,6 @@
  *    grouped mode a tile table maps each block to an expert's bucket of
  *    (token, rank) pairs: rows are gathered through an index list and the
  *    expert's weights are addressed by slab stride.
- *  - k_flash_attn: causal attention over the prompt slots, one block per
- *    (64-query tile, head): S = Q K^T and O += P V on MFMA, fp32 online
- *    softmax in LDS.
  *  - routing (top-6 per token, expert buckets), RoPE + KV scatter, MoE
  *    combine and row RMSNorm kernels.
  * fp16 rounding happens where the decode path rounds (norm, q/k/v, RoPE,
@@ -648,321 +645,6 @@ __global__ __launch_bounds__(PB) void k_reduce_norm(const float *__restrict__ pa
 }
 
 /* ------------------------------------------------------------------------ */
-/* causal flash attention over the prompt                                    */
-/* ------------------------------------------------------------------------ */
-
-#define AQ 64 /* queries per block */
-#define AK 64 /* keys per step */
-#define LDQ (UOCR_K_HEAD_DIM + 8)
-#define LDV (AK + 8)
-
-/* Block (qt, h): queries q0..q0+63 of head h attend to slots 0..q (causal),
- * fp32 online softmax scaled by 1/sqrt(128), output fp16 into ctx [P][1280]
- * (attention_decode.metal arithmetic per query). */
-/* KV split of the causal prefill attention.  Query tile qt (64 queries) sees
- * qt + 1 key tiles; with chunks of CH key tiles it is nsplit(qt) = ceil((qt +
- * 1) / CH) blocks.  Blocks enumerate (qt, head, split) with the split
- * fastest, so the splits of one (qt, head) are consecutive block indices.
- * Each split of a tile with more than one writes its normalised O / l in
- * fp16 (the first half of the O area of its slot) and its row max / sum in
- * fp32 to its own partial slot; k_flash_merge combines them. */
-#define FA_PART_FLOATS (AQ * UOCR_K_HEAD_DIM + 2u * AQ)
-#define FA_MAX_SPLITS 16u /* splits of one query tile (the merge's weight table) */
-
-__device__ __forceinline__ u32 fa_nsplit(u32 qt, u32 ch) {
-    return (qt + ch) / ch;
-}
-
-/* first block index of query tile qt (all heads) */
-__device__ __forceinline__ u32 fa_tile_base(u32 qt, u32 ch) {
-    u32 b = 0;
-    for (u32 q = 0; q < qt; ++q) b += UOCR_K_HEADS * fa_nsplit(q, ch);
-    return b;
-}
-
-/* Wavefront w owns queries q0 + 16w .. + 15 of the block's 64 and keeps
- * everything of them in registers (16x16x32 MFMAs):
- *   S^T = K Q^T per key tile: four 16-key tiles; lane l holds query l % 16
- *   and keys 16t + 4(l / 16) + i (i < 4) of tile t;
- *   the fp32 online softmax per query, its max reduced over the four lanes
- *   that share the query (l, l ^ 16, l ^ 32, l ^ 48), its sum kept per lane
- *   and reduced once at the end;
- *   O^T = V^T P^T: the probabilities stay where S^T left them, because the
- *   B operand's 8 K slots of lane l are chosen as keys {32u + 4(l / 16) + i,
- *   32u + 16 + 4(l / 16) + i} (i < 4) and the A operand (V^T from LDS) is
- *   read at the same keys; lane l holds dims 16d + 4(l / 16) + i of query
- *   l % 16 in O^T tile d.
- * Only the K and V^T tiles go through LDS (two barriers per key tile). */
-__global__ __launch_bounds__(PB) void k_flash_attn(const h16 *__restrict__ Q, const h16 *__restrict__ kc,
-                                                   const h16 *__restrict__ vc, u32 cap, u32 P,
-                                                   h16 *__restrict__ ctx, u32 ch, float *__restrict__ part) {
-    typedef float f32x4 __attribute__((ext_vector_type(4)));
-    __shared__ __attribute__((aligned(16))) h16 ks[AK * LDQ];
-    __shared__ __attribute__((aligned(16))) h16 vt[UOCR_K_HEAD_DIM * LDV];
-    const u32 t = threadIdx.x, lane = t & 63u, wave = t >> 6, qc = lane & 15u, g = lane >> 4;
-    /* which (query tile, head, key chunk) this block computes */
-    u32 qt = blockIdx.x, h = blockIdx.y, sp = 0, ns = 1;
-    if (ch != 0u) {
-        u32 b = blockIdx.x;
-        qt = 0;
-        while (b >= UOCR_K_HEADS * fa_nsplit(qt, ch)) {
-            b -= UOCR_K_HEADS * fa_nsplit(qt, ch);
-            ++qt;
-        }
-        ns = fa_nsplit(qt, ch);
-        h = b / ns;
-        sp = b - h * ns;
-    }
-    const u32 q0 = qt * AQ;
-    const h16 *kh = kc + (size_t)h * cap * 128u, *vh = vc + (size_t)h * cap * 128u;
-    const float scale = 0.08838834764831845f;
-    /* this lane's query row: B operand pieces of Q^T for the four 32-deep
-     * steps over the head dimension */
-    const u32 qr = q0 + 16u * wave + qc; /* query index */
-    U4H8 qreg[4];
-#pragma unroll
-    for (int st = 0; st < 4; ++st) {
-        qreg[st].u = *(const uint4 *)(Q + (size_t)min(qr, P - 1u) * UOCR_K_HIDDEN + h * 128u + 32u * st + 8u * g);
-    }
-    f32x4 o[UOCR_K_HEAD_DIM / 16];
-#pragma unroll
-    for (int d = 0; d < UOCR_K_HEAD_DIM / 16; ++d) o[d] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    float m = -INFINITY, l = 0.0f;
-    const u32 qlast = min(q0 + AQ, P) - 1u;
-    /* this block's keys: tiles [sp * ch, (sp + 1) * ch) of the causal range */
-    const u32 kbeg = ch != 0u ? sp * ch * AK : 0u;
-    const u32 klast = ch != 0u ? min(qlast, (sp + 1u) * ch * AK - 1u) : qlast;
-    /* next K/V tile in registers (words, so they stay in registers) */
-    u32 kr_[4][4], va_[2][4], vb_[2][4];
-    auto load_kv = [&](u32 k0n) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const u32 idx = t + q * PB, r = idx >> 4, c8 = idx & 15u;
-            const uint4 v = *(const uint4 *)(kh + (size_t)min(k0n + r, P - 1u) * 128u + 8u * c8);
-            kr_[q][0] = v.x;
-            kr_[q][1] = v.y;
-            kr_[q][2] = v.z;
-            kr_[q][3] = v.w;
-        }
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const u32 idx = t + q * PB, kp = idx & 31u, c8 = idx >> 5;
-            const uint4 a = *(const uint4 *)(vh + (size_t)min(k0n + 2u * kp, P - 1u) * 128u + 8u * c8);
-            const uint4 b = *(const uint4 *)(vh + (size_t)min(k0n + 2u * kp + 1u, P - 1u) * 128u + 8u * c8);
-            va_[q][0] = a.x;
-            va_[q][1] = a.y;
-            va_[q][2] = a.z;
-            va_[q][3] = a.w;
-            vb_[q][0] = b.x;
-            vb_[q][1] = b.y;
-            vb_[q][2] = b.z;
-            vb_[q][3] = b.w;
-        }
-    };
-    load_kv(kbeg);
-    for (u32 k0 = kbeg; k0 <= klast; k0 += AK) {
-        __syncthreads();
-        /* K tile (row-major) and V tile transposed to [dim][key], from the
-         * registers loaded one tile ahead.  The transpose goes by key pairs:
-         * a thread holds 8 dims of keys 2i and 2i+1 and writes 8 dwords (dim
-         * d: key 2i | key 2i+1 << 16); the 32 lanes of a half-wavefront
-         * cover consecutive pairs, so each write touches consecutive banks. */
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const u32 idx = t + q * PB, r = idx >> 4, c8 = idx & 15u;
-            *(uint4 *)(ks + r * LDQ + 8u * c8) = make_uint4(kr_[q][0], kr_[q][1], kr_[q][2], kr_[q][3]);
-        }
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const u32 idx = t + q * PB, kp = idx & 31u, c8 = idx >> 5;
-            u32 *dst = (u32 *)(vt + 8u * c8 * LDV + 2u * kp);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                /* dims 2j and 2j+1: low halves, then high halves */
-                dst[(2u * j) * (LDV / 2u)] = __builtin_amdgcn_perm(vb_[q][j], va_[q][j], 0x05040100u);
-                dst[(2u * j + 1u) * (LDV / 2u)] = __builtin_amdgcn_perm(vb_[q][j], va_[q][j], 0x07060302u);
-            }
-        }
-        __syncthreads();
-        if (k0 + AK <= klast) load_kv(k0 + AK);
-        /* S^T: four 16-key tiles x this wavefront's 16 queries */
-        float sc[4][4];
-        float tm = -INFINITY;
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt) {
-            f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int st = 0; st < 4; ++st) {
-                U4H8 a;
-                a.u = *(const uint4 *)(ks + (16u * kt + qc) * LDQ + 32u * st + 8u * g);
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a.v, qreg[st].v, acc, 0, 0, 0);
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const u32 ki = k0 + 16u * kt + 4u * g + i;
-                const float v = (ki <= qr && ki < P) ? acc[i] * scale : -INFINITY;
-                sc[kt][i] = v;
-                tm = fmaxf(tm, v);
-            }
-        }
-        tm = fmaxf(tm, __shfl_xor(tm, 16));
-        tm = fmaxf(tm, __shfl_xor(tm, 32));
-        const float mnew = fmaxf(m, tm);
-        /* every query sees key k0 (k0 <= q0 <= q), so mnew is finite */
-        const float corr = m == -INFINITY ? 0.0f : expf(m - mnew);
-        l *= corr;
-#pragma unroll
-        for (int d = 0; d < UOCR_K_HEAD_DIM / 16; ++d) o[d] *= corr;
-        m = mnew;
-        /* probabilities in fp16, two B operands of 8 keys */
-        U4H8 pb[2];
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float e = sc[kt][i] == -INFINITY ? 0.0f : expf(sc[kt][i] - mnew);
-                l += e;
-                pb[kt >> 1].h[4 * (kt & 1) + i] = (h16)e;
-            }
-        }
-        /* O^T += V^T P^T */
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-#pragma unroll
-            for (int d = 0; d < UOCR_K_HEAD_DIM / 16; ++d) {
-                const h16 *vr = vt + (16u * d + qc) * LDV + 32u * u + 4u * g;
-                U4H8 a;
-                const uint2 lo = *(const uint2 *)vr, hi = *(const uint2 *)(vr + 16);
-                a.u = make_uint4(lo.x, lo.y, hi.x, hi.y);
-                o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a.v, pb[u].v, o[d], 0, 0, 0);
-            }
-        }
-    }
-    /* the query's sum over its four lanes */
-    l += __shfl_xor(l, 16);
-    l += __shfl_xor(l, 32);
-    const u32 r = 16u * wave + qc; /* row within the tile */
-    if (ns > 1u) {
-        /* partial of a split tile: O / l in fp16 (a weighted mean of V rows,
-         * so within V's range), row max and row sum in fp32 */
-        float *po = part + (size_t)blockIdx.x * FA_PART_FLOATS;
-        const float li = 1.0f / l;
-#pragma unroll
-        for (int d = 0; d < UOCR_K_HEAD_DIM / 16; ++d) {
-            union {
-                h16 hh[4];
-                uint2 u;
-            } pk;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) pk.hh[i] = (h16)(o[d][i] * li);
-            *(uint2 *)((h16 *)po + r * UOCR_K_HEAD_DIM + 16u * d + 4u * g) = pk.u;
-        }
-        if (g == 0u) {
-            po[AQ * UOCR_K_HEAD_DIM + r] = m;
-            po[AQ * UOCR_K_HEAD_DIM + AQ + r] = l;
-        }
-        return;
-    }
-    if (qr < P) {
-#pragma unroll
-        for (int d = 0; d < UOCR_K_HEAD_DIM / 16; ++d) {
-            union {
-                h16 hh[4];
-                uint2 u;
-            } pk;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) pk.hh[i] = (h16)(o[d][i] / l);
-            *(uint2 *)(ctx + (size_t)qr * UOCR_K_HIDDEN + h * 128u + 16u * d + 4u * g) = pk.u;
-        }
-    }
-}
-
-/* Merge of the split tiles: block (x, h, z) takes rows 16z..16z+15 of query
- * tile ch + x (every tile from ch on has at least two splits): ctx = sum_s
- * (O_s / l_s) l_s e^(m_s - M) / sum_s l_s e^(m_s - M), M = max_s m_s (split 0
- * holds key 0, so every row has L > 0).  Each thread owns two 4-value pieces
- * of the 16 x 128 block and issues the splits' loads four at a time. */
-__global__ __launch_bounds__(PB) void k_flash_merge(const float *__restrict__ part, u32 P, u32 ch,
-                                                    h16 *__restrict__ ctx) {
-    const u32 qt = ch + blockIdx.x, h = blockIdx.y, r0 = 16u * blockIdx.z, ns = fa_nsplit(qt, ch);
-    const float *pb = part + (size_t)(fa_tile_base(qt, ch) + h * ns) * FA_PART_FLOATS;
-    __shared__ float wgt[FA_MAX_SPLITS][16], linv[16];
-    if (threadIdx.x < 16u) {
-        const u32 r = r0 + threadIdx.x;
-        /* all of the row's (m, l) loads in flight at once */
-        float mv[FA_MAX_SPLITS], lv[FA_MAX_SPLITS];
-#pragma unroll
-        for (u32 s = 0; s < FA_MAX_SPLITS; ++s) {
-            if (s < ns) {
-                mv[s] = pb[s * FA_PART_FLOATS + AQ * UOCR_K_HEAD_DIM + r];
-                lv[s] = pb[s * FA_PART_FLOATS + AQ * UOCR_K_HEAD_DIM + AQ + r];
-            }
-        }
-        float M = -INFINITY;
-#pragma unroll
-        for (u32 s = 0; s < FA_MAX_SPLITS; ++s) {
-            if (s < ns) M = fmaxf(M, mv[s]);
-        }
-        float L = 0.0f;
-#pragma unroll
-        for (u32 s = 0; s < FA_MAX_SPLITS; ++s) {
-            if (s < ns) {
-                const float w = mv[s] == -INFINITY ? 0.0f : expf(mv[s] - M);
-                const float wl = w * lv[s];
-                wgt[s][threadIdx.x] = wl; /* the split's O / l times its share */
-                L += wl;
-            }
-        }
-        linv[threadIdx.x] = 1.0f / L;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-        const u32 e4 = threadIdx.x + q * PB;          /* float4 index within the 16 x 128 block */
-        const u32 rl = e4 / (UOCR_K_HEAD_DIM / 4u), d = 4u * (e4 % (UOCR_K_HEAD_DIM / 4u));
-        const size_t off = (size_t)(r0 + rl) * UOCR_K_HEAD_DIM + d;
-        float4 o = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        for (u32 s0 = 0; s0 < ns; s0 += 4u) {
-            float4 v[4];
-#pragma unroll
-            for (u32 u = 0; u < 4u; ++u) {
-                if (s0 + u < ns) {
-                    union {
-                        h16 hh[4];
-                        uint2 u2;
-                    } pk;
-                    pk.u2 = *(const uint2 *)((const h16 *)(pb + (s0 + u) * FA_PART_FLOATS) + off);
-                    v[u] = make_float4((float)pk.hh[0], (float)pk.hh[1], (float)pk.hh[2], (float)pk.hh[3]);
-                }
-            }
-#pragma unroll
-            for (u32 u = 0; u < 4u; ++u) {
-                if (s0 + u < ns) {
-                    const float w = wgt[s0 + u][rl];
-                    o.x += w * v[u].x;
-                    o.y += w * v[u].y;
-                    o.z += w * v[u].z;
-                    o.w += w * v[u].w;
-                }
-            }
-        }
-        const u32 row = qt * AQ + r0 + rl;
-        if (row < P) {
-            const float li = linv[rl];
-            union {
-                h16 hh[4];
-                uint2 u;
-            } pk;
-            pk.hh[0] = (h16)(o.x * li);
-            pk.hh[1] = (h16)(o.y * li);
-            pk.hh[2] = (h16)(o.z * li);
-            pk.hh[3] = (h16)(o.w * li);
-            *(uint2 *)(ctx + (size_t)row * UOCR_K_HIDDEN + h * 128u + d) = pk.u;
-        }
-    }
-}
-
-/* ------------------------------------------------------------------------ */
 /* MoE routing, buckets, combine                                             */
 /* ------------------------------------------------------------------------ */
 
@@ -1526,49 +1208,6 @@ extern "C" hipError_t uocr_launch_gemm_qkv_rope(hipStream_t st, const uocr_gemm_
                                (h16 *)vcache, cap);
             break;
     }
-    return hipGetLastError();
-}
-
-/* Resident blocks of k_flash_attn on the chip (about 80 KB of LDS each: two
- * per CU).  The key chunk is the smallest whose (tile, head, chunk) blocks
- * all fit at once; the longest block then walks ch key tiles instead of all
- * of the last query tile's.  0: one block per (tile, head), no split. */
-#ifndef FA_SLOTS
-#define FA_SLOTS 512u
-#endif
-
-static u32 fa_chunk(u32 P) {
-    const u32 nq = (P + AQ - 1u) / AQ;
-    for (u32 ch = 1; ch < nq; ++ch) {
-        u32 blocks = 0;
-        for (u32 q = 0; q < nq; ++q) blocks += UOCR_K_HEADS * ((q + ch) / ch);
-        if (blocks <= FA_SLOTS && (nq + ch - 1u) / ch <= FA_MAX_SPLITS) return ch;
-    }
-    return 0u;
-}
-
-extern "C" size_t uocr_flash_attn_ws_bytes(void) {
-    return (size_t)FA_SLOTS * FA_PART_FLOATS * sizeof(float);
-}
-
-extern "C" hipError_t uocr_launch_flash_attn(hipStream_t st, const uint16_t *q, const uint16_t *kcache,
-                                             const uint16_t *vcache, uint32_t cap, uint32_t P, uint16_t *ctx,
-                                             float *ws) {
-    if (q == nullptr || kcache == nullptr || vcache == nullptr || ctx == nullptr || P == 0u || P > cap) {
-        return hipErrorInvalidValue;
-    }
-    const u32 nq = (P + AQ - 1u) / AQ, ch = ws != nullptr ? fa_chunk(P) : 0u;
-    if (ch == 0u) {
-        hipLaunchKernelGGL(k_flash_attn, dim3(nq, UOCR_K_HEADS), dim3(PB), 0, st, (const h16 *)q,
-                           (const h16 *)kcache, (const h16 *)vcache, cap, P, (h16 *)ctx, 0u, (float *)nullptr);
-        return hipGetLastError();
-    }
-    u32 blocks = 0;
-    for (u32 qi = 0; qi < nq; ++qi) blocks += UOCR_K_HEADS * ((qi + ch) / ch);
-    hipLaunchKernelGGL(k_flash_attn, dim3(blocks), dim3(PB), 0, st, (const h16 *)q, (const h16 *)kcache,
-                       (const h16 *)vcache, cap, P, (h16 *)ctx, ch, ws);
-    hipLaunchKernelGGL(k_flash_merge, dim3(nq - ch, UOCR_K_HEADS, AQ / 16u), dim3(PB), 0, st, (const float *)ws, P,
-                       ch, (h16 *)ctx);
     return hipGetLastError();
 }
 
