@@ -86,3 +86,97 @@ def test_gemm_misaligned_rows(gpu, qtype):
     uocr.sync()
     got = dy.download(np.float16, 4 + m * n2)[4:].reshape(m, n2)
     check_rows(got, x, wv[:n2], np.zeros((m, n2)))
+
+
+def routed_rows(rng, counts, P):
+    """For each row its 6 experts, so that expert e serves counts[e] rows."""
+    left = np.full(P, 6)
+    chosen = [[] for _ in range(P)]
+    for e in np.argsort(-np.asarray(counts)):
+        rows = np.argsort(-left + rng.random(P) * 0.5, kind="stable")[:counts[e]]
+        assert (left[rows] > 0).all()
+        left[rows] -= 1
+        for r in rows:
+            chosen[r].append(int(e))
+    assert (left == 0).all()
+    return chosen
+
+
+def bucket_counts(P, given):
+    """`given` rows for the first experts, the rest of the 6 P spread evenly."""
+    rest = 6 * P - sum(given)
+    n = 64 - len(given)
+    return list(given) + [rest // n + (i < rest % n) for i in range(n)]
+
+
+@pytest.mark.parametrize("qtype", [1, 3, 4])
+@pytest.mark.parametrize("P,given,static", [(1, [], True), (6, [6, 6], True), (7, [7], True), (64, [64, 33, 32, 31, 1], True),
+                                            (263, [263, 257, 256, 129, 128, 97, 96, 65, 64, 33, 32, 31, 1], False)])
+def test_moe_rows_bucket_edges(gpu, qtype, P, given, static):
+    """Expert buckets on both sides of every tile height (and above one tile),
+    with few rows (weight lines) and more.  The router is a selector, so the
+    bucket sizes are chosen.  Reference: float64 over the kernels' operand
+    values with the mids and the shared output rounded to fp16; a mid whose fp32
+    sum lies at a rounding boundary may differ by one unit (2^-10), so the bound
+    is that share of the magnitudes plus the final rounding."""
+    uocr = gpu
+    rng = np.random.default_rng(P + qtype)
+    counts = [c if c <= P else P for c in bucket_counts(P, given)]
+    chosen = routed_rows(rng, counts, P)
+    x = rand_f16(rng, (P, 1280), 0.5)
+    x[:, :64] = 0
+    for t, es in enumerate(chosen):
+        x[t, es] = np.float16(1) + np.arange(len(es), dtype=np.float16) / 8
+    router = np.zeros((64, 1280), np.float16)
+    router[np.arange(64), np.arange(64)] = 8
+    res = rand_f16(rng, (P, 1280))
+    of = uocr.DeviceBuffer.of
+    m, keep, val = uocr.CMoeWeights(), [], {}
+    m.expert_qtype = m.shared_qtype = qtype
+    for name, rows, k in (("gate", 64 * 896, 1280), ("up", 64 * 896, 1280), ("down", 64 * 1280, 896), ("sgate", 1792, 1280),
+                          ("sup", 1792, 1280), ("sdown", 1280, 1792)):
+        # a few distinct experts' weights, repeated: the bytes are what the test needs, not their number
+        n = rows // 64 if rows > 2000 else rows
+        w, s = weights_for(qtype, rng, 4 * n if rows > 2000 else n, k)
+        val[name] = operand_values(qtype, w, s)
+        if rows > 2000:
+            w = np.tile(w, (16, 1))
+            s = None if s is None else np.tile(s, (16, 1))
+        keep += [of(w), None if s is None else of(s)]
+        setattr(m, name + "_w", keep[-2].ptr)
+        setattr(m, name + "_s", None if s is None else keep[-1].ptr)
+        if name in ("gate", "down"):
+            pre = "gu" if name == "gate" else "dn"
+            setattr(m, pre + "_w_stride", w.nbytes // 64)
+            setattr(m, pre + "_s_stride", 0 if s is None else s.size // 64)
+    dr, dx, dres, dout = of(router), of(x), of(res), uocr.DeviceBuffer(P * 2560)
+    m.router = dr.ptr
+    if static:
+        uocr.op_moe_ffn_rows_static(m, dx, None, dres, P, 0, dout)
+    else:
+        uocr.op_moe_ffn_rows(m, dx, None, dres, P, 0, uocr.moe_rows_workspace(P), dout)
+    uocr.sync()
+    got = dout.download(np.float16).reshape(P, 1280).astype(np.float64)
+
+    xd = x.astype(np.float64)
+
+    def ffn(xin, g, u, d):
+        a = xin @ g.T
+        mid = (a / (1 + np.exp(-a)) * (xin @ u.T)).astype(np.float16).astype(np.float64)
+        return mid @ d.T, np.abs(mid) @ np.abs(d).T
+
+    y, mag = ffn(xd, val["sgate"], val["sup"], val["sdown"])
+    y = y.astype(np.float16).astype(np.float64) + res.astype(np.float64)
+    logits = xd[:, :64] * 8
+    p = np.exp(logits - logits.max(1, keepdims=True))
+    p /= p.sum(1, keepdims=True)
+    for e in range(64):
+        rows = [t for t in range(P) if e in chosen[t]]
+        if rows:
+            part = lambda name, n: val[name][(e % 4) * n:(e % 4 + 1) * n]  # noqa: E731
+            o, a = ffn(xd[rows], part("gate", 896), part("up", 896), part("down", 1280))
+            y[rows] += p[rows, e, None] * o
+            mag[rows] += p[rows, e, None] * a
+    bound = np.abs(y) * 2.0**-11 + mag * 2.0**-10 + 2.0**-24
+    err = np.abs(got - y)
+    assert (err <= bound).all(), float((err / bound).max())

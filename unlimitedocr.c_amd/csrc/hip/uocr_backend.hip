@@ -1014,8 +1014,6 @@ static hipError_t enqueue_prefill_mfma(uocr_hip_ctx *c, uint32_t P) {
             continue;
         }
         const uint32_t SI = UOCR_MOE_SHARED_INTERMEDIATE, EI = UOCR_MOE_EXPERT_INTERMEDIATE;
-        /* the router logits share a launch with the shared gate/up (both read
-         * xn), the shared down with the routed down */
         uocr_gemm_desc dr = gdesc(c->p_xn, H_SIZE, P, UOCR_ROUTED_EXPERTS, H_SIZE, c->p_logits, UOCR_ROUTED_EXPERTS);
         dr.W[0].w = L.router;
         dr.W[0].s = nullptr;
@@ -1024,9 +1022,6 @@ static hipError_t enqueue_prefill_mfma(uocr_hip_ctx *c, uint32_t P) {
         dsg.packed = L.psg != nullptr && L.psu != nullptr;
         dsg.W[0] = dsg.packed ? packed_of(L.sgate, L.psg) : L.sgate;
         dsg.W[1] = dsg.packed ? packed_of(L.sup, L.psu) : L.sup;
-        ENQ(uocr_launch_gemm_pair(s, UOCR_GEMM_SWIGLU, &dsg, UOCR_GEMM_F32, &dr));
-        ENQ(uocr_launch_route_rows(s, c->p_logits, P, 0, c->p_ids, c->p_wts, c->p_offsets, c->p_tile_e, c->p_tile_s0, c->p_tile_s1, c->p_ntiles, c->p_list_tok,
-                                   c->p_list_pair));
         uocr_gemm_desc dsd = gdesc(c->p_smid, SI, P, H_SIZE, SI, c->p_sout, H_SIZE);
         dsd.W[0] = packed_of(L.sdown, L.psd);
         dsd.packed = L.psd != nullptr;
@@ -1043,17 +1038,8 @@ static hipError_t enqueue_prefill_mfma(uocr_hip_ctx *c, uint32_t P) {
         d.tile_s1 = c->p_tile_s1;
         d.ntiles = c->p_ntiles;
         d.max_tiles = c->p_max_tiles;
-        /* the shared down shares the routed down's launch (2.77 against 2.83 ms
-         * beside the routed gate/up; UOCR_HIP_SHARED_DOWN_WITH=gu for that) */
-        static const int sd_down = [] {
-            const char *e = getenv("UOCR_HIP_SHARED_DOWN_WITH");
-            return e != nullptr && strcmp(e, "gu") == 0 ? 0 : 1;
-        }();
-        if (sd_down) {
-            ENQ(uocr_launch_gemm(s, UOCR_GEMM_SWIGLU, &d));
-        } else {
-            ENQ(uocr_launch_gemm_pair(s, UOCR_GEMM_F16, &dsd, UOCR_GEMM_SWIGLU, &d));
-        }
+        d.a_rows = P;
+        d.pairs = P * UOCR_MOE_TOP_K;
         uocr_gemm_desc dd = d;
         dd.A = c->p_rmid;
         dd.lda = EI;
@@ -1065,15 +1051,20 @@ static hipError_t enqueue_prefill_mfma(uocr_hip_ctx *c, uint32_t P) {
         dd.w_stride = L.slab.dn_w_stride;
         dd.s_stride = L.slab.dn_s_stride;
         dd.a_idx = c->p_list_pair;
+        dd.a_rows = P * UOCR_MOE_TOP_K;
         /* per-pair expert outputs in fp16, as the reference keeps them */
         uint16_t *y16 = c->p_y;
         dd.out = y16;
         dd.ldo = H_SIZE;
-        if (sd_down) {
-            ENQ(uocr_launch_gemm_pair(s, UOCR_GEMM_F16, &dsd, UOCR_GEMM_F16, &dd));
-        } else {
-            ENQ(uocr_launch_gemm(s, UOCR_GEMM_F16, &dd));
-        }
+        d.tile_rows = dd.tile_rows = uocr_moe_tile_rows(UOCR_GEMM_F16, &d, &dd, P);
+        /* the shared experts' GEMMs share launches with GEMMs that do not read
+         * their output: gate/up with the router logits, down with the routed
+         * down */
+        ENQ(uocr_launch_gemm_pair(s, UOCR_GEMM_SWIGLU, &dsg, UOCR_GEMM_F32, &dr));
+        ENQ(uocr_launch_route_rows(s, c->p_logits, P, 0, c->p_ids, c->p_wts, c->p_offsets, c->p_tile_e, c->p_tile_s0, c->p_tile_s1, c->p_ntiles, c->p_list_tok,
+                                   c->p_list_pair, d.tile_rows));
+        ENQ(uocr_launch_gemm(s, UOCR_GEMM_SWIGLU, &d));
+        ENQ(uocr_launch_gemm_pair(s, UOCR_GEMM_F16, &dsd, UOCR_GEMM_F16, &dd));
         if (next_norm != nullptr) {
             ENQ(uocr_launch_moe_combine_norm_h(s, y16, c->p_wts, c->p_sout, c->p_a, P, H, next_norm, c->p_xn));
         } else {

@@ -156,5 +156,15 @@ enum { GO_PLAIN = 0, GO_BY_ROW = 1, GO_BY_COL = 2 };
  * fit them (16-byte aligned rows, 32-bit offsets), and its launch. */
 bool uocr_gemm_tile_fits(int epi, u32 qt, const GemmArgs &a);
 hipError_t uocr_gemm_tile_plain(hipStream_t st, int epi, u32 qt, const GemmArgs &a);
+/* The Q | K | V projection (N = 3 nseg) with RoPE and the cache scatter. */
+hipError_t uocr_gemm_tile_rope(hipStream_t st, u32 qt, GemmArgs a, const RopeDst &rd);
+/* Rows per tile (32 or 128) of the grouped GEMMs over `pairs` (token,
+ * rank) pairs whose tile table holds `table` entries; their launch; a plain
+ * GE_F16 GEMM a beside a grouped one of the same weight type and layout (eb:
+ * GE_F16 or GE_F32); and a plain SwiGLU GEMM a beside fp16 router logits b. */
+u32 uocr_gemm_grouped_rows(u32 pairs, u32 table);
+hipError_t uocr_gemm_tile_grouped(hipStream_t st, int epi, u32 qt, const GemmArgs &a, u32 pairs, u32 rows);
+hipError_t uocr_gemm_tile_pair(hipStream_t st, int eb, u32 qt, const GemmArgs &a, const GemmArgs &b, u32 pairs, u32 rows);
+hipError_t uocr_gemm_tile_router(hipStream_t st, u32 qt, const GemmArgs &a, const GemmArgs &b);
 
 #endif /* UOCR_GEMM_H */

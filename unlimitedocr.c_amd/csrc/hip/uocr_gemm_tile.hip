@@ -14,8 +14,7 @@ namespace {
 /* The block's tile.  Blocks go to the 8 XCDs in turn; with by_row or by_col
  * each XCD takes a contiguous run of row tiles (of column tiles) instead, so
  * that its L2 fetches only its share of the activations (of the weights). */
-__device__ __forceinline__ bool tile_of(u32 order, u32 nx, u32 ny, u32 &bx, u32 &by) {
-    const u32 id = blockIdx.x;
+__device__ __forceinline__ bool tile_of(u32 id, u32 order, u32 nx, u32 ny, u32 &bx, u32 &by) {
     if (order == GO_PLAIN) {
         bx = id % nx;
         by = id / nx;
@@ -309,6 +308,7 @@ __device__ __forceinline__ void tile_body(const GemmArgs &p, u32 bx, u32 by, uin
         constexpr u32 LD = 64u * WN + 8u; /* padded row (halves) */
         h16 *tile = (h16 *)sm;
         wait_barrier<0>();
+        if (WK == 1 || kg == 0) {
 #pragma unroll
         for (int k = 0; k < RT; ++k)
 #pragma unroll
@@ -323,6 +323,7 @@ __device__ __forceinline__ void tile_body(const GemmArgs &p, u32 bx, u32 by, uin
                     for (int x = 0; x < 4; ++x) o.x[x] = (h16)acc[k][j][4 * q + x];
                     *(uint2 *)(tile + (32u * k + r) * LD + 64u * wave + 32u * j + 8u * q + 4u * h) = o.u;
                 }
+        }
         __syncthreads();
         const u32 seg = n0 / p.nseg, h0 = (n0 - seg * p.nseg) / 128u;
         /* 8 pairs (d, d + 64) of one head and row per thread and turn */
@@ -360,7 +361,7 @@ __device__ __forceinline__ void tile_body(const GemmArgs &p, u32 bx, u32 by, uin
     constexpr bool F32O = EPI == GE_F32;
     constexpr u32 CPP = F32O ? 4u : 8u;        /* columns per piece */
     constexpr u32 CH = WN * CW / CPP;          /* pieces per row */
-    constexpr int PASS_RT = F32O && RT > 2 ? 2 : RT; /* 32-row tiles per pass */
+    constexpr int PASS_RT = F32O ? (RT == 4 ? 2 : 1) : RT; /* 32-row tiles per pass */
     static_assert(PASS_RT * 32u * CH * 16u <= tile_lds_bytes<RT, WN, WK>(false), "staging fits");
     const u32 ch = t % CH, col = n0 + CPP * ch; /* the piece this thread moves, in rows t / CH, + TT / CH, .. */
 #pragma unroll
@@ -448,12 +449,54 @@ __device__ __forceinline__ void tile_body(const GemmArgs &p, u32 bx, u32 by, uin
     }
 }
 
+/* One block of a tile grid.  A bucket's last tile of 128 rows takes the body
+ * of 32, 64 or 96 rows when that is all it holds (an expert's bucket of a
+ * 932-token prompt is about 87 rows). */
+template <int QT, int EPI, bool GROUPED, bool PACKED, int RT, int WN, int WK>
+__device__ __forceinline__ void tile_block(const GemmArgs &p, u32 id, uint8_t *sm, const RopeDst &rd) {
+    u32 bx, by;
+    if (!tile_of(id, p.order, GROUPED ? (u32)*p.ntiles : p.nx, p.ny, bx, by)) return;
+    if constexpr (GROUPED && RT == 4) {
+        const u32 rows = uni((u32)p.tile_s1[bx]) - uni((u32)p.tile_s0[bx]);
+        if (rows <= 32u) return tile_body<QT, EPI, GROUPED, PACKED, 1, WN, WK>(p, bx, by, sm, rd);
+        if (rows <= 64u) return tile_body<QT, EPI, GROUPED, PACKED, 2, WN, WK>(p, bx, by, sm, rd);
+        if (rows <= 96u) return tile_body<QT, EPI, GROUPED, PACKED, 3, WN, WK>(p, bx, by, sm, rd);
+    }
+    tile_body<QT, EPI, GROUPED, PACKED, RT, WN, WK>(p, bx, by, sm, rd);
+}
+
 template <int QT, int EPI, bool GROUPED, bool PACKED, int RT, int WN, int WK>
 __global__ __launch_bounds__(64 * WN * WK, 2) void k_gemm_tile(GemmArgs p) {
     __shared__ __attribute__((aligned(1024))) uint8_t sm[tile_lds_bytes<RT, WN, WK>(false)];
-    u32 bx, by;
-    if (!tile_of(p.order, GROUPED ? (u32)*p.ntiles : p.nx, p.ny, bx, by)) return;
-    tile_body<QT, EPI, GROUPED, PACKED, RT, WN, WK>(p, bx, by, sm, RopeDst{});
+    tile_block<QT, EPI, GROUPED, PACKED, RT, WN, WK>(p, blockIdx.x, sm, RopeDst{});
+}
+
+/* The Q | K | V projection with RoPE and the cache scatter as its epilogue. */
+template <int QT, bool PACKED, int RT, int WN, int WK>
+__global__ __launch_bounds__(64 * WN * WK, 2) void k_gemm_tile_rope(GemmArgs p, RopeDst rd) {
+    __shared__ __attribute__((aligned(1024))) uint8_t sm[tile_lds_bytes<RT, WN, WK>(true)];
+    tile_block<QT, GE_ROPE, false, PACKED, RT, WN, WK>(p, blockIdx.x, sm, rd);
+}
+
+/* One of the two GEMMs of a launch: weight type, epilogue, layout and tile. */
+template <int QT_, int EPI_, bool GROUPED_, bool PACKED_, int RT_, int WN_, int WK_>
+struct Half {
+    static constexpr int QT = QT_, EPI = EPI_, RT = RT_, WN = WN_, WK = WK_;
+    static constexpr bool GROUPED = GROUPED_, PACKED = PACKED_;
+    static constexpr u32 LDS = tile_lds_bytes<RT_, WN_, WK_>(false), CW = (EPI_ == GE_SWIGLU ? 32u : 64u) * WN_;
+    static_assert(WN_ * WK_ == 4, "both halves run 256 threads");
+    static __device__ __forceinline__ void block(const GemmArgs &p, u32 id, uint8_t *sm) {
+        tile_block<QT, EPI, GROUPED, PACKED, RT, WN, WK>(p, id, sm, RopeDst{});
+    }
+};
+
+/* Two GEMMs that do not read each other's output in one launch: blocks [0, na)
+ * take A's tiles, the others B's. */
+template <typename A, typename B>
+__global__ __launch_bounds__(256, 2) void k_gemm_tile_pair(GemmArgs a, u32 na, GemmArgs b) {
+    __shared__ __attribute__((aligned(1024))) uint8_t sm[A::LDS > B::LDS ? A::LDS : B::LDS];
+    if (blockIdx.x < na) A::block(a, blockIdx.x, sm);
+    else B::block(b, blockIdx.x - na, sm);
 }
 
 /* ---- narrow tiles, K split over the block's wavefronts ---------------------- */
@@ -462,15 +505,14 @@ __global__ __launch_bounds__(64 * WN * WK, 2) void k_gemm_tile(GemmArgs p) {
 #define KS_PLANE (8u * 1040u)           /* bytes of a wavefront's 32 x 64 partials: 8 pieces of 64 float4, padded */
 
 template <int QT, int EPI, bool GROUPED, bool PACKED>
-__global__ __launch_bounds__(64u * KS_WAVES) void k_gemm_ksplit(GemmArgs p) {
+__device__ __forceinline__ void lines_block(const GemmArgs &p, u32 id, uint8_t *ksm) {
     constexpr int NG = groups_per_line<QT>();
     constexpr bool SW = EPI == GE_SWIGLU;
     constexpr int RT = 1; /* 32-row tiles (2 measured slower at 32 to 4096 rows) */
     constexpr u32 CW = SW ? 32u : 64u, ROWS = 32u * RT, RB = QT == 4 ? 32u : 64u;
-    extern __shared__ __attribute__((aligned(16))) uint8_t ksm[];
     const u32 t = threadIdx.x, lane = t & 63u, wave = uni(t >> 6), r = lane & 31u, h = lane >> 5, nw = blockDim.x / 64u;
     u32 bx, by;
-    if (!tile_of(p.order, GROUPED ? (u32)*p.ntiles : p.nx, p.ny, bx, by)) return;
+    if (!tile_of(id, p.order, GROUPED ? (u32)*p.ntiles : p.nx, p.ny, bx, by)) return;
     const u32 n0 = by * CW;
     u32 e = 0, s0 = bx * ROWS, rows;
     if (GROUPED) {
@@ -650,6 +692,19 @@ __global__ __launch_bounds__(64u * KS_WAVES) void k_gemm_ksplit(GemmArgs p) {
     }
 }
 
+template <int QT, int EPI, bool GROUPED, bool PACKED>
+__global__ __launch_bounds__(64u * KS_WAVES) void k_gemm_lines(GemmArgs p) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t ksm[];
+    lines_block<QT, EPI, GROUPED, PACKED>(p, blockIdx.x, ksm);
+}
+
+template <int QT, int EA, int EB, bool PACKED>
+__global__ __launch_bounds__(64u * KS_WAVES) void k_gemm_lines_pair(GemmArgs a, u32 na, GemmArgs b) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t ksm[];
+    if (blockIdx.x < na) lines_block<QT, EA, false, PACKED>(a, blockIdx.x, ksm);
+    else lines_block<QT, EB, true, PACKED>(b, blockIdx.x - na, ksm);
+}
+
 /* The launch's blocks and the order of its tiles. */
 dim3 tile_grid(GemmArgs &a, u32 row_tiles, u32 col_tiles, u32 qt, bool grouped) {
     a.nx = row_tiles;
@@ -660,17 +715,17 @@ dim3 tile_grid(GemmArgs &a, u32 row_tiles, u32 col_tiles, u32 qt, bool grouped) 
 }
 
 /* Wavefronts per block: as many lines of 128 bytes each, at most KS_WAVES. */
-u32 ksplit_waves(u32 qt, u32 K) {
+u32 lines_waves(u32 qt, u32 K) {
     const u32 ng = qt == UOCR_QT_Q4 ? 4u : (qt == UOCR_QT_Q8 ? 2u : 1u), nch = (K / 64u + ng - 1u) / ng;
     const u32 per = (nch + KS_WAVES - 1u) / KS_WAVES;
     return (nch + per - 1u) / per;
 }
 
 template <int EPI, bool GROUPED>
-hipError_t launch_ksplit(hipStream_t st, u32 qt, GemmArgs a, u32 row_tiles) {
-    const u32 nw = ksplit_waves(qt, a.K), cw = EPI == GE_SWIGLU ? 32u : 64u;
+hipError_t launch_lines(hipStream_t st, u32 qt, GemmArgs a, u32 row_tiles) {
+    const u32 nw = lines_waves(qt, a.K), cw = EPI == GE_SWIGLU ? 32u : 64u;
     const dim3 grid = tile_grid(a, row_tiles, (a.N + cw - 1u) / cw, qt, GROUPED);
-#define GO(Q, PK) hipLaunchKernelGGL((k_gemm_ksplit<Q, EPI, GROUPED, PK>), grid, dim3(64u * nw), nw * KS_PLANE, st, a)
+#define GO(Q, PK) hipLaunchKernelGGL((k_gemm_lines<Q, EPI, GROUPED, PK>), grid, dim3(64u * nw), nw * KS_PLANE, st, a)
     if (qt == UOCR_QT_F16) GO(1, false);
     else if (qt == UOCR_QT_Q8 && a.packed) GO(3, true);
     else if (qt == UOCR_QT_Q8) GO(3, false);
@@ -709,10 +764,10 @@ hipError_t plain(hipStream_t st, int epi, u32 qt, const GemmArgs &a) {
 hipError_t plain_lines(hipStream_t st, int epi, u32 qt, const GemmArgs &a) {
     const u32 tiles = (a.M + 31u) / 32u;
     switch (epi) {
-        case GE_F16: return launch_ksplit<GE_F16, false>(st, qt, a, tiles);
-        case GE_F32: return launch_ksplit<GE_F32, false>(st, qt, a, tiles);
-        case GE_VISION: return launch_ksplit<GE_VISION, false>(st, qt, a, tiles);
-        case GE_SWIGLU: return launch_ksplit<GE_SWIGLU, false>(st, qt, a, tiles);
+        case GE_F16: return launch_lines<GE_F16, false>(st, qt, a, tiles);
+        case GE_F32: return launch_lines<GE_F32, false>(st, qt, a, tiles);
+        case GE_VISION: return launch_lines<GE_VISION, false>(st, qt, a, tiles);
+        case GE_SWIGLU: return launch_lines<GE_SWIGLU, false>(st, qt, a, tiles);
         default: return hipErrorInvalidValue;
     }
 }
@@ -750,6 +805,103 @@ bool uocr_gemm_tile_fits(int epi, u32 qt, const GemmArgs &a) {
     uintptr_t al = (uintptr_t)a.A | (uintptr_t)a.W[0].w | (epi == GE_SWIGLU ? (uintptr_t)a.W[1].w : 0u);
     return a.vec != 0u && (epi == GE_F16 || epi == GE_F32 || epi == GE_SWIGLU || epi == GE_VISION) && a.nseg == 0u && al % 16u == 0u &&
            (uint64_t)a.M * a.lda * 2u < lim && (uint64_t)a.M * a.ldr * 2u < lim && a.N * rowb < lim && (!a.packed || a.N % 32u == 0u);
+}
+
+hipError_t uocr_gemm_tile_rope(hipStream_t st, u32 qt, GemmArgs a, const RopeDst &rd) {
+    /* 932 rows: 64 x 128 tiles, K in 2 (450 blocks); from 160 large tiles on
+     * those (a head pair per tile) */
+    const bool large = choose(false, a.M, a.N, a.K) == CFG_LARGE;
+    const dim3 grid = tile_grid(a, (a.M + (large ? 127u : 63u)) / (large ? 128u : 64u), a.N / (large ? 256u : 128u), qt, false);
+#define GO(Q, PK)                                                                                                      \
+    do {                                                                                                               \
+        if (large) hipLaunchKernelGGL((k_gemm_tile_rope<Q, PK, 4, 4, 1>), grid, dim3(256), 0, st, a, rd);              \
+        else hipLaunchKernelGGL((k_gemm_tile_rope<Q, PK, 2, 2, 2>), grid, dim3(256), 0, st, a, rd);                    \
+    } while (0)
+    if (qt == UOCR_QT_F16) GO(1, false);
+    else if (qt == UOCR_QT_Q8 && a.packed) GO(3, true);
+    else if (qt == UOCR_QT_Q8) GO(3, false);
+    else if (a.packed) GO(4, true);
+    else GO(4, false);
+#undef GO
+    return hipGetLastError();
+}
+
+/* Row tiles of a grouped launch at most: a bucket's last tile may be partial. */
+static u32 grouped_tiles(u32 pairs, u32 tile_rows) {
+    const u32 t = pairs / tile_rows + UOCR_K_EXPERTS;
+    return t < pairs ? t : pairs;
+}
+
+u32 uocr_gemm_grouped_rows(u32 pairs, u32 table) {
+    /* whole MoE of P rows (us, 128-row tiles / weight lines): Q4 P = 2: 56 / 43,
+     * 9: 67 / 66, 23: 77 / 86; Q8 2: 55 / 47, 9: 75 / 84 */
+    return pairs <= 36u && grouped_tiles(pairs, 32u) <= table ? 32u : 128u;
+}
+
+hipError_t uocr_gemm_tile_grouped(hipStream_t st, int epi, u32 qt, const GemmArgs &a, u32 pairs, u32 rows) {
+    const u32 tiles = grouped_tiles(pairs, rows);
+#define GO(E) return rows == 32u ? launch_lines<E, true>(st, qt, a, tiles) : launch<E, true, 4, 4, 1>(st, qt, a, tiles)
+    switch (epi) {
+        case GE_F16: GO(GE_F16);
+        case GE_F32: GO(GE_F32);
+        case GE_SWIGLU: GO(GE_SWIGLU);
+        default: return hipErrorInvalidValue;
+    }
+#undef GO
+}
+
+namespace {
+
+template <typename A, typename B>
+void launch_halves(hipStream_t st, u32 qa, GemmArgs a, u32 ta, u32 qb, GemmArgs b, u32 tb) {
+    const dim3 ga = tile_grid(a, ta, (a.N + A::CW - 1u) / A::CW, qa, A::GROUPED);
+    const dim3 gb = tile_grid(b, tb, (b.N + B::CW - 1u) / B::CW, qb, B::GROUPED);
+    hipLaunchKernelGGL((k_gemm_tile_pair<A, B>), dim3(ga.x + gb.x), dim3(256), 0, st, a, ga.x, b);
+}
+
+/* The plain GEMM a, EPI GE_F16, beside the grouped b. */
+template <int EB>
+hipError_t launch_pair(hipStream_t st, u32 qt, GemmArgs a, GemmArgs b, u32 pairs, u32 rows) {
+    const u32 tiles = grouped_tiles(pairs, rows), ta = (a.M + 63u) / 64u;
+    if (rows == 32u) {
+        const u32 wa = lines_waves(qt, a.K), wb = lines_waves(qt, b.K), nw = wa > wb ? wa : wb;
+        const dim3 ga = tile_grid(a, (a.M + 31u) / 32u, (a.N + 63u) / 64u, qt, false), gb = tile_grid(b, tiles, (b.N + 63u) / 64u, qt, true);
+#define GO(Q, PK) hipLaunchKernelGGL((k_gemm_lines_pair<Q, GE_F16, EB, PK>), dim3(ga.x + gb.x), dim3(64u * nw), nw * KS_PLANE, st, a, ga.x, b)
+        if (qt == UOCR_QT_F16) GO(1, false);
+        else if (qt == UOCR_QT_Q8 && a.packed) GO(3, true);
+        else if (qt == UOCR_QT_Q8) GO(3, false);
+        else if (a.packed) GO(4, true);
+        else GO(4, false);
+#undef GO
+        return hipGetLastError();
+    }
+#define GO(Q, PK) launch_halves<Half<Q, GE_F16, false, PK, 2, 2, 2>, Half<Q, EB, true, PK, 4, 4, 1>>(st, qt, a, ta, qt, b, tiles)
+    if (qt == UOCR_QT_F16) GO(1, false);
+    else if (qt == UOCR_QT_Q8 && a.packed) GO(3, true);
+    else if (qt == UOCR_QT_Q8) GO(3, false);
+    else if (a.packed) GO(4, true);
+    else GO(4, false);
+#undef GO
+    return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t uocr_gemm_tile_pair(hipStream_t st, int eb, u32 qt, const GemmArgs &a, const GemmArgs &b, u32 pairs, u32 rows) {
+    return eb == GE_F16 ? launch_pair<GE_F16>(st, qt, a, b, pairs, rows) : launch_pair<GE_F32>(st, qt, a, b, pairs, rows);
+}
+
+hipError_t uocr_gemm_tile_router(hipStream_t st, u32 qt, const GemmArgs &a, const GemmArgs &b) {
+    const u32 ta = (a.M + 63u) / 64u, tb = (b.M + 31u) / 32u;
+    typedef Half<1, GE_F32, false, false, 1, 1, 4> R;
+#define GO(Q, PK) launch_halves<Half<Q, GE_SWIGLU, false, PK, 2, 2, 2>, R>(st, qt, a, ta, UOCR_QT_F16, b, tb)
+    if (qt == UOCR_QT_F16) GO(1, false);
+    else if (qt == UOCR_QT_Q8 && a.packed) GO(3, true);
+    else if (qt == UOCR_QT_Q8) GO(3, false);
+    else if (a.packed) GO(4, true);
+    else GO(4, false);
+#undef GO
+    return hipGetLastError();
 }
 
 hipError_t uocr_gemm_tile_plain(hipStream_t st, int epi, u32 qt, const GemmArgs &a) {

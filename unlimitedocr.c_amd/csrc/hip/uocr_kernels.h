@@ -233,6 +233,9 @@ typedef struct uocr_gemm_desc {
     uint64_t w_stride, s_stride;
     const int32_t *tile_e, *tile_s0, *tile_s1, *ntiles;
     uint32_t max_tiles;
+    /* grouped: rows of A, and the rows per tile that the table was built with
+     * (uocr_gemm_grouped_rows; 0: the general kernel's 64) */
+    uint32_t a_rows, tile_rows, pairs;
     void *out;
     uint32_t ldo;
     const uint16_t *res;
@@ -262,11 +265,9 @@ hipError_t uocr_launch_gemm(hipStream_t st, int epi, const uocr_gemm_desc *d);
 /* 1 when uocr_launch_gemm runs d in one launch that needs no partials (ksplit
  * and part are then ignored). */
 int uocr_gemm_splits_itself(int epi, const uocr_gemm_desc *d);
-/* Two independent GEMMs in one launch (blocks split between their tile
- * grids): A plain SwiGLU with B the fp16 router (F32), or A plain F16 with B
- * grouped SwiGLU or grouped F32 of the same qtype; neither split-K, fused
- * norm nor nseg.
- * Other pairs, or UOCR_HIP_GEMM_PAIR=0, run as two launches. */
+/* Two independent GEMMs in one launch where both fit the tiled kernels: A
+ * plain F16 with B grouped F16 or F32 of the same weight type and layout, or A
+ * plain SwiGLU with B plain fp16 F32 (the router); two launches else. */
 hipError_t uocr_launch_gemm_pair(hipStream_t st, int epi_a, const uocr_gemm_desc *da, int epi_b,
                                  const uocr_gemm_desc *db);
 /* GEMM-packed copy of a Q4_0 / Q8_0 payload of `rows` x K (rows % 32 == 0,
@@ -295,14 +296,20 @@ hipError_t uocr_launch_gemm_qkv_rope(hipStream_t st, const uocr_gemm_desc *d, co
 hipError_t uocr_launch_flash_attn(hipStream_t st, const uint16_t *q, const uint16_t *kcache, const uint16_t *vcache,
                                   uint32_t cap, uint32_t P, uint16_t *ctx);
 /* Per-token top-6 over logits [P][64] -> ids/wts [P][6]; expert buckets:
- * offsets (64), grouped-GEMM tile table (up to P*6/64 + 64 entries) and the
+ * offsets (64), grouped-GEMM tile table (up to P*6/tile_rows + 64 entries;
+ * tile_rows 0 means 64) and the
  * (token, pair) slot lists [P*6], built in LDS by one block (no global
  * counters, nothing to clear between calls, so the call can be captured
  * into a graph). */
 hipError_t uocr_launch_route_rows(hipStream_t st, const float *logits, uint32_t P, int norm_topk, int32_t *ids,
                                   float *wts, int32_t *offsets, int32_t *tile_e,
                                   int32_t *tile_s0, int32_t *tile_s1, int32_t *ntiles, int32_t *list_tok,
-                                  int32_t *list_pair);
+                                  int32_t *list_pair, uint32_t tile_rows);
+/* Rows per tile for the grouped GEMMs of gu and dn over P x 6 pairs with a
+ * table of max_tiles entries (pass it to uocr_launch_route_rows and in
+ * tile_rows): 0 (64-row tiles, general kernel) where their operands do not
+ * fit the tiled kernels. */
+uint32_t uocr_moe_tile_rows(int epi_dn, const uocr_gemm_desc *gu, const uocr_gemm_desc *dn, uint32_t P);
 /* out[t] = f16(sum_r wts[t][r] * Y[t*6+r] + shared[t] + res[t]). */
 /* uocr_launch_moe_combine, then norm_out = f16(rmsnorm(out) * norm_w) of each
  * row (the next layer's input norm), in one launch. */

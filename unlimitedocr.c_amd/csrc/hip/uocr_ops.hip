@@ -352,8 +352,9 @@ extern "C" int uocr_op_gemm(uint32_t qtype, const void *w, const void *s, uint32
 static float *g_vision_part = nullptr;
 static size_t g_vision_part_bytes = 0;
 /* Guards the lazily allocated operator buffer (g_vision_part): held from the
- * size check through the launch, so two threads never allocate twice or launch into a buffer being replaced; the
- * launches then serialise on the operator stream. */
+ * size check through the launch, so two threads never allocate twice or launch
+ * into a buffer being replaced; the launches then serialise on the operator
+ * stream. */
 static pthread_mutex_t g_lazy_mu = PTHREAD_MUTEX_INITIALIZER;
 struct lazy_lock {
     lazy_lock() { pthread_mutex_lock(&g_lazy_mu); }
@@ -499,7 +500,7 @@ static int moe_rows(hipStream_t st, const uocr_op_moe_weights *m, const void *x,
     } else {
         r = hip_status(hipMemcpyAsync(xn, x, (size_t)P * 1280u * 2u, hipMemcpyDeviceToDevice, st), "copy");
     }
-    uocr_gemm_desc d;
+    uocr_gemm_desc d; /* router logits */
     memset(&d, 0, sizeof(d));
     d.A = xn;
     d.lda = 1280u;
@@ -509,22 +510,15 @@ static int moe_rows(hipStream_t st, const uocr_op_moe_weights *m, const void *x,
     d.W[0] = qm(UOCR_QT_F16, m->router, nullptr);
     d.out = b + L.logits;
     d.ldo = 64u;
-    if (r == UOCR_OK) r = hip_status(uocr_launch_gemm(st, UOCR_GEMM_F32, &d), "router gemm");
     int32_t *ids = (int32_t *)(b + L.ids);
     float *wts = (float *)(b + L.wts);
-    if (r == UOCR_OK) {
-        r = hip_status(uocr_launch_route_rows(st, (const float *)(b + L.logits), P, norm_topk, ids, wts,
-                                              (int32_t *)(b + L.offsets), (int32_t *)(b + L.te), (int32_t *)(b + L.ts0),
-                                              (int32_t *)(b + L.ts1), (int32_t *)(b + L.nt), (int32_t *)(b + L.ltok),
-                                              (int32_t *)(b + L.lpair)),
-                       "routing");
-    }
-    d.N = 1792u;
-    d.W[0] = qm(m->shared_qtype, m->sgate_w, m->sgate_s);
-    d.W[1] = qm(m->shared_qtype, m->sup_w, m->sup_s);
-    d.out = b + L.smid;
-    d.ldo = 1792u;
-    if (r == UOCR_OK) r = hip_status(uocr_launch_gemm(st, UOCR_GEMM_SWIGLU, &d), "shared gate/up gemm");
+    uocr_gemm_desc sg = d;
+    sg.N = 1792u;
+    sg.W[0] = qm(m->shared_qtype, m->sgate_w, m->sgate_s);
+    sg.W[1] = qm(m->shared_qtype, m->sup_w, m->sup_s);
+    sg.out = b + L.smid;
+    sg.ldo = 1792u;
+    if (r == UOCR_OK) r = hip_status(uocr_launch_gemm_pair(st, UOCR_GEMM_SWIGLU, &sg, UOCR_GEMM_F32, &d), "router and shared gate/up gemm");
     uocr_gemm_desc sd;
     memset(&sd, 0, sizeof(sd));
     sd.A = (const uint16_t *)(b + L.smid);
@@ -535,7 +529,6 @@ static int moe_rows(hipStream_t st, const uocr_op_moe_weights *m, const void *x,
     sd.W[0] = qm(m->shared_qtype, m->sdown_w, m->sdown_s);
     sd.out = b + L.sout;
     sd.ldo = 1280u;
-    if (r == UOCR_OK) r = hip_status(uocr_launch_gemm(st, UOCR_GEMM_F16, &sd), "shared down gemm");
     uocr_gemm_desc gd;
     memset(&gd, 0, sizeof(gd));
     gd.A = xn;
@@ -553,9 +546,10 @@ static int moe_rows(hipStream_t st, const uocr_op_moe_weights *m, const void *x,
     gd.tile_s1 = (const int32_t *)(b + L.ts1);
     gd.ntiles = (const int32_t *)(b + L.nt);
     gd.max_tiles = L.max_tiles;
+    gd.a_rows = P;
+    gd.pairs = P * 6u;
     gd.out = b + L.rmid;
     gd.ldo = 896u;
-    if (r == UOCR_OK) r = hip_status(uocr_launch_gemm(st, UOCR_GEMM_SWIGLU, &gd), "routed gate/up gemm");
     uocr_gemm_desc dd = gd;
     dd.A = (const uint16_t *)(b + L.rmid);
     dd.lda = 896u;
@@ -566,9 +560,19 @@ static int moe_rows(hipStream_t st, const uocr_op_moe_weights *m, const void *x,
     dd.w_stride = m->dn_w_stride;
     dd.s_stride = m->dn_s_stride;
     dd.a_idx = (const int32_t *)(b + L.lpair);
+    dd.a_rows = P * 6u;
     dd.out = b + L.y;
     dd.ldo = 1280u;
-    if (r == UOCR_OK) r = hip_status(uocr_launch_gemm(st, UOCR_GEMM_F32, &dd), "routed down gemm");
+    gd.tile_rows = dd.tile_rows = uocr_moe_tile_rows(UOCR_GEMM_F32, &gd, &dd, P);
+    if (r == UOCR_OK) {
+        r = hip_status(uocr_launch_route_rows(st, (const float *)(b + L.logits), P, norm_topk, ids, wts,
+                                              (int32_t *)(b + L.offsets), (int32_t *)(b + L.te), (int32_t *)(b + L.ts0),
+                                              (int32_t *)(b + L.ts1), (int32_t *)(b + L.nt), (int32_t *)(b + L.ltok),
+                                              (int32_t *)(b + L.lpair), gd.tile_rows),
+                       "routing");
+    }
+    if (r == UOCR_OK) r = hip_status(uocr_launch_gemm(st, UOCR_GEMM_SWIGLU, &gd), "routed gate/up gemm");
+    if (r == UOCR_OK) r = hip_status(uocr_launch_gemm_pair(st, UOCR_GEMM_F16, &sd, UOCR_GEMM_F32, &dd), "down gemm");
     if (r == UOCR_OK) {
         r = hip_status(uocr_launch_moe_combine(st, (const float *)(b + L.y), wts, (const uint16_t *)(b + L.sout),
                                                (const uint16_t *)residual, P, (uint16_t *)out),

@@ -26,7 +26,6 @@
 
 #define PB 256 /* threads per prefill block */
 #define TM 64  /* GEMM tile rows */
-#define GTM TM /* tile rows of the grouped (expert-bucket) GEMMs */
 #define TN 128 /* GEMM tile columns */
 #define TK 64  /* one quantisation group */
 #define LDA (TK + 8) /* padded LDS row of the activation tile (halves) */
@@ -113,7 +112,7 @@ __device__ __forceinline__ void b_dequant(const u32 (&w)[BPiece<QT>::NW], u32 sc
 #endif
 
 template <int QT, int EPI, bool GROUPED, int TMR>
-__device__ __forceinline__ void gemm_body(GemmArgs p, u32 bx, u32 by, u32 bz, RopeDst rd = RopeDst{}) {
+__device__ __forceinline__ void gemm_body(GemmArgs p, u32 bx, u32 by, u32 bz) {
     constexpr int AQ4 = TMR * (TK / 8) / PB; /* activation pieces (8 halves) per thread per K step */
     static_assert(TMR % 32 == 0 && TMR <= PB && AQ4 * PB == TMR * (TK / 8), "tile rows");
     constexpr int NMAT = EPI == GE_SWIGLU ? 2 : 1;
@@ -324,61 +323,6 @@ __device__ __forceinline__ void gemm_body(GemmArgs p, u32 bx, u32 by, u32 bz, Ro
         if (st + (u32)decltype(D)::value < NS) step(D, st + (u32)decltype(D)::value);
     });
 
-    if constexpr (EPI == GE_ROPE) {
-        /* The Q | K | V projection with RoPE and the cache scatter as its
-         * epilogue: the block's 128 columns are one head of one of the three
-         * segments.  The tile is rounded to fp16 (the projection's output
-         * type) into LDS, then wavefront w takes rows w, w + 4, ..: lane d
-         * rotates the pair (x_d, x_{d+64}) in fp32 by the angle tok * f[d],
-         * cos and sin from the prompt's table (q and k; v is copied). */
-        static_assert(GROUPED == false && TMR == 64 && TN == UOCR_K_HEAD_DIM, "rope tile");
-        constexpr u32 RLD = TN + 8u; /* padded LDS row (halves) */
-        static_assert(TMR * RLD <= 2u * TMR * LDA, "rope tile in the activation buffers");
-        h16 *tile = &as[0][0];
-        const u32 seg = n0 / p.nseg, h = (n0 - seg * p.nseg) / TN, d = lane;
-        __syncthreads(); /* every wavefront's last MFMA reads of as[] are done */
-#pragma unroll
-        for (int j = 0; j < TMR / 32; ++j)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const u32 r = 32u * j + 8u * (i / 4) + 4u * hf + (i % 4);
-                tile[r * RLD + 32u * wave + (lane & 31u)] = (h16)acc[0][j][i];
-            }
-        /* the wavefront's cos / sin loads, all in flight across the barrier
-         * (issued after the accumulators are staged, so they add no
-         * registers to the main loop's) */
-        constexpr int RW = TMR / (PB / 64); /* rows per wavefront */
-        float2 csr[RW];
-        if (seg != 2u) {
-#pragma unroll
-            for (int k = 0; k < RW; ++k) {
-                const u32 r = min(wave + (PB / 64u) * k, rows - 1u);
-                csr[k] = rd.cs[(size_t)(s0 + r) * 64u + d];
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < RW; ++k) {
-            const u32 r = wave + (PB / 64u) * k;
-            if (r >= rows) break;
-            const u32 tok = s0 + r;
-            const h16 xa = tile[r * RLD + d], xb = tile[r * RLD + d + 64u];
-            if (seg == 2u) {
-                const size_t ci = ((size_t)h * rd.cap + tok) * UOCR_K_HEAD_DIM + d;
-                rd.v[ci] = xa;
-                rd.v[ci + 64u] = xb;
-                continue;
-            }
-            const float cs = csr[k].x, sn = csr[k].y;
-            const float a = (float)xa, b = (float)xb;
-            h16 *dst = seg == 0u ? rd.q + (size_t)tok * UOCR_K_HIDDEN + h * UOCR_K_HEAD_DIM + d
-                                 : rd.k + ((size_t)h * rd.cap + tok) * UOCR_K_HEAD_DIM + d;
-            dst[0] = (h16)(a * cs - b * sn);
-            dst[64] = (h16)(a * sn + b * cs);
-        }
-        return;
-    }
-
     /* C layout of a 32x32 MFMA tile: lane l, element i -> row 8*(i/4) +
      * 4*(l/32) + i%4, column l%32.  Everything that depends only on the
      * column (output pointer, split routing, bias) is resolved once per lane;
@@ -431,34 +375,12 @@ __global__ __launch_bounds__(PB) void k_gemm(GemmArgs p) {
     gemm_body<QT, EPI, GROUPED, TMR>(p, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
-template <int QT>
-__global__ __launch_bounds__(PB) void k_gemm_rope(GemmArgs p, const float2 *cs, h16 *q, h16 *kc, h16 *vc, u32 cap) {
-    gemm_body<QT, GE_ROPE, false, TM>(p, blockIdx.x, blockIdx.y, 0u, RopeDst{cs, q, kc, vc, cap});
-}
-
 /* cs[64 t + d] = (cos, sin)(t * f[d]) for the P prompt tokens. */
 __global__ __launch_bounds__(PB) void k_rope_table(RopeTabP rope, u32 P, float2 *__restrict__ cs) {
     const u32 idx = blockIdx.x * PB + threadIdx.x;
     if (idx >= P * 64u) return;
     const float ang = (float)(idx / 64u) * rope.f[idx % 64u];
     cs[idx] = make_float2(cosf(ang), sinf(ang));
-}
-
-/* Two independent GEMMs in one launch: blocks [0, na) run A's tile grid
- * (ax columns of tiles), the rest B's (bx columns).  For GEMMs that read the
- * same input or at least not each other's output, and that each leave most
- * CUs idle or waiting (the router logits beside the shared gate/up, the
- * shared down beside the routed down): one launch overlaps them where a second
- * stream would turn the captured graph into a slower parallel one. */
-template <int QA, int EA, bool GA, int QB, int EB, bool GB>
-__global__ __launch_bounds__(PB) void k_gemm_pair(GemmArgs a, u32 ax, u32 na, GemmArgs b, u32 bx) {
-    const u32 i = blockIdx.x;
-    if (i < na) {
-        gemm_body<QA, EA, GA, TM>(a, i % ax, i / ax, 0u);
-    } else {
-        const u32 j = i - na;
-        gemm_body<QB, EB, GB, TM>(b, j % bx, j / bx, 0u);
-    }
 }
 
 /* Split-K epilogue: the z partials summed in order (the result does not
@@ -692,7 +614,7 @@ __global__ __launch_bounds__(PB) void k_route_rows(const float *__restrict__ log
 
 /* One block builds the expert buckets of all P*6 (token, rank) pairs in
  * LDS: the 64 bucket sizes (LDS atomics), their exclusive scan (offsets),
- * the tile table of the grouped GEMMs (TM rows per tile) and every pair's
+ * the tile table of the grouped GEMMs (tile_rows rows per tile) and every pair's
  * slot in its bucket (list_tok, list_pair).  The order of pairs inside a
  * bucket does not matter: each pair's row is computed on its own and the
  * combine reads it by pair index.  Nothing is left in global memory that the
@@ -705,7 +627,7 @@ __global__ __launch_bounds__(BUCKET_THREADS) void k_bucket_build(const int32_t *
                                                                  int32_t *__restrict__ tile_s1,
                                                                  int32_t *__restrict__ ntiles,
                                                                  int32_t *__restrict__ list_tok,
-                                                                 int32_t *__restrict__ list_pair) {
+                                                                 int32_t *__restrict__ list_pair, int32_t tile_rows) {
     __shared__ int32_t cnt[64], off[65], toff[65], cur[64];
     const u32 t = threadIdx.x, n = P * UOCR_K_TOPK;
     if (t < 64u) {
@@ -734,7 +656,7 @@ __global__ __launch_bounds__(BUCKET_THREADS) void k_bucket_build(const int32_t *
     if (t < 64u) {
         /* exclusive scans of the bucket sizes and tile counts: one wavefront,
          * a lane per expert */
-        const int32_t c = cnt[t], tl = (c + GTM - 1) / GTM;
+        const int32_t c = cnt[t], tl = (c + tile_rows - 1) / tile_rows;
         int32_t a = c, b = tl;
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
@@ -756,11 +678,11 @@ __global__ __launch_bounds__(BUCKET_THREADS) void k_bucket_build(const int32_t *
     if (t < 64u) {
         offsets[t] = off[t];
         const int32_t c = cnt[t];
-        for (int32_t k = 0; k * GTM < c; ++k) {
+        for (int32_t k = 0; k * tile_rows < c; ++k) {
             const int32_t ti = toff[t] + k;
             tile_e[ti] = (int32_t)t;
-            tile_s0[ti] = off[t] + k * GTM;
-            tile_s1[ti] = off[t] + min(c, (k + 1) * GTM);
+            tile_s0[ti] = off[t] + k * tile_rows;
+            tile_s1[ti] = off[t] + min(c, (k + 1) * tile_rows);
         }
     }
     if (inreg) {
@@ -965,7 +887,7 @@ static GemmArgs gemm_args(const uocr_gemm_desc *d) {
     a.lda = d->lda;
     a.a_idx = d->a_idx;
     a.o_idx = d->o_idx;
-    a.M = d->M;
+    a.M = d->tile_e != nullptr ? d->a_rows : d->M;
     a.N = d->N;
     a.K = d->K;
     for (int i = 0; i < 3; ++i) a.W[i] = d->W[i];
@@ -1021,6 +943,7 @@ extern "C" hipError_t uocr_launch_gemm(hipStream_t st, int epi, const uocr_gemm_
         return hipErrorInvalidValue;
     }
     const bool fuse_norm = want_norm && splittable;
+    if (grouped && d->tile_rows != 0u) return uocr_gemm_tile_grouped(st, epi, qt, a, d->pairs, d->tile_rows);
     if (!grouped && uocr_gemm_tile_fits(epi, qt, a)) {
         const hipError_t e = uocr_gemm_tile_plain(st, epi, qt, a);
         if (e != hipSuccess || !want_norm) return e;
@@ -1069,103 +992,32 @@ extern "C" hipError_t uocr_launch_gemm(hipStream_t st, int epi, const uocr_gemm_
     return hipGetLastError();
 }
 
-/* Scales in LDS for a paired GEMM (as gemm_dispatch decides them). */
-static size_t gemm_scales(u32 qt, u32 nmat, GemmArgs &a) {
-    const u32 nt = a.K / TK;
-    a.sc_lds = qt != UOCR_QT_F16 && nmat * nt <= SC_LDS_STEPS ? 1u : 0u;
-    return a.sc_lds ? (size_t)nmat * TN * nt * sizeof(unsigned short) : 0;
+extern "C" uint32_t uocr_moe_tile_rows(int epi_dn, const uocr_gemm_desc *gu, const uocr_gemm_desc *dn, uint32_t P) {
+    const bool strides = (gu->w_stride | dn->w_stride) % 16u == 0u;
+    if (!strides || !uocr_gemm_tile_fits(UOCR_GEMM_SWIGLU, gu->W[0].qtype, gemm_args(gu)) ||
+        !uocr_gemm_tile_fits(epi_dn, dn->W[0].qtype, gemm_args(dn))) {
+        return 0u;
+    }
+    return uocr_gemm_grouped_rows(P * UOCR_K_TOPK, gu->max_tiles);
 }
 
 extern "C" hipError_t uocr_launch_gemm_pair(hipStream_t st, int epi_a, const uocr_gemm_desc *da, int epi_b,
                                             const uocr_gemm_desc *db) {
     if (!gemm_desc_ok(epi_a, da) || !gemm_desc_ok(epi_b, db)) return hipErrorInvalidValue;
-    static const int on = [] {
-        const char *e = getenv("UOCR_HIP_GEMM_PAIR");
-        return e == nullptr ? 1 : atoi(e);
-    }();
-    const u32 qa = da->W[0].qtype, qb = db->W[0].qtype;
-    auto simple = [](const uocr_gemm_desc *d) {
-        return !(d->ksplit > 1u && d->part != nullptr) && d->norm_w == nullptr && d->nseg == 0u;
-    };
-    const bool ok = on != 0 && simple(da) && simple(db) && da->tile_e == nullptr;
-    const bool router = ok && epi_a == UOCR_GEMM_SWIGLU && epi_b == UOCR_GEMM_F32 && db->tile_e == nullptr &&
-                        qb == UOCR_QT_F16;
-    const bool experts = ok && epi_a == UOCR_GEMM_F16 && epi_b == UOCR_GEMM_SWIGLU && db->tile_e != nullptr && qa == qb;
-    const bool downs = ok && epi_a == UOCR_GEMM_F16 && epi_b == UOCR_GEMM_F32 && db->tile_e != nullptr && qa == qb;
-    const bool downs16 = ok && epi_a == UOCR_GEMM_F16 && epi_b == UOCR_GEMM_F16 && db->tile_e != nullptr && qa == qb;
-    if (!router && !experts && !downs && !downs16) {
-        const hipError_t e = uocr_launch_gemm(st, epi_a, da);
-        return e != hipSuccess ? e : uocr_launch_gemm(st, epi_b, db);
-    }
-    GemmArgs a = gemm_args(da), b = gemm_args(db);
-    const size_t sa = gemm_scales(qa, epi_a == UOCR_GEMM_SWIGLU ? 2u : 1u, a);
-    const size_t sb = gemm_scales(qb, epi_b == UOCR_GEMM_SWIGLU ? 2u : 1u, b);
-    const u32 ax = (da->M + TM - 1u) / TM, na = ax * ((da->N + TN - 1u) / TN);
-    const u32 bx = db->tile_e != nullptr ? db->max_tiles : (db->M + TM - 1u) / TM;
-    const dim3 grid(na + bx * ((db->N + TN - 1u) / TN));
-    const size_t shm = sa > sb ? sa : sb;
-    if (router) {
-        switch (qa) {
-            case UOCR_QT_F16:
-                hipLaunchKernelGGL((k_gemm_pair<1, GE_SWIGLU, false, 1, GE_F32, false>), grid, dim3(PB), shm, st, a, ax,
-                                   na, b, bx);
-                break;
-            case UOCR_QT_Q8:
-                hipLaunchKernelGGL((k_gemm_pair<3, GE_SWIGLU, false, 1, GE_F32, false>), grid, dim3(PB), shm, st, a, ax,
-                                   na, b, bx);
-                break;
-            default:
-                hipLaunchKernelGGL((k_gemm_pair<4, GE_SWIGLU, false, 1, GE_F32, false>), grid, dim3(PB), shm, st, a, ax,
-                                   na, b, bx);
-                break;
+    const u32 q = da->W[0].qtype;
+    const GemmArgs a = gemm_args(da), b = gemm_args(db);
+    if (da->tile_e == nullptr && da->norm_w == nullptr && uocr_gemm_tile_fits(epi_a, q, a)) {
+        if (epi_a == UOCR_GEMM_F16 && (epi_b == UOCR_GEMM_F16 || epi_b == UOCR_GEMM_F32) && db->tile_rows != 0u &&
+            q == db->W[0].qtype && a.packed == b.packed) {
+            return uocr_gemm_tile_pair(st, epi_b, q, a, b, db->pairs, db->tile_rows);
         }
-    } else if (downs16) {
-        switch (qa) {
-            case UOCR_QT_F16:
-                hipLaunchKernelGGL((k_gemm_pair<1, GE_F16, false, 1, GE_F16, true>), grid, dim3(PB), shm, st, a, ax, na,
-                                   b, bx);
-                break;
-            case UOCR_QT_Q8:
-                hipLaunchKernelGGL((k_gemm_pair<3, GE_F16, false, 3, GE_F16, true>), grid, dim3(PB), shm, st, a, ax, na,
-                                   b, bx);
-                break;
-            default:
-                hipLaunchKernelGGL((k_gemm_pair<4, GE_F16, false, 4, GE_F16, true>), grid, dim3(PB), shm, st, a, ax, na,
-                                   b, bx);
-                break;
-        }
-    } else if (downs) {
-        switch (qa) {
-            case UOCR_QT_F16:
-                hipLaunchKernelGGL((k_gemm_pair<1, GE_F16, false, 1, GE_F32, true>), grid, dim3(PB), shm, st, a, ax, na,
-                                   b, bx);
-                break;
-            case UOCR_QT_Q8:
-                hipLaunchKernelGGL((k_gemm_pair<3, GE_F16, false, 3, GE_F32, true>), grid, dim3(PB), shm, st, a, ax, na,
-                                   b, bx);
-                break;
-            default:
-                hipLaunchKernelGGL((k_gemm_pair<4, GE_F16, false, 4, GE_F32, true>), grid, dim3(PB), shm, st, a, ax, na,
-                                   b, bx);
-                break;
-        }
-    } else {
-        switch (qa) {
-            case UOCR_QT_F16:
-                hipLaunchKernelGGL((k_gemm_pair<1, GE_F16, false, 1, GE_SWIGLU, true>), grid, dim3(PB), shm, st, a, ax,
-                                   na, b, bx);
-                break;
-            case UOCR_QT_Q8:
-                hipLaunchKernelGGL((k_gemm_pair<3, GE_F16, false, 3, GE_SWIGLU, true>), grid, dim3(PB), shm, st, a, ax,
-                                   na, b, bx);
-                break;
-            default:
-                hipLaunchKernelGGL((k_gemm_pair<4, GE_F16, false, 4, GE_SWIGLU, true>), grid, dim3(PB), shm, st, a, ax,
-                                   na, b, bx);
-                break;
+        if (epi_a == UOCR_GEMM_SWIGLU && epi_b == UOCR_GEMM_F32 && db->tile_e == nullptr && db->W[0].qtype == UOCR_QT_F16 &&
+            uocr_gemm_tile_fits(epi_b, UOCR_QT_F16, b)) {
+            return uocr_gemm_tile_router(st, q, a, b);
         }
     }
-    return hipGetLastError();
+    const hipError_t e = uocr_launch_gemm(st, epi_a, da);
+    return e != hipSuccess ? e : uocr_launch_gemm(st, epi_b, db);
 }
 
 extern "C" hipError_t uocr_launch_rows_rmsnorm(hipStream_t st, const uint16_t *x, const uint16_t *w, uint32_t P,
@@ -1191,37 +1043,29 @@ extern "C" hipError_t uocr_launch_gemm_qkv_rope(hipStream_t st, const uocr_gemm_
         return hipErrorInvalidValue;
     }
     GemmArgs a = gemm_args(d);
-    const size_t shm = gemm_scales(d->W[0].qtype, 1u, a);
-    const float2 *tab = (const float2 *)cs;
-    const dim3 grid((d->M + TM - 1u) / TM, d->N / TN);
-    switch (d->W[0].qtype) {
-        case UOCR_QT_F16:
-            hipLaunchKernelGGL(k_gemm_rope<1>, grid, dim3(PB), 0, st, a, tab, (h16 *)qout, (h16 *)kcache,
-                               (h16 *)vcache, cap);
-            break;
-        case UOCR_QT_Q8:
-            hipLaunchKernelGGL(k_gemm_rope<3>, grid, dim3(PB), shm, st, a, tab, (h16 *)qout, (h16 *)kcache,
-                               (h16 *)vcache, cap);
-            break;
-        default:
-            hipLaunchKernelGGL(k_gemm_rope<4>, grid, dim3(PB), shm, st, a, tab, (h16 *)qout, (h16 *)kcache,
-                               (h16 *)vcache, cap);
-            break;
+    a.nseg = 0u;
+    uintptr_t al = 0;
+    for (int i = 0; i < 3; ++i) al |= (uintptr_t)d->W[i].w;
+    a.vec = 1u; /* the epilogue writes q and the cache slots only */
+    if (al % 16u != 0u || (((uintptr_t)qout | (uintptr_t)kcache | (uintptr_t)vcache | (uintptr_t)cs) % 16u) != 0u ||
+        !uocr_gemm_tile_fits(UOCR_GEMM_F16, d->W[0].qtype, a)) {
+        return hipErrorInvalidValue;
     }
-    return hipGetLastError();
+    a.nseg = d->nseg;
+    return uocr_gemm_tile_rope(st, d->W[0].qtype, a, RopeDst{(const float2 *)cs, (h16 *)qout, (h16 *)kcache, (h16 *)vcache, cap});
 }
 
 extern "C" hipError_t uocr_launch_route_rows(hipStream_t st, const float *logits, uint32_t P, int norm_topk,
                                              int32_t *ids, float *wts, int32_t *offsets, int32_t *tile_e,
                                              int32_t *tile_s0, int32_t *tile_s1, int32_t *ntiles, int32_t *list_tok,
-                                             int32_t *list_pair) {
+                                             int32_t *list_pair, uint32_t tile_rows) {
     if (logits == nullptr || P == 0u || ids == nullptr || wts == nullptr || offsets == nullptr || tile_e == nullptr || tile_s0 == nullptr || tile_s1 == nullptr || ntiles == nullptr ||
         list_tok == nullptr || list_pair == nullptr) {
         return hipErrorInvalidValue;
     }
     hipLaunchKernelGGL(k_route_rows, dim3((P + 3u) / 4u), dim3(PB), 0, st, logits, P, norm_topk, ids, wts);
     hipLaunchKernelGGL(k_bucket_build, dim3(1), dim3(BUCKET_THREADS), 0, st, (const int32_t *)ids, P, offsets,
-                       tile_e, tile_s0, tile_s1, ntiles, list_tok, list_pair);
+                       tile_e, tile_s0, tile_s1, ntiles, list_tok, list_pair, (int32_t)(tile_rows != 0u ? tile_rows : TM));
     return hipGetLastError();
 }
 
