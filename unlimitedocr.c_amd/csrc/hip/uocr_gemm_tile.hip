@@ -188,13 +188,16 @@ __device__ __forceinline__ void tile_body(const GemmArgs &p, u32 bx, u32 by, uin
         for (int g = 0; g < NG; ++g) {
             const u32 s = c * NG + g;
             if (g > 0 && s >= NS) break;
-            /* A step issues its share of line c + 1, then the activations of
-             * step s + 2.  Needed here: the activations of step s, issued in
-             * step s - 2, and at g = 0 line c, older than step s - 1's
-             * activations; in flight may stay all of step s - 1's loads (at g
-             * = 0 only its activations). */
+            /* A step issues the activations of step s + 2, then its share of
+             * line c + 1 (f16, whose line lasts one step: the line first).
+             * Loads complete in order, so what must have landed here is the
+             * activations of step s, issued in step s - 2, and at g = 0 line c;
+             * in flight may stay what was issued after them.  The weights,
+             * which come from HBM, so have three steps to arrive (Q8: two). */
             constexpr int NB = NG == 4 ? 4 : 8, BS = 8 / NB; /* loads of a line per step, in the line's first BS steps */
-            if (g >= 1 && g <= BS && c + 1u < NCH) wait_barrier<AL + NB>();
+            const int after = NG == 1 ? 0 : (g >= 1 && g <= BS ? NB : 0) + (g >= 2 && g <= BS + 1 ? NB : 0);
+            if (after == 2 * NB && c + 1u < NCH) wait_barrier<AL + 2 * NB>();
+            else if (after == NB && c + 1u < NCH) wait_barrier<AL + NB>();
             else wait_barrier<AL>();
             if (g == 0) {
 #pragma unroll
@@ -227,6 +230,8 @@ __device__ __forceinline__ void tile_body(const GemmArgs &p, u32 bx, u32 by, uin
             }
             if (WK == 1 || s < NT) {
             const uint8_t *abuf = gsm + cur;
+            /* computing goes before the CU's other block's loads and waits */
+            __builtin_amdgcn_s_setprio(1);
             U4H8 a[2][RT]; /* substep i's operands and the next one's */
 #pragma unroll
             for (int k = 0; k < RT; ++k) a[0][k].u = *(const uint4 *)(abuf + ao[0] + 4096u * k);
@@ -247,22 +252,25 @@ __device__ __forceinline__ void tile_body(const GemmArgs &p, u32 bx, u32 by, uin
                     /* the loads spread over the step, between its MFMAs: issued
                      * together they fill the memory pipe's queue and the
                      * wavefront's MFMAs wait behind them */
-                    const int slot = 2 * i + j;
-                    if (g < BS && slot >= 1 && slot <= 4 && c + 1u < NCH) {
-                        /* the line is in registers: its LDS takes the next one */
-                        if (slot == 1) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-                        for (int x = 0; x < NB / 4; ++x) issue_b(c + 1u, NB * g + NB / 4 * (slot - 1) + x);
-                    }
+                    const int slot = 2 * i + j, bslot = NG > 1 ? 4 : 1, aslot = NG > 1 ? 0 : 4;
                     /* (past the end the last step again, which nothing reads:
                      * the count of loads in flight stays the same) */
-                    if (slot >= 4) {
+                    auto slot_a = [&]() {
 #pragma unroll
                         for (int q = 0; q < AL; ++q)
-                            if (4 + q * 4 / AL == slot) issue_a(min(s + 2u, sl), nxt, q);
+                            if (aslot + q * 4 / AL == slot) issue_a(min(s + 2u, sl), nxt, q);
+                    };
+                    if (NG > 1) slot_a();
+                    if (g < BS && slot >= bslot && slot < bslot + 4 && c + 1u < NCH) {
+                        /* the line is in registers: its LDS takes the next one */
+                        if (slot == bslot) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+                        for (int x = 0; x < NB / 4; ++x) issue_b(c + 1u, NB * g + NB / 4 * (slot - bslot) + x);
                     }
+                    if (NG == 1) slot_a();
                 }
             }
+            __builtin_amdgcn_s_setprio(0);
             }
             nxt = cur;
             cur = cur + ABUF == NA * ABUF ? 0u : cur + ABUF;
