@@ -180,3 +180,43 @@ def test_moe_rows_bucket_edges(gpu, qtype, P, given, static):
     bound = np.abs(y) * 2.0**-11 + mag * 2.0**-10 + 2.0**-24
     err = np.abs(got - y)
     assert (err <= bound).all(), float((err / bound).max())
+
+
+@pytest.mark.parametrize("P", [1, 170, 171, 1365, 1366, 4096, 4097])
+def test_moe_rows_routing_edges(gpu, P):
+    """Row counts at which the bucket build changes its pairs per thread (8 up to
+    1,365 rows, 24 up to 4,096, two passes above) and the edges of its batches:
+    every row equals its own single-row MoE of the decode operators up to the
+    rounding of fp16 (the single-row path rounds the same values)."""
+    uocr = gpu
+    rng = np.random.default_rng(P)
+    of = uocr.DeviceBuffer.of
+    m, keep = uocr.CMoeWeights(), []
+    m.expert_qtype = m.shared_qtype = 4
+    for name, rows, k in (("gate", 64 * 896, 1280), ("up", 64 * 896, 1280), ("down", 64 * 1280, 896), ("sgate", 1792, 1280),
+                          ("sup", 1792, 1280), ("sdown", 1280, 1792)):
+        w, s = weights_for(4, rng, rows, k)
+        keep += [of(w), of(s)]
+        setattr(m, name + "_w", keep[-2].ptr)
+        setattr(m, name + "_s", keep[-1].ptr)
+        if name in ("gate", "down"):
+            pre = "gu" if name == "gate" else "dn"
+            setattr(m, pre + "_w_stride", w.nbytes // 64)
+            setattr(m, pre + "_s_stride", s.size // 64)
+    router = of(rand_f16(rng, (64, 1280), 0.03))
+    m.router = router.ptr
+    x, res = rand_f16(rng, (P, 1280)), rand_f16(rng, (P, 1280))
+    dx, dres, dout = of(x), of(res), uocr.DeviceBuffer(P * 2560)
+    uocr.op_moe_ffn_rows(m, dx, None, dres, P, 1, uocr.moe_rows_workspace(P), dout)
+    uocr.sync()
+    got = dout.download(np.float16).reshape(P, 1280).astype(np.float64)
+    ws, one, ids, wts = uocr.workspace(), uocr.DeviceBuffer(2560), uocr.DeviceBuffer(64), uocr.DeviceBuffer(64)
+    for t in np.unique(np.concatenate([np.arange(min(P, 20)), np.arange(max(0, P - 20), P)])):
+        uocr.op_moe_ffn(m, dx.ptr + 2560 * int(t), None, dres.ptr + 2560 * int(t), 1, ws, one, ids, wts)
+        uocr.sync()
+        ref = one.download(np.float16).astype(np.float64)
+        # weights rounded to fp16(q * scale) here and exact there: 2^-11 of each
+        # product, which add up like a random walk; 2^-7 of the row's size is
+        # over ten times that, a wrong expert or weight is 0.1 and more of it
+        size = np.sqrt(np.mean((ref - res[t].astype(np.float64)) ** 2))
+        assert np.abs(got[t] - ref).max() <= 2.0**-7 * size + 2.0**-10 * np.abs(ref).max(), int(t)

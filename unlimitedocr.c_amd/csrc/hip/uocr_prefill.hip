@@ -612,96 +612,117 @@ __global__ __launch_bounds__(PB) void k_route_rows(const float *__restrict__ log
     }
 }
 
-/* One block builds the expert buckets of all P*6 (token, rank) pairs in
- * LDS: the 64 bucket sizes (LDS atomics), their exclusive scan (offsets),
- * the tile table of the grouped GEMMs (tile_rows rows per tile) and every pair's
- * slot in its bucket (list_tok, list_pair).  The order of pairs inside a
- * bucket does not matter: each pair's row is computed on its own and the
- * combine reads it by pair index.  Nothing is left in global memory that the
- * next routing has to find cleared. */
+/* The routing's outputs for the grouped GEMMs. */
+struct BucketOut {
+    int32_t *offsets, *tile_e, *tile_s0, *tile_s1, *ntiles, *list_tok, *list_pair;
+    int32_t tile_rows;
+};
+
 #define BUCKET_THREADS 1024
-__global__ __launch_bounds__(BUCKET_THREADS) void k_bucket_build(const int32_t *__restrict__ ids, u32 P,
-                                                                 int32_t *__restrict__ offsets,
-                                                                 int32_t *__restrict__ tile_e,
-                                                                 int32_t *__restrict__ tile_s0,
-                                                                 int32_t *__restrict__ tile_s1,
-                                                                 int32_t *__restrict__ ntiles,
-                                                                 int32_t *__restrict__ list_tok,
-                                                                 int32_t *__restrict__ list_pair, int32_t tile_rows) {
-    __shared__ int32_t cnt[64], off[65], toff[65], cur[64];
-    const u32 t = threadIdx.x, n = P * UOCR_K_TOPK;
+
+/* Exclusive scans of the 64 bucket sizes and tile counts (one wavefront, a
+ * lane per expert) and the tile table of the grouped GEMMs. */
+__device__ __forceinline__ void bucket_tables(const int32_t *cnt, int32_t *off, const BucketOut &o) {
+    const u32 t = threadIdx.x;
     if (t < 64u) {
-        cnt[t] = 0;
-        cur[t] = 0;
-    }
-    /* the thread's pairs' ids, all loads in flight at once (up to BUCKET_R
-     * per thread; longer prompts loop) */
-    constexpr u32 BUCKET_R = 8u;
-    const bool inreg = n <= BUCKET_R * BUCKET_THREADS;
-    int32_t idr[BUCKET_R];
-    if (inreg) {
-#pragma unroll
-        for (u32 k = 0; k < BUCKET_R; ++k) idr[k] = t + k * BUCKET_THREADS < n ? ids[t + k * BUCKET_THREADS] : -1;
-    }
-    __syncthreads();
-    if (inreg) {
-#pragma unroll
-        for (u32 k = 0; k < BUCKET_R; ++k) {
-            if (idr[k] >= 0) atomicAdd(&cnt[idr[k]], 1);
-        }
-    } else {
-        for (u32 pr = t; pr < n; pr += BUCKET_THREADS) atomicAdd(&cnt[ids[pr]], 1);
-    }
-    __syncthreads();
-    if (t < 64u) {
-        /* exclusive scans of the bucket sizes and tile counts: one wavefront,
-         * a lane per expert */
-        const int32_t c = cnt[t], tl = (c + tile_rows - 1) / tile_rows;
+        const int32_t c = cnt[t], tl = (c + o.tile_rows - 1) / o.tile_rows;
         int32_t a = c, b = tl;
 #pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int32_t x = __shfl_up(a, o), y = __shfl_up(b, o);
-            if ((int)t >= o) {
+        for (int d = 1; d < 64; d <<= 1) {
+            const int32_t x = __shfl_up(a, d), y = __shfl_up(b, d);
+            if ((int)t >= d) {
                 a += x;
                 b += y;
             }
         }
         off[t] = a - c;
-        toff[t] = b - tl;
-        if (t == 63u) {
-            off[64] = a;
-            toff[64] = b;
-            *ntiles = b;
+        o.offsets[t] = a - c;
+        if (t == 63u) *o.ntiles = b;
+        for (int32_t k = 0; k * o.tile_rows < c; ++k) {
+            const int32_t ti = b - tl + k;
+            o.tile_e[ti] = (int32_t)t;
+            o.tile_s0[ti] = a - c + k * o.tile_rows;
+            o.tile_s1[ti] = a - c + min(c, (k + 1) * o.tile_rows);
         }
     }
     __syncthreads();
+}
+
+/* One block builds the expert buckets of all P*6 (token, rank) pairs in LDS:
+ * the bucket sizes (LDS atomics, which also give each pair its place in its
+ * bucket), their scan, the tile table and the slot lists.  The order of pairs
+ * inside a bucket does not matter: each pair's row is computed on its own and
+ * the combine reads it by pair index.  Nothing is left in global memory that
+ * the next routing has to find cleared.  One CU does all of it, so what
+ * bounds it are its dependent loads and its scattered stores: a thread's R pairs
+ * are loaded together and stay in registers with their places, and the lists
+ * are put in order in LDS and leave as whole lines: 4,001 rows 28 us with 8
+ * pairs in registers and loops above, 25 with 24, 9.5 with the lists in LDS;
+ * 932 rows 4.4 us.
+ * More than R per thread take two passes in batches with direct stores. */
+template <u32 R>
+__global__ __launch_bounds__(BUCKET_THREADS) void k_bucket_build(const int32_t *__restrict__ ids, u32 P, BucketOut o) {
+    __shared__ int32_t cnt[64], off[64], cur[64];
+    __shared__ uint16_t list[R * BUCKET_THREADS];
+    const u32 t = threadIdx.x, n = P * UOCR_K_TOPK;
     if (t < 64u) {
-        offsets[t] = off[t];
-        const int32_t c = cnt[t];
-        for (int32_t k = 0; k * tile_rows < c; ++k) {
-            const int32_t ti = toff[t] + k;
-            tile_e[ti] = (int32_t)t;
-            tile_s0[ti] = off[t] + k * tile_rows;
-            tile_s1[ti] = off[t] + min(c, (k + 1) * tile_rows);
-        }
+        cnt[t] = 0;
+        cur[t] = 0;
     }
-    if (inreg) {
+    int32_t id[R], place[R];
+    auto load = [&](u32 base) {
 #pragma unroll
-        for (u32 k = 0; k < BUCKET_R; ++k) {
-            const u32 pr = t + k * BUCKET_THREADS;
-            if (idr[k] >= 0) {
-                const int32_t slot = off[idr[k]] + atomicAdd(&cur[idr[k]], 1);
-                list_tok[slot] = (int32_t)(pr / UOCR_K_TOPK);
-                list_pair[slot] = (int32_t)pr;
+        for (u32 k = 0; k < R; ++k) {
+            const u32 pr = base + t + k * BUCKET_THREADS;
+            id[k] = pr < n ? ids[pr] : -1;
+        }
+    };
+    auto count = [&](int32_t *c) {
+#pragma unroll
+        for (u32 k = 0; k < R; ++k)
+            if (id[k] >= 0) place[k] = atomicAdd(&c[id[k]], 1);
+    };
+    auto store = [&](u32 base) {
+#pragma unroll
+        for (u32 k = 0; k < R; ++k) {
+            const u32 pr = base + t + k * BUCKET_THREADS;
+            if (id[k] >= 0) {
+                const int32_t slot = off[id[k]] + place[k];
+                o.list_tok[slot] = (int32_t)(pr / UOCR_K_TOPK);
+                o.list_pair[slot] = (int32_t)pr;
             }
         }
-    } else {
-        for (u32 pr = t; pr < n; pr += BUCKET_THREADS) {
-            const int32_t e = ids[pr];
-            const int32_t slot = off[e] + atomicAdd(&cur[e], 1);
-            list_tok[slot] = (int32_t)(pr / UOCR_K_TOPK);
-            list_pair[slot] = (int32_t)pr;
+    };
+    load(0u);
+    __syncthreads();
+    count(cnt);
+    const bool once = n <= R * BUCKET_THREADS;
+    for (u32 base = R * BUCKET_THREADS; base < n; base += R * BUCKET_THREADS) {
+        load(base);
+        count(cnt);
+    }
+    __syncthreads();
+    bucket_tables(cnt, off, o);
+    if (once) {
+#pragma unroll
+        for (u32 k = 0; k < R; ++k)
+            if (id[k] >= 0) list[off[id[k]] + place[k]] = (uint16_t)(t + k * BUCKET_THREADS);
+        __syncthreads();
+#pragma unroll
+        for (u32 k = 0; k < R; ++k) {
+            const u32 s = t + k * BUCKET_THREADS;
+            if (s < n) {
+                const u32 pr = list[s];
+                o.list_tok[s] = (int32_t)(pr / UOCR_K_TOPK);
+                o.list_pair[s] = (int32_t)pr;
+            }
         }
+        return;
+    }
+    for (u32 base = 0; base < n; base += R * BUCKET_THREADS) {
+        load(base);
+        count(cur);
+        store(base);
     }
 }
 
@@ -1063,9 +1084,12 @@ extern "C" hipError_t uocr_launch_route_rows(hipStream_t st, const float *logits
         list_tok == nullptr || list_pair == nullptr) {
         return hipErrorInvalidValue;
     }
+    const BucketOut o = {offsets, tile_e, tile_s0, tile_s1, ntiles, list_tok, list_pair, (int32_t)(tile_rows != 0u ? tile_rows : TM)};
     hipLaunchKernelGGL(k_route_rows, dim3((P + 3u) / 4u), dim3(PB), 0, st, logits, P, norm_topk, ids, wts);
-    hipLaunchKernelGGL(k_bucket_build, dim3(1), dim3(BUCKET_THREADS), 0, st, (const int32_t *)ids, P, offsets,
-                       tile_e, tile_s0, tile_s1, ntiles, list_tok, list_pair, (int32_t)(tile_rows != 0u ? tile_rows : TM));
+    if (P * UOCR_K_TOPK <= 8u * BUCKET_THREADS)
+        hipLaunchKernelGGL(k_bucket_build<8u>, dim3(1), dim3(BUCKET_THREADS), 0, st, (const int32_t *)ids, P, o);
+    else
+        hipLaunchKernelGGL(k_bucket_build<24u>, dim3(1), dim3(BUCKET_THREADS), 0, st, (const int32_t *)ids, P, o);
     return hipGetLastError();
 }
 
