@@ -88,6 +88,23 @@ def test_gemm_misaligned_rows(gpu, qtype):
     check_rows(got, x, wv[:n2], np.zeros((m, n2)))
 
 
+@pytest.mark.parametrize("qtype", [1, 3, 4])
+@pytest.mark.parametrize("m,n,k", [(70, 132, 2048), (70, 130, 2048), (257, 132, 192)])
+def test_vision_linear_misaligned_rows(gpu, qtype, m, n, k):
+    """Widths off 16-byte pieces take the general kernel: split over K with its
+    reduce (long K, n % 4 == 0) and unsplit."""
+    uocr = gpu
+    rng = np.random.default_rng(qtype + n)
+    w, s = weights_for(qtype, rng, n, k)
+    x, bias = rand_f16(rng, (m, k)), rand_f16(rng, (n,))
+    of = uocr.DeviceBuffer.of
+    dw, ds, dx, db, dy = of(w), None if s is None else of(s), of(x), of(bias), uocr.DeviceBuffer(m * n * 2)
+    uocr.op_vision_linear(qtype, dw, ds, db, m, k, n, 0, 0, dx, dy)
+    uocr.sync()
+    got = dy.download(np.float16, m * n).reshape(m, n)
+    check_rows(got, x, operand_values(qtype, w, s), np.tile(bias.astype(np.float64), (m, 1)))
+
+
 def routed_rows(rng, counts, P):
     """For each row its 6 experts, so that expert e serves counts[e] rows."""
     left = np.full(P, 6)

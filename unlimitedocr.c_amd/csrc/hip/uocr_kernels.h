@@ -246,7 +246,7 @@ typedef struct uocr_gemm_desc {
     const uint16_t *bias;
     uint32_t act, split;
     void *out1, *out2;
-    /* UOCR_GEMM_VISION, F16 and F32 (not grouped): ksplit > 1 splits K over
+    /* UOCR_GEMM_VISION: ksplit > 1 splits K over
      * that many blocks per tile, each writing fp32 partials into part
      * ([ksplit][M][N] floats), reduced in order by a second kernel that
      * applies the epilogue; ksplit <= 1 or part NULL: no split */
@@ -256,7 +256,7 @@ typedef struct uocr_gemm_desc {
      * copy of uocr_launch_pack_gemm_rows instead of the row-major payload */
     uint32_t packed;
     /* UOCR_GEMM_F16, not grouped, N == ldo == 1280: norm_w set also writes
-     * norm_out = f16(rmsnorm(out) * norm_w) (fused into the split-K reduce) */
+     * norm_out = f16(rmsnorm(out) * norm_w) */
     const uint16_t *norm_w;
     uint16_t *norm_out;
 } uocr_gemm_desc;
@@ -278,9 +278,6 @@ hipError_t uocr_launch_gemm_pair(hipStream_t st, int epi_a, const uocr_gemm_desc
  * contiguous run per step (lane 32h + r takes row r's half h). */
 hipError_t uocr_launch_pack_gemm_rows(hipStream_t st, uint32_t qtype, const void *src, void *dst, uint32_t rows,
                                       uint32_t K, uint32_t count, uint64_t stride);
-/* K splits (1: none) for a plain GEMM of M x N x K whose tile grid is under
- * one block per CU; UOCR_GEMM_F16 / F32 / VISION honour desc ksplit + part. */
-uint32_t uocr_gemm_ksplit(uint32_t M, uint32_t N, uint32_t K);
 /* y[t] = rmsnorm(x[t], w) for P rows of 1280. */
 hipError_t uocr_launch_rows_rmsnorm(hipStream_t st, const uint16_t *x, const uint16_t *w, uint32_t P, uint16_t *y);
 /* cs [P][64][2] = (cos, sin) of t * inv_freq[d] for tokens t < P (inv_freq:

@@ -4,19 +4,22 @@
  * with its tiled GEMMs gemm_q4.metal / gemm_q8.metal).
  *
  * All P prompt rows go through each layer together, so the projections are
- * real GEMMs [P x K] x [K x N]:
- *  - k_gemm: 64 x 128 output tiles, K in 64-column steps (one quantisation
- *    group).  Activation tiles are staged in LDS as fp16 (double-buffered);
- *    each wavefront dequantises its own 32 weight rows straight into MFMA
- *    operand registers as fp16(q * scale), the reference's prefill staging
- *    (gemm_q4.metal:48-55: half(float(q) * scale)), and
- *    v_mfma_f32_32x32x16_f16 accumulates in fp32.  Epilogues: fp16 store with
+ * real GEMMs [P x K] x [K x N]; the tiled kernels (uocr_gemm_tile.hip) and the
+ * attention (uocr_attn_prefill.hip) have files of their own.  Here:
+ *  - the launchers, which check a GEMM and choose its kernel;
+ *  - k_gemm, the general GEMM for operands that are off 16-byte pieces (the
+ *    operators accept them, the engine has none): 64 x 128 output tiles, K in
+ *    64-column steps (one quantisation group), activations staged in LDS as
+ *    fp16, each wavefront dequantising its own 32 weight rows straight into
+ *    MFMA operand registers as fp16(q * scale), the reference's prefill
+ *    staging (gemm_q4.metal:48-55: half(float(q) * scale)), with fp32
+ *    accumulation by v_mfma_f32_32x32x16_f16.  Epilogues: fp16 store with
  *    optional residual, fp32 store, and SwiGLU over two weight matrices.  In
  *    grouped mode a tile table maps each block to an expert's bucket of
  *    (token, rank) pairs: rows are gathered through an index list and the
- *    expert's weights are addressed by slab stride.
- *  - routing (top-6 per token, expert buckets), RoPE + KV scatter, MoE
- *    combine and row RMSNorm kernels.
+ *    expert's weights are addressed by slab stride;
+ *  - routing (top-6 per token, expert buckets), RoPE table, MoE combine and
+ *    row RMSNorm kernels.
  * fp16 rounding happens where the decode path rounds (norm, q/k/v, RoPE,
  * attention output, O + residual, SwiGLU mids, shared output, layer output).
  */
@@ -383,17 +386,13 @@ __global__ __launch_bounds__(PB) void k_rope_table(RopeTabP rope, u32 P, float2 
     cs[idx] = make_float2(cosf(ang), sinf(ang));
 }
 
-/* Split-K epilogue: the z partials summed in order (the result does not
- * depend on block timing), then
- *   RD_VISION: out = f16(act(sum + bias)), split into o0/o1/o2 when split;
- *   RD_F16:    out = f16(sum (+ res)), row stride ldo (res: ldr);
- *   RD_F32:    out = sum (fp32), row stride ldo. */
-enum { RD_VISION = 0, RD_F16 = 1, RD_F32 = 2 };
-__global__ __launch_bounds__(PB) void k_split_reduce(const float *__restrict__ part, u32 S, u32 M, u32 N, u32 mode,
+/* Split-K epilogue of the vision GEMM: the z partials summed in order (the
+ * result does not depend on block timing), out = f16(act(sum + bias)), split
+ * into o0/o1/o2 when split. */
+__global__ __launch_bounds__(PB) void k_split_reduce(const float *__restrict__ part, u32 S, u32 M, u32 N,
                                                      const h16 *__restrict__ bias, u32 act, u32 split,
-                                                     const h16 *__restrict__ res, u32 ldr, void *__restrict__ o0,
-                                                     h16 *__restrict__ o1, h16 *__restrict__ o2, u32 ldo) {
-    /* four consecutive columns per thread (N, split, ldo and ldr are
+                                                     h16 *__restrict__ o0, h16 *__restrict__ o1, h16 *__restrict__ o2) {
+    /* four consecutive columns per thread (N and split are
      * multiples of 4, checked by the launcher), so every load is 16 bytes */
     const size_t i = 4u * ((size_t)blockIdx.x * PB + threadIdx.x), MN = (size_t)M * N;
     if (i >= MN) return;
@@ -414,22 +413,11 @@ __global__ __launch_bounds__(PB) void k_split_reduce(const float *__restrict__ p
         }
     }
     const u32 row = (u32)(i / N), col = (u32)(i - (size_t)row * N);
-    if (mode == RD_F32) {
-        *(float4 *)((float *)o0 + (size_t)row * ldo + col) = v;
-        return;
-    }
     float r[4] = {v.x, v.y, v.z, v.w};
     union {
         h16 h[4];
         uint2 u;
-    } o, rr;
-    if (mode == RD_F16) {
-        if (res != nullptr) rr.u = *(const uint2 *)(res + (size_t)row * ldr + col);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) o.h[c] = (h16)(res != nullptr ? r[c] + (float)rr.h[c] : r[c]);
-        *(uint2 *)((h16 *)o0 + (size_t)row * ldo + col) = o.u;
-        return;
-    }
+    } o;
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
         float x = r[c] + (float)bias[col + c];
@@ -438,10 +426,10 @@ __global__ __launch_bounds__(PB) void k_split_reduce(const float *__restrict__ p
         o.h[c] = (h16)x;
     }
     if (split == 0u) {
-        *(uint2 *)((h16 *)o0 + (size_t)row * ldo + col) = o.u;
+        *(uint2 *)(o0 + (size_t)row * N + col) = o.u;
     } else {
         const u32 pj = col / split, lc = col - pj * split;
-        *(uint2 *)((pj == 0u ? (h16 *)o0 : (pj == 1u ? o1 : o2)) + (size_t)row * split + lc) = o.u;
+        *(uint2 *)((pj == 0u ? o0 : (pj == 1u ? o1 : o2)) + (size_t)row * split + lc) = o.u;
     }
 }
 
@@ -496,72 +484,6 @@ __global__ __launch_bounds__(PB) void k_rows_rmsnorm(const h16 *__restrict__ x, 
     for (int q = 0; q < 3; ++q) {
         const u32 i = lane + 64u * q;
         if (i < UOCR_K_HIDDEN / 8u) v[q].u = ((const uint4 *)xr)[i];
-    }
-    row_norm_tail(v, lane, wv, y + (size_t)row * UOCR_K_HIDDEN);
-}
-
-/* Split-K reduce of a 1280-column fp16 GEMM output with its residual, fused
- * with the RMSNorm that reads it: per row (one wavefront), out = f16(sum of
- * the S planes in order + res) as k_split_reduce (RD_F16) rounds it, then
- * y = rmsnorm(out) * w as k_rows_rmsnorm rounds it. */
-__global__ __launch_bounds__(PB) void k_reduce_norm(const float *__restrict__ part, u32 S, u32 M,
-                                                    const h16 *__restrict__ res, u32 ldr, h16 *__restrict__ out,
-                                                    u32 ldo, const h16 *__restrict__ w, h16 *__restrict__ y) {
-    const u32 row = blockIdx.x * (PB / 64) + (threadIdx.x >> 6), lane = threadIdx.x & 63u;
-    if (row >= M) return;
-    const size_t MN = (size_t)M * UOCR_K_HIDDEN;
-    /* the first two planes of the row's pieces (and the residual), all in
-     * flight before any sum; planes beyond the second are added in order
-     * after them */
-    float4 pa[3][2], pb2[3][2];
-    U4H8 rr[3], wv[3];
-    norm_w_load(w, lane, wv);
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-        const u32 i = min(lane + 64u * q, UOCR_K_HIDDEN / 8u - 1u);
-        const float *p0 = part + (size_t)row * UOCR_K_HIDDEN + 8u * i;
-#pragma unroll
-        for (u32 z = 0; z < 2u; ++z) {
-            if (z < S) {
-                pa[q][z] = *(const float4 *)(p0 + z * MN);
-                pb2[q][z] = *(const float4 *)(p0 + z * MN + 4);
-            }
-        }
-        if (res != nullptr) rr[q].u = *(const uint4 *)(res + (size_t)row * ldr + 8u * i);
-    }
-    U4H8 v[3];
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-        const u32 i = lane + 64u * q;
-        if (i >= UOCR_K_HIDDEN / 8u) continue;
-        const float *p0 = part + (size_t)row * UOCR_K_HIDDEN + 8u * i;
-        float4 a = pa[q][0], b = pb2[q][0];
-        if (S > 1u) {
-            const float4 c = pa[q][1], d = pb2[q][1];
-            a.x += c.x;
-            a.y += c.y;
-            a.z += c.z;
-            a.w += c.w;
-            b.x += d.x;
-            b.y += d.y;
-            b.z += d.z;
-            b.w += d.w;
-        }
-        for (u32 z = 2; z < S; ++z) {
-            const float4 c = *(const float4 *)(p0 + z * MN), d = *(const float4 *)(p0 + z * MN + 4);
-            a.x += c.x;
-            a.y += c.y;
-            a.z += c.z;
-            a.w += c.w;
-            b.x += d.x;
-            b.y += d.y;
-            b.z += d.z;
-            b.w += d.w;
-        }
-        const float r[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[q].h[j] = (h16)(res != nullptr ? r[j] + (float)rr[q].h[j] : r[j]);
-        *(uint4 *)(out + (size_t)row * ldo + 8u * i) = v[q].u;
     }
     row_norm_tail(v, lane, wv, y + (size_t)row * UOCR_K_HIDDEN);
 }
@@ -835,14 +757,6 @@ static bool pmat_ok(uocr_qmat m) {
     return m.w != nullptr && pq_ok(m.qtype) && (m.qtype == UOCR_QT_F16 || m.s != nullptr);
 }
 
-/* Tile rows of a GEMM.  128-row tiles (each dequantised weight operand
- * feeding four MFMAs instead of two) measured slower at the prefill shapes:
- * 3.83 against 3.17 ms, the grouped gate/up dropping to one wavefront per
- * SIMD; the kernel keeps the template parameter. */
-static inline u32 gemm_tm(bool, u32) {
-    return (u32)TM;
-}
-
 template <int EPI, bool GROUPED, int TMR>
 static void gemm_dispatch_tm(hipStream_t st, u32 qt, const GemmArgs &a, dim3 grid, size_t shm) {
     switch (qt) {
@@ -853,28 +767,11 @@ static void gemm_dispatch_tm(hipStream_t st, u32 qt, const GemmArgs &a, dim3 gri
 }
 
 template <int EPI, bool GROUPED>
-static void gemm_dispatch(hipStream_t st, u32 qt, GemmArgs a, dim3 grid, u32 tmr) {
+static void gemm_dispatch(hipStream_t st, u32 qt, GemmArgs a, dim3 grid) {
     const u32 nm = EPI == GE_SWIGLU ? 2u : 1u, nt = a.K / TK;
     a.sc_lds = qt != UOCR_QT_F16 && nm * nt <= SC_LDS_STEPS ? 1u : 0u;
     const size_t shm = a.sc_lds ? (size_t)nm * TN * nt * sizeof(unsigned short) : 0;
-    (void)tmr;
     gemm_dispatch_tm<EPI, GROUPED, TM>(st, qt, a, grid, shm);
-}
-
-/* K splits for a plain GEMM whose tile grid is under one block per CU: the
- * largest power of two <= 8 that keeps the grid in one round of resident
- * blocks (about 512) with at least 5 K steps per split. */
-extern "C" uint32_t uocr_gemm_ksplit(uint32_t M, uint32_t N, uint32_t K) {
-    const u32 tm = gemm_tm(false, M);
-    const u32 blocks = ((M + tm - 1u) / tm) * ((N + TN - 1u) / TN), steps = K / TK;
-    if (blocks >= 256u) return 1u;
-    u32 s = 1u;
-    /* doubling while the split grid stays within 512 blocks and a split keeps
-     * 5 K steps, or a split keeps 16: the O projection at P = 932 (150 tiles,
-     * 20 steps) takes 2 (4 measured the same GEMM time and a longer reduce),
-     * layer 0's dense down (150 tiles, 107 steps) 4 (44.8 -> 36.0 us) */
-    while (s < 8u && ((blocks * 2u * s <= 512u && steps / (2u * s) >= 5u) || steps / (2u * s) >= 16u)) s *= 2u;
-    return s;
 }
 
 static bool gemm_desc_ok(int epi, const uocr_gemm_desc *d) {
@@ -943,27 +840,21 @@ extern "C" hipError_t uocr_launch_gemm(hipStream_t st, int epi, const uocr_gemm_
     if (!gemm_desc_ok(epi, d)) return hipErrorInvalidValue;
     const bool grouped = d->tile_e != nullptr;
     GemmArgs a = gemm_args(d);
-    const u32 tmr = gemm_tm(grouped, d->M);
-    const dim3 grid(grouped ? d->max_tiles : (d->M + tmr - 1u) / tmr, (d->N + TN - 1u) / TN);
+    const dim3 grid(grouped ? d->max_tiles : (d->M + TM - 1u) / TM, (d->N + TN - 1u) / TN);
     const u32 qt = d->W[0].qtype;
     if (epi == UOCR_GEMM_VISION && (grouped || d->bias == nullptr || d->act > UOCR_VISION_ACT_GELU_ERF ||
                                     (d->split != 0u && (d->N != 3u * d->split || d->out1 == nullptr ||
                                                         d->out2 == nullptr)))) {
         return hipErrorInvalidValue;
     }
-    const bool splittable = !grouped && d->ksplit > 1u && d->part != nullptr && d->N % 4u == 0u &&
-                            (epi == UOCR_GEMM_VISION ? d->split % 4u == 0u
-                                                     : (epi == UOCR_GEMM_F16 || epi == UOCR_GEMM_F32) &&
-                                                           d->ldo % 4u == 0u &&
-                                                           (d->res == nullptr || d->ldr % 4u == 0u));
-    /* norm_w: the F16 output rows also go through the RMSNorm into norm_out
-     * (fused into the split-K reduce, else a row-norm launch after the GEMM) */
+    const bool splittable = epi == UOCR_GEMM_VISION && d->ksplit > 1u && d->part != nullptr && d->N % 4u == 0u && d->split % 4u == 0u;
+    /* norm_w: the F16 output rows also go through the RMSNorm into norm_out,
+     * a row-norm launch after the GEMM */
     const bool want_norm = d->norm_w != nullptr;
     if (want_norm && (epi != UOCR_GEMM_F16 || grouped || d->norm_out == nullptr || d->N != UOCR_K_HIDDEN ||
                       d->ldo != UOCR_K_HIDDEN || (d->res != nullptr && d->ldr % 8u != 0u))) {
         return hipErrorInvalidValue;
     }
-    const bool fuse_norm = want_norm && splittable;
     if (grouped && d->tile_rows != 0u) return uocr_gemm_tile_grouped(st, epi, qt, a, d->pairs, d->tile_rows);
     if (!grouped && uocr_gemm_tile_fits(epi, qt, a)) {
         const hipError_t e = uocr_gemm_tile_plain(st, epi, qt, a);
@@ -981,30 +872,22 @@ extern "C" hipError_t uocr_launch_gemm(hipStream_t st, int epi, const uocr_gemm_
         a.kst = kst;
         a.out = d->part;
         a.ldo = d->N;
-        gemm_dispatch<GE_PART, false>(st, qt, a, dim3(grid.x, grid.y, S), tmr);
+        gemm_dispatch<GE_PART, false>(st, qt, a, dim3(grid.x, grid.y, S));
         const size_t mn = (size_t)d->M * d->N;
-        const u32 mode = epi == UOCR_GEMM_VISION ? RD_VISION : (epi == UOCR_GEMM_F16 ? RD_F16 : RD_F32);
-        if (fuse_norm) {
-            hipLaunchKernelGGL(k_reduce_norm, dim3((d->M + 3u) / 4u), dim3(PB), 0, st, (const float *)d->part, S,
-                               d->M, (const h16 *)d->res, d->ldr, (h16 *)d->out, d->ldo, (const h16 *)d->norm_w,
-                               (h16 *)d->norm_out);
-            return hipGetLastError();
-        }
         hipLaunchKernelGGL(k_split_reduce, dim3((unsigned)((mn / 4u + PB - 1u) / PB)), dim3(PB), 0, st,
-                           (const float *)d->part, S, d->M, d->N, mode, (const h16 *)d->bias, d->act, d->split,
-                           (const h16 *)d->res, d->ldr, d->out, (h16 *)d->out1, (h16 *)d->out2,
-                           epi == UOCR_GEMM_VISION ? d->N : d->ldo);
+                           (const float *)d->part, S, d->M, d->N, (const h16 *)d->bias, d->act, d->split, (h16 *)d->out,
+                           (h16 *)d->out1, (h16 *)d->out2);
     } else if (epi == UOCR_GEMM_VISION) {
-        gemm_dispatch<GE_VISION, false>(st, qt, a, grid, tmr);
+        gemm_dispatch<GE_VISION, false>(st, qt, a, grid);
     } else if (epi == UOCR_GEMM_F32) {
-        if (grouped) gemm_dispatch<GE_F32, true>(st, qt, a, grid, tmr);
-        else gemm_dispatch<GE_F32, false>(st, qt, a, grid, tmr);
+        if (grouped) gemm_dispatch<GE_F32, true>(st, qt, a, grid);
+        else gemm_dispatch<GE_F32, false>(st, qt, a, grid);
     } else if (epi == UOCR_GEMM_SWIGLU) {
-        if (grouped) gemm_dispatch<GE_SWIGLU, true>(st, qt, a, grid, tmr);
-        else gemm_dispatch<GE_SWIGLU, false>(st, qt, a, grid, tmr);
+        if (grouped) gemm_dispatch<GE_SWIGLU, true>(st, qt, a, grid);
+        else gemm_dispatch<GE_SWIGLU, false>(st, qt, a, grid);
     } else {
-        if (grouped) gemm_dispatch<GE_F16, true>(st, qt, a, grid, tmr);
-        else gemm_dispatch<GE_F16, false>(st, qt, a, grid, tmr);
+        if (grouped) gemm_dispatch<GE_F16, true>(st, qt, a, grid);
+        else gemm_dispatch<GE_F16, false>(st, qt, a, grid);
         if (want_norm) {
             hipLaunchKernelGGL(k_rows_rmsnorm, dim3((d->M + 3u) / 4u), dim3(PB), 0, st, (const h16 *)d->out,
                                (const h16 *)d->norm_w, d->M, (h16 *)d->norm_out);
