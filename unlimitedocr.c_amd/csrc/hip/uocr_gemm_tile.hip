@@ -802,7 +802,9 @@ int choose(bool sw, u32 M, u32 N, u32 K) {
     if (K >= 3072u && narrow <= 256u) return CFG_NARROW_K8;
     if (narrow <= 384u) return CFG_LINES;
     /* 932 x 1280 x 6848: 65.1 (old), 47.3 (K in 2), 41.1 (K in 4); 1600 x 768
-     * x 3072: 32.4, 26.4, 26.0 */
+     * x 3072: 32.4, 26.4, 26.0; shorter sums lose with K in 4, whose steps are
+     * half as many and take twice as long: 932 x 1280 x 1280 13.9 -> 14.5, x
+     * 320 7.2 -> 8.1 */
     return K >= 4096u ? CFG_MID_K4 : CFG_MID;
 }
 
