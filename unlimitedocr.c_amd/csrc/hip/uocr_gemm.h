@@ -155,6 +155,8 @@ enum { GO_PLAIN = 0, GO_BY_ROW = 1, GO_BY_COL = 2 };
 /* The kernels of uocr_gemm_tile.hip: whether a plain GEMM's operands and sizes
  * fit them (16-byte aligned rows, 32-bit offsets), and its launch. */
 bool uocr_gemm_tile_fits(int epi, u32 qt, const GemmArgs &a);
+/* Whether a plain fp16 GEMM with fp32 output can take the router's half of uocr_gemm_tile_router. */
+bool uocr_gemm_router_fits(const GemmArgs &a);
 hipError_t uocr_gemm_tile_plain(hipStream_t st, int epi, u32 qt, const GemmArgs &a);
 /* The Q | K | V projection (N = 3 nseg) with RoPE and the cache scatter. */
 hipError_t uocr_gemm_tile_rope(hipStream_t st, u32 qt, GemmArgs a, const RopeDst &rd);

@@ -498,6 +498,68 @@ struct Half {
     }
 };
 
+/* The router's fp32 logits [M][64] of fp16 rows and weights.  Each logit is one
+ * sum over K in steps of 16 in ascending order, as the general kernel forms it:
+ * the six experts are chosen from the logits, and another order of the sum picks
+ * another expert where the 6th and 7th logit are a rounding apart (K in four
+ * partial sums: one row of 1.9 million).  So K cannot be split, and what bounds a
+ * block is the latency of its 20 steps: 4 of them are in flight, in lines of 128
+ * bytes (64 lanes on 64 rows, straight to registers, took 8.5 us more at 64 rows
+ * and above).  A block takes 64 rows, a wavefront 32 rows and 32 experts. */
+struct RouterHalf {
+    static constexpr u32 ROWS = 64u, CW = UOCR_K_EXPERTS, STAGE = (ROWS + CW) * 128u, RD = 5u, LDS = RD * STAGE;
+    static constexpr bool GROUPED = false;
+    static __device__ __forceinline__ void block(const GemmArgs &p, u32 id, uint8_t *sm) {
+        constexpr int NT = UOCR_K_HIDDEN / 64, NL = (int)(STAGE / 4096u); /* K steps, loads of a wavefront per step */
+        static_assert(UOCR_K_EXPERTS == 64, "two wavefronts along the experts");
+        const u32 lane = threadIdx.x & 63u, r = lane & 31u, h = lane >> 5, wave = uni(threadIdx.x >> 6);
+        const u32 row0 = id * ROWS;
+        if (row0 >= p.M) return;
+        const u32 lds0 = uni((u32)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)sm) + 2048u * wave;
+        /* the wavefront's 16 activation rows and 16 weight rows, swizzled as in tile_body */
+        u32 vx[2], vw[2];
+#pragma unroll
+        for (u32 i = 0; i < 2; ++i) {
+            const u32 row = 16u * wave + 8u * i + (lane >> 3), pc = 16u * ((lane & 7u) ^ (row >> 1 & 7u));
+            vx[i] = min(row0 + row, p.M - 1u) * p.lda * 2u + pc;
+            vw[i] = row * (UOCR_K_HIDDEN * 2u) + pc;
+        }
+        auto issue = [&](u32 s) {
+#pragma unroll
+            for (u32 i = 0; i < 2; ++i) {
+                lds_load16((const uint8_t *)p.A + 128u * s, vx[i], lds0 + s % RD * STAGE + 1024u * i);
+                lds_load16((const uint8_t *)p.W[0].w + 128u * s, vw[i], lds0 + s % RD * STAGE + ROWS * 128u + 1024u * i);
+            }
+        };
+        f32x16 acc;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
+#pragma unroll
+        for (u32 s = 0; s + 1u < RD; ++s) issue(s);
+        const uint8_t *xs = sm + 4096u * (wave >> 1) + 128u * r, *ws = sm + ROWS * 128u + 4096u * (wave & 1u) + 128u * r;
+        static_for<NT>([&](auto S) {
+            constexpr int s = decltype(S)::value, after = NT - 1 - s < (int)RD - 2 ? NT - 1 - s : (int)RD - 2;
+            /* step s has landed for all wavefronts; step s - 1's place is free */
+            wait_barrier<NL * after>();
+            if constexpr (s + (int)RD - 1 < NT) issue(s + RD - 1u);
+#pragma unroll
+            for (u32 i = 0; i < 4; ++i) {
+                const u32 at = s % RD * STAGE + 16u * ((b_koff<1>(i, h) / 8u) ^ (r >> 1 & 7u));
+                U4H8 x, w;
+                x.u = *(const uint4 *)(xs + at);
+                w.u = *(const uint4 *)(ws + at);
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(w.v, x.v, acc, 0, 0, 0);
+            }
+        });
+        const u32 row = row0 + 32u * (wave >> 1) + r;
+        if (row < p.M) {
+            float *o = (float *)p.out + (size_t)row * p.ldo + 32u * (wave & 1u) + 4u * h;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) *(float4 *)(o + 8 * q) = make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]);
+        }
+    }
+};
+
 /* Two GEMMs that do not read each other's output in one launch: blocks [0, na)
  * take A's tiles, the others B's. */
 template <typename A, typename B>
@@ -762,7 +824,6 @@ hipError_t plain(hipStream_t st, int epi, u32 qt, const GemmArgs &a) {
     const u32 tiles = (a.M + 32u * RT - 1u) / (32u * RT);
     switch (epi) {
         case GE_F16: return launch<GE_F16, false, RT, WN, WK>(st, qt, a, tiles);
-        case GE_F32: return launch<GE_F32, false, RT, WN, WK>(st, qt, a, tiles);
         case GE_VISION: return launch<GE_VISION, false, RT, WN, WK>(st, qt, a, tiles);
         case GE_SWIGLU: return launch<GE_SWIGLU, false, RT, WN, WK>(st, qt, a, tiles);
         default: return hipErrorInvalidValue;
@@ -773,7 +834,6 @@ hipError_t plain_lines(hipStream_t st, int epi, u32 qt, const GemmArgs &a) {
     const u32 tiles = (a.M + 31u) / 32u;
     switch (epi) {
         case GE_F16: return launch_lines<GE_F16, false>(st, qt, a, tiles);
-        case GE_F32: return launch_lines<GE_F32, false>(st, qt, a, tiles);
         case GE_VISION: return launch_lines<GE_VISION, false>(st, qt, a, tiles);
         case GE_SWIGLU: return launch_lines<GE_SWIGLU, false>(st, qt, a, tiles);
         default: return hipErrorInvalidValue;
@@ -813,8 +873,16 @@ int choose(bool sw, u32 M, u32 N, u32 K) {
 bool uocr_gemm_tile_fits(int epi, u32 qt, const GemmArgs &a) {
     const uint64_t rowb = qt == UOCR_QT_Q4 ? a.K / 2u : (qt == UOCR_QT_Q8 ? a.K : 2ull * a.K), lim = 1ull << 32;
     uintptr_t al = (uintptr_t)a.A | (uintptr_t)a.W[0].w | (epi == GE_SWIGLU ? (uintptr_t)a.W[1].w : 0u);
-    return a.vec != 0u && (epi == GE_F16 || epi == GE_F32 || epi == GE_SWIGLU || epi == GE_VISION) && a.nseg == 0u && al % 16u == 0u &&
+    /* a plain fp32 GEMM is the router's: its sums keep their order (RouterHalf, or the general kernel) */
+    const bool known = epi == GE_F16 || (epi == GE_F32 && a.tile_e != nullptr) || epi == GE_SWIGLU || epi == GE_VISION;
+    return a.vec != 0u && known && a.nseg == 0u && al % 16u == 0u &&
            (uint64_t)a.M * a.lda * 2u < lim && (uint64_t)a.M * a.ldr * 2u < lim && a.N * rowb < lim && (!a.packed || a.N % 32u == 0u);
+}
+
+bool uocr_gemm_router_fits(const GemmArgs &a) {
+    const uintptr_t al = (uintptr_t)a.A | (uintptr_t)a.W[0].w;
+    return a.vec != 0u && a.tile_e == nullptr && a.nseg == 0u && a.res == nullptr && a.N == UOCR_K_EXPERTS && a.K == UOCR_K_HIDDEN && al % 16u == 0u &&
+           (uint64_t)a.M * a.lda * 2u < 1ull << 32;
 }
 
 hipError_t uocr_gemm_tile_rope(hipStream_t st, u32 qt, GemmArgs a, const RopeDst &rd) {
@@ -902,9 +970,9 @@ hipError_t uocr_gemm_tile_pair(hipStream_t st, int eb, u32 qt, const GemmArgs &a
 }
 
 hipError_t uocr_gemm_tile_router(hipStream_t st, u32 qt, const GemmArgs &a, const GemmArgs &b) {
-    const u32 ta = (a.M + 63u) / 64u, tb = (b.M + 31u) / 32u;
-    typedef Half<1, GE_F32, false, false, 1, 1, 4> R;
-#define GO(Q, PK) launch_halves<Half<Q, GE_SWIGLU, false, PK, 2, 2, 2>, R>(st, qt, a, ta, UOCR_QT_F16, b, tb)
+    const u32 ta = (a.M + 63u) / 64u, tb = (b.M + RouterHalf::ROWS - 1u) / RouterHalf::ROWS;
+    /* the router first: its blocks are the longest chains of the launch */
+#define GO(Q, PK) launch_halves<RouterHalf, Half<Q, GE_SWIGLU, false, PK, 2, 2, 2>>(st, UOCR_QT_F16, b, tb, qt, a, ta)
     if (qt == UOCR_QT_F16) GO(1, false);
     else if (qt == UOCR_QT_Q8 && a.packed) GO(3, true);
     else if (qt == UOCR_QT_Q8) GO(3, false);

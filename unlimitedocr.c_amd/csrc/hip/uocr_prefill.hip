@@ -915,8 +915,7 @@ extern "C" hipError_t uocr_launch_gemm_pair(hipStream_t st, int epi_a, const uoc
             q == db->W[0].qtype && a.packed == b.packed) {
             return uocr_gemm_tile_pair(st, epi_b, q, a, b, db->pairs, db->tile_rows);
         }
-        if (epi_a == UOCR_GEMM_SWIGLU && epi_b == UOCR_GEMM_F32 && db->tile_e == nullptr && db->W[0].qtype == UOCR_QT_F16 &&
-            uocr_gemm_tile_fits(epi_b, UOCR_QT_F16, b)) {
+        if (epi_a == UOCR_GEMM_SWIGLU && epi_b == UOCR_GEMM_F32 && db->W[0].qtype == UOCR_QT_F16 && uocr_gemm_router_fits(b)) {
             return uocr_gemm_tile_router(st, q, a, b);
         }
     }
