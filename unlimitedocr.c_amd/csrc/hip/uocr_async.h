@@ -25,12 +25,18 @@ __device__ __forceinline__ T *uni(T *p) {
 
 /* 16 bytes per lane from base + voff straight into LDS at lds + 16 lane.  In
  * inline assembly because the compiler's own LDS-direct load makes every later
- * LDS read wait for all of them; wait_barrier counts them instead. */
+ * LDS read wait for all of them; wait_barrier counts them instead.  m0 holds
+ * the LDS address and is named as changed; the compiler warns that it reserves
+ * the register, yet only so it does not keep a value of its own there across
+ * the statement. */
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void lds_load16(const void *base, u32 voff, u32 lds) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                  :
                  : "v"(voff), "s"(uni(base)), "s"(lds)
-                 : "memory");
+                 : "memory", "m0");
 }
+#pragma clang diagnostic pop
 
 #endif /* UOCR_ASYNC_H */
