@@ -242,9 +242,10 @@ UOCR_API int uocr_op_gemm(uint32_t qtype, const void *w, const void *s, uint32_t
  * 161-221) and uocr_vision_gemm_q4_0_to_f16 (kernels/gemm_q4.metal:63-131),
  * and the fp16 path MPS matmul + bias/activation (uocr_metal.m:17232-17250,
  * kernels/dense.metal:68-79, kernels/sam.metal:93-104), which is fused here
- * (one fp16 rounding instead of two).  Where an output's rows are not
- * whole 16-byte pieces (n or split not a multiple of 8, or a pointer off a
- * 16-byte boundary), GEMMs with k >= 2048 on grids of fewer than 128 output
+ * (one fp16 rounding instead of two).  On the general kernel
+ * (uocr_op_gemm_kernel; also where an output's rows are not whole 16-byte
+ * pieces: n or split not a multiple of 8, or a pointer off a 16-byte boundary),
+ * GEMMs with k >= 2048 on grids of fewer than 128 output
  * tiles split K over up to 8 blocks per tile through an fp32 partials buffer that
  * the library allocates on first need (outside graph capture; under capture
  * without room the unsplit kernel runs) and keeps: such calls must not overlap.
@@ -253,6 +254,14 @@ UOCR_API int uocr_op_gemm(uint32_t qtype, const void *w, const void *s, uint32_t
 UOCR_API int uocr_op_vision_linear(uint32_t qtype, const void *w, const void *s, const void *bias, uint32_t m,
                                    uint32_t k, uint32_t n, uint32_t act, uint32_t split, const void *x, void *dst0,
                                    void *dst1, void *dst2);
+
+/* Which kernel uocr_op_vision_linear (vision != 0; act as there) or uocr_op_gemm
+ * (vision 0) runs for these sizes on operands whose rows are whole 16-byte
+ * pieces (no counterpart in the reference; for tests and diagnostics; needs no
+ * GPU): 0 the general kernel, 1 tiles of 128 x 256, 2 of 64 x 128 with K in 2
+ * groups of wavefronts, 3 the same in 4, 4 of 32 x 64 with K in 8, 5 of 32 x 64
+ * with K by lines of the weight rows; -1 bad arguments. */
+UOCR_API int uocr_op_gemm_kernel(uint32_t qtype, uint32_t m, uint32_t n, uint32_t k, int vision, uint32_t act);
 
 /* Causal attention of P prompt queries (fp16 [P][1280], RoPE applied) over
  * cache slots 0..P-1 of caches laid out [10][cache_capacity][128]; ctx fp16

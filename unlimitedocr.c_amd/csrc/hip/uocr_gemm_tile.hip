@@ -861,32 +861,54 @@ hipError_t plain_lines(hipStream_t st, int epi, u32 qt, const GemmArgs &a) {
     }
 }
 
-/* Which kernel a plain GEMM of M x N (SwiGLU: N pairs) x K takes.  A K step of
- * a block takes 0.6-0.9 us whatever it computes (its loads' latency), so the
- * large tile, the cheapest per output, is taken once its grid gives two thirds
- * of the CUs a block, and smaller grids split K over the wavefronts instead.
- * Measured (us, Q8, old kernel / large / 64 x 128, K in 2 / 32 x 64, K in 8 /
- * 32 x 64, K by lines):
- *   4001 x 1280 x 1280   34.9 / 27.7 / 28.9 / 78  / 62    160 large tiles
- *   4096 x 768 x 768     15.0 / 20.8 / 15.1 / 43  / 27     96
- *   932 x 1280 x 1280    25.2 / 25.6 / 13.6 / 25  / 22     40
- *   257 x 3072 x 1024    14.6 / 24.4 / 12.6 / 17  / 13.4   432 narrow tiles
- *   196 x 3072 x 768     13.2 / 23.2 / 13.0 / 17  / 10.0   336
- *   257 x 1024 x 4096    18.0 / 69   / 33   / 17  / 22     144
- *   300 x 1280 x 6848    68.2 / 109  / 47   / 23.5 / 28    200
- *   77 x 1280 x 896      13.4 / 17.0 / 9.2  / 6.8 / 6.2     60 */
-enum { CFG_LARGE, CFG_MID, CFG_MID_K4, CFG_NARROW_K8, CFG_LINES };
-
-int choose(bool sw, u32 M, u32 N, u32 K) {
-    const u32 n2 = sw ? 2u * N : N, large = ((M + 127u) / 128u) * ((n2 + 255u) / 256u), narrow = ((M + 31u) / 32u) * ((n2 + 63u) / 64u);
-    if (large >= 160u) return CFG_LARGE;
-    if (K >= 3072u && narrow <= 256u) return CFG_NARROW_K8;
-    if (narrow <= 384u) return CFG_LINES;
-    /* 932 x 1280 x 6848: 65.1 (old), 47.3 (K in 2), 41.1 (K in 4); 1600 x 768
-     * x 3072: 32.4, 26.4, 26.0; shorter sums lose with K in 4, whose steps are
-     * half as many and take twice as long: 932 x 1280 x 1280 13.9 -> 14.5, x
-     * 320 7.2 -> 8.1 */
-    return K >= 4096u ? CFG_MID_K4 : CFG_MID;
+/* Which kernel a plain GEMM of M x N (SwiGLU: N pairs) x K takes, by the blocks
+ * of its grids (large, mid, narrow: tiles of 128 x 256, 64 x 128, 32 x 64).  A K
+ * step of a block takes 0.6-0.9 us whatever it computes (its loads' latency):
+ *  - the large tile, the cheapest per output, once the mid grid is over its two
+ *    blocks per CU;
+ *  - up to a narrow block per CU, K split over the block's wavefronts: by lines
+ *    while a line holds several K steps, in 8 groups for long sums;
+ *  - else the mid tile, K in 2 groups, or in 4 where the sums are long and each
+ *    block has a CU of its own (at 1280 the groups' merge costs more: 932 x 1280
+ *    x 1280 13.9 -> 14.5).  Q4 lines hold 4 K steps, so K by lines stays the
+ *    better one there for another half a round.
+ * The general kernel (64 x 128, K split over blocks for long vision sums) is
+ * the better one for vision linears
+ *  - with long sums on so few rows that its K splits are what fills the CUs, and,
+ *    for quantised weights, between a narrow block per CU and 100 mid tiles;
+ *  - with Q4 weights and an activation at up to one and a half rounds: its
+ *    weights skip LDS and all its wavefronts share the epilogue.
+ * Measured (us): general / large / mid, K in 2 / in 4 / narrow, K in 8 / lines
+ *   Q8   3500 x 1280 x 6848   123  /  97  / 118  / 128  / 200  / 229    550 mid
+ *   Q8   2000 x 1280 x 6848   78.7 / 93.9 / 65.8 / 85.2 / 113  / 130    320
+ *   Q8    932 x 1280 x 6848   68.9 / 94.5 / 46.9 / 41.5                 150
+ *   F16   500 x 1280 x 6848   52.3 / 92.4 / 45.6 / 39.9 / 43.1 / 74.5   320 narrow
+ *   Q8    257 x 1280 x 6848   67.5 / 94.7 / 46.3 / 41.5 / 23.4 / 28.3   180
+ *   Q4    500 x 1280 x 1280   16.2 / 25.1 / 12.8 / 12.8 / 16.7 / 12.2   320
+ *   Q8    500 x 1280 x 1280   16.9 / 23.6 / 11.9 / 11.7 / 15.8 / 15.0   320
+ *   Q4    257 x 1280 x 1280   16.2 / 25.0 / 12.7 / 12.6 /  9.1 /  7.3   180
+ *   F16   257 x 1280 x 1792   23.0 / 26.3 / 11.7 / 12.0 /  8.3 / 12.6   180
+ *  vision:
+ *   Q8   1960 x 2304 x 768    20.0 / 16.7 / 18.7 / 25.8                 558 mid
+ *   Q8   1600 x 768 x 768     10.9 / 15.1 /  8.9 /  9.5 / 18.5 / 13.6   150
+ *   Q4   1600 x 3072 x 768    19.8 / 21.1 / 23.6   (GELU)               600
+ *   Q4   1176 x 3072 x 768    15.3 / 20.5 / 15.9   (GELU)               456
+ *   Q4    514 x 1024 x 4096   21.8 / 60.6 / 28.6 / 26.3 / 29.8 / 32.4   272 narrow
+ *   F16   514 x 1024 x 4096   25.4 / 55.6 / 26.6 / 23.9 / 24.9 / 41.6   272
+ *   Q8    257 x 1024 x 4096   17.5 / 57.1 / 26.3 / 24.4 / 14.8 / 21.1   144
+ *   Q4    300 x 768 x 3072    13.1 /                      14.2          120
+ *   Q4    101 x 1024 x 4096   12.1 / 60.0 / 28.6 / 26.4 / 15.7 / 17.2    64 */
+int choose(int epi, u32 qt, u32 M, u32 N, u32 K, u32 act) {
+    const u32 n2 = epi == GE_SWIGLU ? 2u * N : N;
+    const u32 mid = ((M + 63u) / 64u) * ((n2 + 127u) / 128u), narrow = ((M + 31u) / 32u) * ((n2 + 63u) / 64u);
+    if (epi == GE_VISION) {
+        if (K >= 2048u && (narrow < (qt == UOCR_QT_Q4 ? 128u : 100u) || (qt != UOCR_QT_F16 && narrow > 256u && mid < 100u))) return UOCR_GEMM_KERNEL_GENERAL;
+        if (qt == UOCR_QT_Q4 && act != UOCR_VISION_ACT_NONE && K <= 1024u && mid > 256u && mid <= 768u) return UOCR_GEMM_KERNEL_GENERAL;
+    }
+    if (mid > 512u) return UOCR_GEMM_KERNEL_LARGE;
+    if (narrow <= 256u) return K >= (qt == UOCR_QT_F16 ? 1280u : 3072u) ? UOCR_GEMM_KERNEL_NARROW : UOCR_GEMM_KERNEL_LINES;
+    if (qt == UOCR_QT_Q4 && K < 3072u && narrow <= 384u) return UOCR_GEMM_KERNEL_LINES;
+    return K >= 3072u && mid <= 256u ? UOCR_GEMM_KERNEL_MID_K4 : UOCR_GEMM_KERNEL_MID;
 }
 
 }  // namespace
@@ -895,6 +917,7 @@ bool uocr_gemm_tile_fits(int epi, u32 qt, const GemmArgs &a) {
     const uint64_t rowb = qt == UOCR_QT_Q4 ? a.K / 2u : (qt == UOCR_QT_Q8 ? a.K : 2ull * a.K), lim = 1ull << 32;
     uintptr_t al = (uintptr_t)a.A | (uintptr_t)a.W[0].w | (epi == GE_SWIGLU ? (uintptr_t)a.W[1].w : 0u);
     /* a plain fp32 GEMM is the router's: its sums keep their order (RouterHalf, or the general kernel) */
+    if (epi == GE_VISION && choose(epi, qt, a.M, a.N, a.K, a.act) == UOCR_GEMM_KERNEL_GENERAL) return false;
     const bool known = epi == GE_F16 || (epi == GE_F32 && a.tile_e != nullptr) || epi == GE_SWIGLU || epi == GE_VISION;
     return a.vec != 0u && known && a.nseg == 0u && al % 16u == 0u &&
            (uint64_t)a.M * a.lda * 2u < lim && (uint64_t)a.M * a.ldr * 2u < lim && a.N * rowb < lim && (!a.packed || a.N % 32u == 0u);
@@ -907,9 +930,9 @@ bool uocr_gemm_router_fits(const GemmArgs &a) {
 }
 
 hipError_t uocr_gemm_tile_rope(hipStream_t st, u32 qt, GemmArgs a, const RopeDst &rd) {
-    /* 932 rows: 64 x 128 tiles, K in 2 (450 blocks); from 160 large tiles on
-     * those (a head pair per tile) */
-    const bool large = choose(false, a.M, a.N, a.K) == CFG_LARGE;
+    /* 932 rows: 64 x 128 tiles, K in 2 (450 blocks); over two of them per CU
+     * large tiles (a head pair per tile) */
+    const bool large = choose(GE_ROPE, qt, a.M, a.N, a.K, 0u) == UOCR_GEMM_KERNEL_LARGE;
     const dim3 grid = tile_grid(a, (a.M + (large ? 127u : 63u)) / (large ? 128u : 64u), a.N / (large ? 256u : 128u), qt, false);
 #define GO(Q, PK)                                                                                                      \
     do {                                                                                                               \
@@ -1004,11 +1027,15 @@ hipError_t uocr_gemm_tile_router(hipStream_t st, u32 qt, const GemmArgs &a, cons
 }
 
 hipError_t uocr_gemm_tile_plain(hipStream_t st, int epi, u32 qt, const GemmArgs &a) {
-    switch (choose(epi == GE_SWIGLU, a.M, a.N, a.K)) {
-        case CFG_LARGE: return plain<4, 4, 1>(st, epi, qt, a);
-        case CFG_MID: return plain<2, 2, 2>(st, epi, qt, a);
-        case CFG_MID_K4: return plain<2, 2, 4>(st, epi, qt, a);
-        case CFG_NARROW_K8: return plain<1, 1, 8>(st, epi, qt, a);
+    switch (choose(epi, qt, a.M, a.N, a.K, a.act)) {
+        case UOCR_GEMM_KERNEL_LARGE: return plain<4, 4, 1>(st, epi, qt, a);
+        case UOCR_GEMM_KERNEL_MID: return plain<2, 2, 2>(st, epi, qt, a);
+        case UOCR_GEMM_KERNEL_MID_K4: return plain<2, 2, 4>(st, epi, qt, a);
+        case UOCR_GEMM_KERNEL_NARROW: return plain<1, 1, 8>(st, epi, qt, a);
         default: return plain_lines(st, epi, qt, a);
     }
+}
+
+extern "C" int uocr_gemm_kernel_choice(uint32_t qtype, uint32_t M, uint32_t N, uint32_t K, int vision, uint32_t act) {
+    return choose(vision ? GE_VISION : GE_F16, qtype, M, N, K, act);
 }

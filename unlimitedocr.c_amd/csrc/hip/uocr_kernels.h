@@ -265,6 +265,17 @@ hipError_t uocr_launch_gemm(hipStream_t st, int epi, const uocr_gemm_desc *d);
 /* 1 when uocr_launch_gemm runs d in one launch that needs no partials (ksplit
  * and part are then ignored). */
 int uocr_gemm_splits_itself(int epi, const uocr_gemm_desc *d);
+/* The kernel that a plain GEMM (F16 output, or a vision linear) takes whose rows
+ * are whole 16-byte pieces; as uocr_op_gemm_kernel returns it. */
+enum {
+    UOCR_GEMM_KERNEL_GENERAL = 0,
+    UOCR_GEMM_KERNEL_LARGE = 1,
+    UOCR_GEMM_KERNEL_MID = 2,
+    UOCR_GEMM_KERNEL_MID_K4 = 3,
+    UOCR_GEMM_KERNEL_NARROW = 4,
+    UOCR_GEMM_KERNEL_LINES = 5
+};
+int uocr_gemm_kernel_choice(uint32_t qtype, uint32_t M, uint32_t N, uint32_t K, int vision, uint32_t act);
 /* Two independent GEMMs in one launch where both fit the tiled kernels: A
  * plain F16 with B grouped F16 or F32 of the same weight type and layout, or A
  * plain SwiGLU with B plain fp16 F32 (the router); two launches else. */

@@ -418,6 +418,11 @@ extern "C" int uocr_op_vision_linear(uint32_t qtype, const void *w, const void *
     return hip_status(uocr_launch_gemm(st, UOCR_GEMM_VISION, &d), "vision linear");
 }
 
+extern "C" int uocr_op_gemm_kernel(uint32_t qtype, uint32_t m, uint32_t n, uint32_t k, int vision, uint32_t act) {
+    if (!qt_ok(qtype) || m == 0u || n == 0u || k == 0u || k % 64u != 0u || act > UOCR_VISION_ACT_GELU_ERF) return -1;
+    return n % 8u != 0u ? (int)UOCR_GEMM_KERNEL_GENERAL : uocr_gemm_kernel_choice(qtype, m, n, k, vision, act);
+}
+
 extern "C" int uocr_op_prefill_attention(const void *q, const void *k_cache, const void *v_cache,
                                          uint32_t cache_capacity, uint32_t prompt_length, void *ctx) {
     if (q == nullptr || k_cache == nullptr || v_cache == nullptr || ctx == nullptr || prompt_length == 0u ||

@@ -141,6 +141,7 @@ SIGNATURES = {
     "uocr_op_embed": ([_U32, _VP, _VP, _U32, _VP, _VP], ct.c_int),
     "uocr_op_gemm": ([_U32, _VP, _VP, _U32, _U32, _U32, _VP, _VP, _VP], ct.c_int),
     "uocr_op_vision_linear": ([_U32, _VP, _VP, _VP, _U32, _U32, _U32, _U32, _U32, _VP, _VP, _VP, _VP], ct.c_int),
+    "uocr_op_gemm_kernel": ([_U32, _U32, _U32, _U32, ct.c_int, _U32], ct.c_int),
     "uocr_op_prefill_attention": ([_VP, _VP, _VP, _U32, _U32, _VP], ct.c_int),
     "uocr_op_moe_rows_workspace_bytes": ([_U32], _SZ),
     "uocr_op_moe_ffn_rows": ([ct.POINTER(CMoeWeights), _VP, _VP, _VP, _U32, ct.c_int, _VP, _VP], ct.c_int),
@@ -567,6 +568,17 @@ def op_vision_linear(qtype, w, s, bias, m, k, n, act, split, x, dst0, dst1=None,
     """dst = f16(act(x . W^T + bias)); split != 0 routes column thirds to dst0/dst1/dst2."""
     _check_op(load_library().uocr_op_vision_linear(qtype, _p(w), _p(s), _p(bias), m, k, n, act, split, _p(x),
                                                    _p(dst0), _p(dst1), _p(dst2)), "op_vision_linear")
+
+
+GEMM_KERNELS = ("general", "large", "mid", "mid_k4", "narrow", "lines")
+
+
+def op_gemm_kernel(qtype, m, n, k, vision=False, act=0) -> str:
+    """Name of the kernel that op_gemm (or op_vision_linear) takes on rows of whole 16-byte pieces."""
+    r = load_library().uocr_op_gemm_kernel(qtype, m, n, k, int(vision), act)
+    if r < 0:
+        raise ValueError("op_gemm_kernel: bad arguments")
+    return GEMM_KERNELS[r]
 
 
 def op_prefill_attention(q, kc, vc, cap, prompt_len, ctx) -> None:
