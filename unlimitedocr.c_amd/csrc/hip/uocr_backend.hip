@@ -89,10 +89,12 @@ struct uocr_hip_ctx {
     float *lg_part; /* [4 x 64] quarters of the exact router logits (folded router) */
     int64_t *racc; /* un-normalised router logits, fixed point (k_attn_out -> k_moe_gate_up) */
     int fold_select; /* the token is chosen in layer 0's QKV launch (not a finalize launch) */
+    int prefill_ksplit; /* small-grid prefill GEMMs split K */
     uint32_t *route_ids;
     /* MFMA prefill scratch, sized for prompt_cap rows */
     uint16_t *p_xn, *p_q, *p_ctx, *p_a, *p_mid, *p_smid, *p_sout, *p_rmid;
     float *p_rope;  /* prefill RoPE (cos, sin) per token and pair */
+    float *p_kpart; /* prefill GEMM split-K partials */
     float *p_logits, *p_wts;
     uint16_t *p_y; /* per-pair routed expert outputs, fp16 */
     int32_t *p_ids, *p_offsets, *p_tile_e, *p_tile_s0, *p_tile_s1, *p_ntiles, *p_list_tok,
@@ -505,6 +507,9 @@ extern "C" int uocr_hip_context_map_model(uocr_hip_ctx *ctx, const uocr_decoder_
     /* UOCR_HIP_NO_SELECT_FOLD=1 chooses each token in a finalize launch after the LM head */
     const char *ns = getenv("UOCR_HIP_NO_SELECT_FOLD");
     ctx->fold_select = !(ns != nullptr && atoi(ns) != 0);
+    /* UOCR_HIP_NO_PREFILL_KSPLIT=1 runs every prefill GEMM unsplit */
+    const char *nk = getenv("UOCR_HIP_NO_PREFILL_KSPLIT");
+    ctx->prefill_ksplit = !(nk != nullptr && atoi(nk) != 0);
     /* size pass */
     uint64_t total = tensor_bytes(b->embed) + tensor_bytes(b->lm_head) + tensor_bytes(b->final_norm);
     for (uint32_t l = 0; l < UOCR_DECODER_LAYERS; ++l) {
@@ -677,6 +682,8 @@ extern "C" int uocr_hip_context_allocate_runtime(uocr_hip_ctx *ctx, uint32_t pro
     const uint64_t o_poff = p.take(64u * 4u);
     const uint64_t o_pte = p.take(max_tiles * 4u), o_pts0 = p.take(max_tiles * 4u), o_pts1 = p.take(max_tiles * 4u);
     const uint64_t o_pnt = p.take(4u), o_plt = p.take(PK * 4u), o_plp = p.take(PK * 4u);
+    /* split-K partials of the O projection and the dense down, fp32 */
+    const uint64_t o_pkp = p.take(std::min<uint64_t>(Pc, UOCR_KSPLIT_ROWS) * H_SIZE * UOCR_KSPLIT_MAX * 4u);
     const uint64_t o_run = p.take(uocr_run_arena_bytes());
     const uint64_t total = p.off;
     HIPCHK(counted_malloc(ctx, (void **)&ctx->rarena, total), "runtime arena allocation");
@@ -726,6 +733,7 @@ extern "C" int uocr_hip_context_allocate_runtime(uocr_hip_ctx *ctx, uint32_t pro
     ctx->p_list_tok = (int32_t *)(b + o_plt);
     ctx->p_list_pair = (int32_t *)(b + o_plp);
     ctx->p_rope = (float *)(b + o_prope);
+    ctx->p_kpart = (float *)(b + o_pkp);
     ctx->run_arena = b + o_run;
     ctx->run_tag = 1u; /* the arena is zero: tag 0 never matches */
     ctx->p_max_tiles = max_tiles;
@@ -902,6 +910,14 @@ static hipError_t enqueue_prefill_step(uocr_hip_ctx *c) {
     return e;
 }
 
+/* K split over blocks where that is the faster form (the O projection and
+ * layer 0's dense down). */
+static void with_ksplit(const uocr_hip_ctx *c, uocr_gemm_desc &d) {
+    if (!c->prefill_ksplit || d.norm_w == nullptr || d.M > UOCR_KSPLIT_ROWS || d.N > H_SIZE) return;
+    d.ksplit = uocr_gemm_ksplit(d.W[0].qtype, d.M, d.N, d.K);
+    d.part = c->p_kpart;
+}
+
 static uocr_gemm_desc gdesc(const uint16_t *A, uint32_t lda, uint32_t M, uint32_t N, uint32_t K, void *out,
                            uint32_t ldo) {
     uocr_gemm_desc d;
@@ -966,6 +982,7 @@ static hipError_t enqueue_prefill_mfma(uocr_hip_ctx *c, uint32_t P) {
         d.ldr = H_SIZE;
         d.norm_w = L.post_norm;
         d.norm_out = c->p_xn;
+        with_ksplit(c, d);
         ENQ(uocr_launch_gemm(s, UOCR_GEMM_F16, &d));
         if (l == 0u) {
             const uint32_t I0 = UOCR_DENSE_LAYER0_INTERMEDIATE;
@@ -981,6 +998,7 @@ static hipError_t enqueue_prefill_mfma(uocr_hip_ctx *c, uint32_t P) {
             d.ldr = H_SIZE;
             d.norm_w = next_norm;
             d.norm_out = next_norm != nullptr ? c->p_xn : nullptr;
+            with_ksplit(c, d);
             ENQ(uocr_launch_gemm(s, UOCR_GEMM_F16, &d));
             continue;
         }

@@ -246,7 +246,7 @@ typedef struct uocr_gemm_desc {
     const uint16_t *bias;
     uint32_t act, split;
     void *out1, *out2;
-    /* UOCR_GEMM_VISION: ksplit > 1 splits K over
+    /* UOCR_GEMM_VISION, and UOCR_GEMM_F16 with norm_w: ksplit > 1 splits K over
      * that many blocks per tile, each writing fp32 partials into part
      * ([ksplit][M][N] floats), reduced in order by a second kernel that
      * applies the epilogue; ksplit <= 1 or part NULL: no split */
@@ -256,7 +256,7 @@ typedef struct uocr_gemm_desc {
      * copy of uocr_launch_pack_gemm_rows instead of the row-major payload */
     uint32_t packed;
     /* UOCR_GEMM_F16, not grouped, N == ldo == 1280: norm_w set also writes
-     * norm_out = f16(rmsnorm(out) * norm_w) */
+     * norm_out = f16(rmsnorm(out) * norm_w) (fused into the split-K reduce) */
     const uint16_t *norm_w;
     uint16_t *norm_out;
 } uocr_gemm_desc;
@@ -289,6 +289,12 @@ hipError_t uocr_launch_gemm_pair(hipStream_t st, int epi_a, const uocr_gemm_desc
  * contiguous run per step (lane 32h + r takes row r's half h). */
 hipError_t uocr_launch_pack_gemm_rows(hipStream_t st, uint32_t qtype, const void *src, void *dst, uint32_t rows,
                                       uint32_t K, uint32_t count, uint64_t stride);
+/* K splits (1: none) for the prompt's F16 GEMM of M x N x K with norm_w; the
+ * partials of at most UOCR_KSPLIT_MAX splits and UOCR_KSPLIT_ROWS rows (from
+ * there on a grid of 1280 columns has 256 blocks and more). */
+#define UOCR_KSPLIT_MAX 4u
+#define UOCR_KSPLIT_ROWS 1600u
+uint32_t uocr_gemm_ksplit(uint32_t qtype, uint32_t M, uint32_t N, uint32_t K);
 /* y[t] = rmsnorm(x[t], w) for P rows of 1280. */
 hipError_t uocr_launch_rows_rmsnorm(hipStream_t st, const uint16_t *x, const uint16_t *w, uint32_t P, uint16_t *y);
 /* cs [P][64][2] = (cos, sin) of t * inv_freq[d] for tokens t < P (inv_freq:

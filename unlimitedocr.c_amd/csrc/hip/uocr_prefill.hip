@@ -488,6 +488,72 @@ __global__ __launch_bounds__(PB) void k_rows_rmsnorm(const h16 *__restrict__ x, 
     row_norm_tail(v, lane, wv, y + (size_t)row * UOCR_K_HIDDEN);
 }
 
+/* Split-K reduce of a 1280-column fp16 GEMM output with its residual, fused
+ * with the RMSNorm that reads it: per row (one wavefront), out = f16(sum of
+ * the S planes in order + res), then y = rmsnorm(out) * w as k_rows_rmsnorm
+ * rounds it. */
+__global__ __launch_bounds__(PB) void k_reduce_norm(const float *__restrict__ part, u32 S, u32 M,
+                                                    const h16 *__restrict__ res, u32 ldr, h16 *__restrict__ out,
+                                                    u32 ldo, const h16 *__restrict__ w, h16 *__restrict__ y) {
+    const u32 row = blockIdx.x * (PB / 64) + (threadIdx.x >> 6), lane = threadIdx.x & 63u;
+    if (row >= M) return;
+    const size_t MN = (size_t)M * UOCR_K_HIDDEN;
+    /* the first two planes of the row's pieces (and the residual), all in
+     * flight before any sum; planes beyond the second are added in order
+     * after them */
+    float4 pa[3][2], pb2[3][2];
+    U4H8 rr[3], wv[3];
+    norm_w_load(w, lane, wv);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        const u32 i = min(lane + 64u * q, UOCR_K_HIDDEN / 8u - 1u);
+        const float *p0 = part + (size_t)row * UOCR_K_HIDDEN + 8u * i;
+#pragma unroll
+        for (u32 z = 0; z < 2u; ++z) {
+            if (z < S) {
+                pa[q][z] = *(const float4 *)(p0 + z * MN);
+                pb2[q][z] = *(const float4 *)(p0 + z * MN + 4);
+            }
+        }
+        if (res != nullptr) rr[q].u = *(const uint4 *)(res + (size_t)row * ldr + 8u * i);
+    }
+    U4H8 v[3];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        const u32 i = lane + 64u * q;
+        if (i >= UOCR_K_HIDDEN / 8u) continue;
+        const float *p0 = part + (size_t)row * UOCR_K_HIDDEN + 8u * i;
+        float4 a = pa[q][0], b = pb2[q][0];
+        if (S > 1u) {
+            const float4 c = pa[q][1], d = pb2[q][1];
+            a.x += c.x;
+            a.y += c.y;
+            a.z += c.z;
+            a.w += c.w;
+            b.x += d.x;
+            b.y += d.y;
+            b.z += d.z;
+            b.w += d.w;
+        }
+        for (u32 z = 2; z < S; ++z) {
+            const float4 c = *(const float4 *)(p0 + z * MN), d = *(const float4 *)(p0 + z * MN + 4);
+            a.x += c.x;
+            a.y += c.y;
+            a.z += c.z;
+            a.w += c.w;
+            b.x += d.x;
+            b.y += d.y;
+            b.z += d.z;
+            b.w += d.w;
+        }
+        const float r[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[q].h[j] = (h16)(res != nullptr ? r[j] + (float)rr[q].h[j] : r[j]);
+        *(uint4 *)(out + (size_t)row * ldo + 8u * i) = v[q].u;
+    }
+    row_norm_tail(v, lane, wv, y + (size_t)row * UOCR_K_HIDDEN);
+}
+
 /* ------------------------------------------------------------------------ */
 /* MoE routing, buckets, combine                                             */
 /* ------------------------------------------------------------------------ */
@@ -774,6 +840,29 @@ static void gemm_dispatch(hipStream_t st, u32 qt, GemmArgs a, dim3 grid) {
     gemm_dispatch_tm<EPI, GROUPED, TM>(st, qt, a, grid, shm);
 }
 
+/* Splits of K over blocks for the prompt's O projection (K = 1280) and layer 0's
+ * dense down (6848), N = 1280 both, summed by k_reduce_norm together with the
+ * residual and the next norm; 1: the tiled kernel and a norm launch.  A split
+ * grid fills the chip where the tiles' grids do not: with quantised weights from
+ * one round of 32 x 64 tiles up to 190 tiles of 64 x 128, with fp16 weights
+ * also below (each 32-row tile fetches all of the weights, four times the bytes
+ * of Q4) and up to a tile per CU.  Measured in a prompt's first layer (us, GEMM + reduce or norm, split / tiled):
+ *   rows                      64          384         400         932        1200        1600
+ *   O projection, Q8     13.8 / 13.4  15.2 / 13.8 16.4 / 19.6 19.4 / 20.2 20.8 / 20.7 23.7 / 21.9
+ *   O projection, F16    13.0 / 16.6  14.1 / 16.4 16.7 / 22.0 19.9 / 23.5 21.6 / 24.1 23.0 / 23.7
+ *   dense down, Q4       28.1 / 28.1  30.1 / 29.6 32.3 / 44.8 43.4 / 48.3 46.1 / 49.4 62.3 / 53.1
+ *   dense down, Q8       28.9 / 30.1  30.2 / 30.9 32.8 / 47.3 46.1 / 51.5 49.9 / 51.9 66.4 / 52.9
+ *   dense down, F16      23.3 / 38.3  29.6 / 37.2 40.6 / 60.8 55.9 / 64.5 56.5 / 66.1 65.9 / 66.5
+ * The split count: doubling while the grid stays within 512 blocks and a split
+ * keeps 5 K steps, or a split keeps 16. */
+extern "C" uint32_t uocr_gemm_ksplit(uint32_t qtype, uint32_t M, uint32_t N, uint32_t K) {
+    const u32 blocks = ((M + TM - 1u) / TM) * ((N + TN - 1u) / TN), narrow = ((M + 31u) / 32u) * ((N + 63u) / 64u), steps = K / TK;
+    if (qtype == UOCR_QT_F16 ? blocks >= 256u : narrow <= 256u || blocks > 190u) return 1u;
+    u32 s = 1u;
+    while (s < UOCR_KSPLIT_MAX && ((blocks * 2u * s <= 512u && steps / (2u * s) >= 5u) || steps / (2u * s) >= 16u)) s *= 2u;
+    return s;
+}
+
 static bool gemm_desc_ok(int epi, const uocr_gemm_desc *d) {
     if (d == nullptr || d->A == nullptr || d->out == nullptr || d->N == 0u || d->K == 0u || d->K % 64u != 0u ||
         d->lda % 8u != 0u || !pmat_ok(d->W[0]) || (epi == UOCR_GEMM_SWIGLU && (!pmat_ok(d->W[1]) || d->W[1].qtype != d->W[0].qtype)) ||
@@ -847,16 +936,17 @@ extern "C" hipError_t uocr_launch_gemm(hipStream_t st, int epi, const uocr_gemm_
                                                         d->out2 == nullptr)))) {
         return hipErrorInvalidValue;
     }
-    const bool splittable = epi == UOCR_GEMM_VISION && d->ksplit > 1u && d->part != nullptr && d->N % 4u == 0u && d->split % 4u == 0u;
-    /* norm_w: the F16 output rows also go through the RMSNorm into norm_out,
-     * a row-norm launch after the GEMM */
+    const bool split = !grouped && d->ksplit > 1u && d->part != nullptr;
+    /* norm_w: the F16 output rows also go through the RMSNorm into norm_out
+     * (fused into the split-K reduce, else a row-norm launch after the GEMM) */
     const bool want_norm = d->norm_w != nullptr;
     if (want_norm && (epi != UOCR_GEMM_F16 || grouped || d->norm_out == nullptr || d->N != UOCR_K_HIDDEN ||
                       d->ldo != UOCR_K_HIDDEN || (d->res != nullptr && d->ldr % 8u != 0u))) {
         return hipErrorInvalidValue;
     }
     if (grouped && d->tile_rows != 0u) return uocr_gemm_tile_grouped(st, epi, qt, a, d->pairs, d->tile_rows);
-    if (!grouped && uocr_gemm_tile_fits(epi, qt, a)) {
+    const bool fused = split && want_norm, splittable = fused || (split && epi == UOCR_GEMM_VISION && d->N % 4u == 0u && d->split % 4u == 0u);
+    if (!grouped && !fused && uocr_gemm_tile_fits(epi, qt, a)) {
         const hipError_t e = uocr_gemm_tile_plain(st, epi, qt, a);
         if (e != hipSuccess || !want_norm) return e;
         hipLaunchKernelGGL(k_rows_rmsnorm, dim3((d->M + 3u) / 4u), dim3(PB), 0, st, (const h16 *)d->out,
@@ -873,6 +963,11 @@ extern "C" hipError_t uocr_launch_gemm(hipStream_t st, int epi, const uocr_gemm_
         a.out = d->part;
         a.ldo = d->N;
         gemm_dispatch<GE_PART, false>(st, qt, a, dim3(grid.x, grid.y, S));
+        if (fused) {
+            hipLaunchKernelGGL(k_reduce_norm, dim3((d->M + 3u) / 4u), dim3(PB), 0, st, (const float *)d->part, S, d->M, (const h16 *)d->res, d->ldr,
+                               (h16 *)d->out, d->ldo, (const h16 *)d->norm_w, (h16 *)d->norm_out);
+            return hipGetLastError();
+        }
         const size_t mn = (size_t)d->M * d->N;
         hipLaunchKernelGGL(k_split_reduce, dim3((unsigned)((mn / 4u + PB - 1u) / PB)), dim3(PB), 0, st,
                            (const float *)d->part, S, d->M, d->N, (const h16 *)d->bias, d->act, d->split, (h16 *)d->out,
