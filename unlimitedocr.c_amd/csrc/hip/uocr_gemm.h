@@ -147,10 +147,8 @@ struct GemmArgs {
     u32 sc_lds;          /* the block's scale rows are preloaded into dynamic LDS */
     u32 packed;          /* Q4/Q8 payloads in the GEMM-packed layout */
     u32 vec;             /* rows of the outputs, the residual and the bias are whole 16-byte pieces */
-    u32 nx, ny, order;   /* row tiles, column tiles and GO_* */
+    u32 nx, ny, by_row;  /* row tiles, column tiles; each XCD takes a run of row (else column) tiles */
 };
-
-enum { GO_PLAIN = 0, GO_BY_ROW = 1, GO_BY_COL = 2 };
 
 /* The kernels of uocr_gemm_tile.hip: whether a plain GEMM's operands and sizes
  * fit them (16-byte aligned rows, 32-bit offsets), and its launch. */

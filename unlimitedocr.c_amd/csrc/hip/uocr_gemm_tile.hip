@@ -11,19 +11,14 @@
 
 namespace {
 
-/* The block's tile.  Blocks go to the 8 XCDs in turn; with by_row or by_col
- * each XCD takes a contiguous run of row tiles (of column tiles) instead, so
- * that its L2 fetches only its share of the activations (of the weights). */
-__device__ __forceinline__ bool tile_of(u32 id, u32 order, u32 nx, u32 ny, u32 &bx, u32 &by) {
-    if (order == GO_PLAIN) {
-        bx = id % nx;
-        by = id / nx;
-        return by < ny;
-    }
+/* The block's tile.  Blocks go to the 8 XCDs in turn; each XCD takes a
+ * contiguous run of row tiles (by_row; else of column tiles), so that its L2
+ * fetches only its share of the activations (of the weights). */
+__device__ __forceinline__ bool tile_of(u32 id, bool by_row, u32 nx, u32 ny, u32 &bx, u32 &by) {
     const u32 total = nx * ny, q = total / 8u, rem = total % 8u, x = id % 8u, slot = id / 8u;
     if (slot >= q + (x < rem ? 1u : 0u)) return false;
     const u32 l = x * q + min(x, rem) + slot;
-    if (order == GO_BY_ROW) {
+    if (by_row) {
         bx = l / ny;
         by = l % ny;
     } else {
@@ -479,7 +474,7 @@ __device__ __forceinline__ void tile_body(const GemmArgs &p, u32 bx, u32 by, uin
 template <int QT, int EPI, bool GROUPED, bool PACKED, int RT, int WN, int WK>
 __device__ __forceinline__ void tile_block(const GemmArgs &p, u32 id, uint8_t *sm, const RopeDst &rd) {
     u32 bx, by;
-    if (!tile_of(id, p.order, GROUPED ? (u32)*p.ntiles : p.nx, p.ny, bx, by)) return;
+    if (!tile_of(id, p.by_row != 0u, GROUPED ? (u32)*p.ntiles : p.nx, p.ny, bx, by)) return;
     if constexpr (GROUPED && RT == 4) {
         const u32 rows = uni((u32)p.tile_s1[bx]) - uni((u32)p.tile_s0[bx]);
         if (rows <= 32u) return tile_body<QT, EPI, GROUPED, PACKED, 1, WN, WK>(p, bx, by, sm, rd);
@@ -594,11 +589,11 @@ template <int QT, int EPI, bool GROUPED, bool PACKED>
 __device__ __forceinline__ void lines_block(const GemmArgs &p, u32 id, uint8_t *ksm) {
     constexpr int NG = groups_per_line<QT>();
     constexpr bool SW = EPI == GE_SWIGLU;
-    constexpr int RT = 1; /* 32-row tiles (2 measured slower at 32 to 4096 rows) */
-    constexpr u32 CW = SW ? 32u : 64u, ROWS = 32u * RT, RB = QT == 4 ? 32u : 64u;
+    /* 32 rows (64 measured slower at 32 to 4096 rows) */
+    constexpr u32 CW = SW ? 32u : 64u, ROWS = 32u, RB = QT == 4 ? 32u : 64u;
     const u32 t = threadIdx.x, lane = t & 63u, wave = uni(t >> 6), r = lane & 31u, h = lane >> 5, nw = blockDim.x / 64u;
     u32 bx, by;
-    if (!tile_of(id, p.order, GROUPED ? (u32)*p.ntiles : p.nx, p.ny, bx, by)) return;
+    if (!tile_of(id, p.by_row != 0u, GROUPED ? (u32)*p.ntiles : p.nx, p.ny, bx, by)) return;
     const u32 n0 = by * CW;
     u32 e = 0, s0 = bx * ROWS, rows;
     if (GROUPED) {
@@ -622,14 +617,10 @@ __device__ __forceinline__ void lines_block(const GemmArgs &p, u32 id, uint8_t *
         vb[j] = PACKED ? 0u : row * rowb;
         srow[j] = (const unsigned short *)m.s + (GROUPED ? e * p.s_stride : 0) + (size_t)row * NT;
     }
-    u32 va[RT];
-#pragma unroll
-    for (int k = 0; k < RT; ++k) {
-        const u32 rr = min(32u * k + r, rows - 1u), ar = GROUPED ? (u32)p.a_idx[s0 + rr] : s0 + rr;
-        va[k] = ar * p.lda * 2u + 2u * b_koff<QT>(0u, h);
-    }
+    const u32 ar = GROUPED ? (u32)p.a_idx[s0 + min(r, rows - 1u)] : s0 + min(r, rows - 1u);
+    const u32 va = ar * p.lda * 2u + 2u * b_koff<QT>(0u, h);
     u32 bn[2][16], sn[2][NG], bc[2][16], sc[2][NG];
-    U4H8 an[4][RT], ac[4][RT];
+    U4H8 an[4], ac[4];
     /* line c of the lane's two weight rows: its half of every group (past the
      * row's end the last piece again) */
     auto load_b = [&](u32 c) {
@@ -659,17 +650,13 @@ __device__ __forceinline__ void lines_block(const GemmArgs &p, u32 id, uint8_t *
     auto load_a = [&](u32 s) {
         const uint8_t *base = (const uint8_t *)p.A + (size_t)s * 128u;
 #pragma unroll
-        for (u32 i = 0; i < 4; ++i)
-#pragma unroll
-            for (int k = 0; k < RT; ++k) an[i][k].u = *(const uint4 *)(base + (va[k] + 2u * b_koff<QT>(i, 0u)));
+        for (u32 i = 0; i < 4; ++i) an[i].u = *(const uint4 *)(base + (va + 2u * b_koff<QT>(i, 0u)));
     };
-    f32x16 acc[RT][2];
+    f32x16 acc[2];
 #pragma unroll
-    for (int k = 0; k < RT; ++k)
+    for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int x = 0; x < 16; ++x) acc[k][j][x] = 0.0f;
+        for (int x = 0; x < 16; ++x) acc[j][x] = 0.0f;
 
     if (wave < NCH) {
         load_b(wave);
@@ -689,9 +676,7 @@ __device__ __forceinline__ void lines_block(const GemmArgs &p, u32 id, uint8_t *
             const u32 s = c * NG + g;
             if (g > 0 && s >= NT) break;
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int k = 0; k < RT; ++k) ac[i][k] = an[i][k];
+            for (int i = 0; i < 4; ++i) ac[i] = an[i];
             if (g + 1 < NG) load_a(min(s + 1u, NT - 1u));
             if (g == 0 && more) load_b(c + nw);
             if (g + 1 == NG && more) load_a((c + nw) * NG);
@@ -703,83 +688,77 @@ __device__ __forceinline__ void lines_block(const GemmArgs &p, u32 id, uint8_t *
                     if (QT == 4) wv = dequant_q4(bc[j][4 * g + 2 * (i & 1)], bc[j][4 * g + 2 * (i & 1) + 1], (i & 2) != 0, sc[j][g]);
                     else if (QT == 3) wv = dequant_q8(bc[j][(8 * g + 2 * i) & 15], bc[j][(8 * g + 2 * i + 1) & 15], sc[j][g]);
                     else wv = operand_f16(bc[j][4 * i], bc[j][4 * i + 1], bc[j][4 * i + 2], bc[j][4 * i + 3]);
-#pragma unroll
-                    for (int k = 0; k < RT; ++k) acc[k][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wv, ac[i][k].v, acc[k][j], 0, 0, 0);
+                    acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wv, ac[i].v, acc[j], 0, 0, 0);
                 }
             }
         }
     }
 
     /* The wavefronts' partials are added in order, 8 columns of a row per
-     * thread and turn; 32 rows at a time.  Piece (j, q) of a plane: the four
-     * values of row r and half h at 16 (32 h + r). */
+     * thread and turn.  Piece (j, q) of a plane: the four values of row r and
+     * half h at 16 (32 h + r). */
     constexpr u32 CH = CW / 8u;
 #pragma unroll
-    for (int k = 0; k < RT; ++k) {
-        if (k > 0 && 32u * k >= rows) break;
-        if (k > 0) __syncthreads();
+    for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int q = 0; q < 4; ++q)
+            *(float4 *)(ksm + wave * KS_PLANE + (4u * j + q) * 1040u + 16u * lane) =
+                make_float4(acc[j][4 * q], acc[j][4 * q + 1], acc[j][4 * q + 2], acc[j][4 * q + 3]);
+    __syncthreads();
+    for (u32 it = t; it < 32u * CH; it += blockDim.x) {
+        const u32 row = it / CH, pc = it % CH, col = n0 + 8u * pc;
+        if (row >= rows || col >= p.N) continue;
+        const size_t orow = GROUPED ? (size_t)p.o_idx[s0 + row] : (size_t)(s0 + row);
+        U4H8 rs;
+        if (EPI == GE_F16 && p.res != nullptr) rs.u = *(const uint4 *)(p.res + orow * p.ldr + col);
+        if (EPI == GE_VISION) rs.u = *(const uint4 *)(p.bias + col);
+        float v[8], u[8];
+        auto sum = [&](u32 piece, float (&o)[8]) {
+            const uint8_t *src = ksm + piece * 1040u + 16u * row;
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
-                *(float4 *)(ksm + wave * KS_PLANE + (4u * j + q) * 1040u + 16u * lane) =
-                    make_float4(acc[k][j][4 * q], acc[k][j][4 * q + 1], acc[k][j][4 * q + 2], acc[k][j][4 * q + 3]);
-        __syncthreads();
-        for (u32 it = t; it < 32u * CH; it += blockDim.x) {
-            const u32 row = it / CH, pc = it % CH, rr = 32u * k + row, col = n0 + 8u * pc;
-            if (rr >= rows || col >= p.N) continue;
-            const size_t orow = GROUPED ? (size_t)p.o_idx[s0 + rr] : (size_t)(s0 + rr);
-            U4H8 rs;
-            if (EPI == GE_F16 && p.res != nullptr) rs.u = *(const uint4 *)(p.res + orow * p.ldr + col);
-            if (EPI == GE_VISION) rs.u = *(const uint4 *)(p.bias + col);
-            float v[8], u[8];
-            auto sum = [&](u32 piece, float (&o)[8]) {
-                const uint8_t *src = ksm + piece * 1040u + 16u * row;
-#pragma unroll
-                for (int x = 0; x < 8; ++x) o[x] = 0.0f;
-                for (u32 w = 0; w < nw; ++w) {
-                    const float4 a = *(const float4 *)(src + w * KS_PLANE), b = *(const float4 *)(src + w * KS_PLANE + 512u);
-                    o[0] += a.x;
-                    o[1] += a.y;
-                    o[2] += a.z;
-                    o[3] += a.w;
-                    o[4] += b.x;
-                    o[5] += b.y;
-                    o[6] += b.z;
-                    o[7] += b.w;
-                }
-            };
-            sum(pc, v);
-            if constexpr (SW) {
-                sum(pc + 4u, u);
-#pragma unroll
-                for (int x = 0; x < 8; ++x) v[x] = silu_p(v[x]) * u[x];
+            for (int x = 0; x < 8; ++x) o[x] = 0.0f;
+            for (u32 w = 0; w < nw; ++w) {
+                const float4 a = *(const float4 *)(src + w * KS_PLANE), b = *(const float4 *)(src + w * KS_PLANE + 512u);
+                o[0] += a.x;
+                o[1] += a.y;
+                o[2] += a.z;
+                o[3] += a.w;
+                o[4] += b.x;
+                o[5] += b.y;
+                o[6] += b.z;
+                o[7] += b.w;
             }
-            if constexpr (EPI == GE_F32) {
-                float4 *o = (float4 *)((float *)p.out + orow * p.ldo + col);
-                o[0] = make_float4(v[0], v[1], v[2], v[3]);
-                o[1] = make_float4(v[4], v[5], v[6], v[7]);
-                continue;
-            }
-            h16 *dst = (h16 *)p.out + orow * p.ldo + col;
-            if (EPI == GE_VISION && p.split != 0u) {
-                const u32 pj = col / p.split;
-                dst = (h16 *)(pj == 0u ? p.out : (pj == 1u ? p.out1 : p.out2)) + orow * p.split + (col - pj * p.split);
-            }
-            U4H8 o;
-            if constexpr (EPI == GE_VISION) {
-                with_act(p.act, [&](auto ACT) {
+        };
+        sum(pc, v);
+        if constexpr (SW) {
+            sum(pc + 4u, u);
 #pragma unroll
-                    for (int x = 0; x < 8; ++x) v[x] = vision_act<decltype(ACT)::value>(v[x] + (float)rs.h[x]);
-                });
-            }
-#pragma unroll
-            for (int x = 0; x < 8; ++x) {
-                if (EPI == GE_F16 && p.res != nullptr) v[x] += (float)rs.h[x];
-                o.h[x] = (h16)v[x];
-            }
-            *(uint4 *)dst = o.u;
+            for (int x = 0; x < 8; ++x) v[x] = silu_p(v[x]) * u[x];
         }
+        if constexpr (EPI == GE_F32) {
+            float4 *o = (float4 *)((float *)p.out + orow * p.ldo + col);
+            o[0] = make_float4(v[0], v[1], v[2], v[3]);
+            o[1] = make_float4(v[4], v[5], v[6], v[7]);
+            continue;
+        }
+        h16 *dst = (h16 *)p.out + orow * p.ldo + col;
+        if (EPI == GE_VISION && p.split != 0u) {
+            const u32 pj = col / p.split;
+            dst = (h16 *)(pj == 0u ? p.out : (pj == 1u ? p.out1 : p.out2)) + orow * p.split + (col - pj * p.split);
+        }
+        U4H8 o;
+        if constexpr (EPI == GE_VISION) {
+            with_act(p.act, [&](auto ACT) {
+#pragma unroll
+                for (int x = 0; x < 8; ++x) v[x] = vision_act<decltype(ACT)::value>(v[x] + (float)rs.h[x]);
+            });
+        }
+#pragma unroll
+        for (int x = 0; x < 8; ++x) {
+            if (EPI == GE_F16 && p.res != nullptr) v[x] += (float)rs.h[x];
+            o.h[x] = (h16)v[x];
+        }
+        *(uint4 *)dst = o.u;
     }
 }
 
@@ -801,7 +780,7 @@ dim3 tile_grid(GemmArgs &a, u32 row_tiles, u32 col_tiles, u32 qt, bool grouped) 
     a.nx = row_tiles;
     a.ny = col_tiles;
     const uint64_t wb = (uint64_t)a.N * a.K * (qt == UOCR_QT_F16 ? 4u : (qt == UOCR_QT_Q8 ? 2u : 1u)), ab = (uint64_t)a.M * a.K * 4u;
-    a.order = grouped || ab > wb ? GO_BY_ROW : GO_BY_COL;
+    a.by_row = grouped || ab > wb ? 1u : 0u;
     return dim3((row_tiles * col_tiles + 7u) / 8u * 8u);
 }
 

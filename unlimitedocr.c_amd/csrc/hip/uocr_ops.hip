@@ -344,11 +344,11 @@ extern "C" int uocr_op_gemm(uint32_t qtype, const void *w, const void *s, uint32
 /* Split-K partials of the vision linear: grown on demand, kept until the
  * process ends (outgrown buffers too, since captured graphs may reference
  * them; one current buffer per process, so concurrent calls are not
- * supported).  Only long-K GEMMs on grids under half a block per CU split K
- * (at least 4 K steps per split, at most 8 splits): the partials round trip
- * and the reduce launch cost more than the unsplit kernel elsewhere (257 x
- * 4096 -> 1024: 56 -> 20 us split; 640 x 1024 -> 3072: 28 us split against
- * 14-20 us unsplit). */
+ * supported).  Of the GEMMs on the general kernel, those with long K on grids
+ * under half a block per CU split K (at least 4 K steps per split, at most 8
+ * splits): the partials round trip and the reduce launch cost more than the
+ * unsplit kernel elsewhere (on that kernel 257 x 4096 -> 1024 Q8: 56 -> 17.5 us
+ * split; 640 x 1024 -> 3072: 28 us split against 14-20 unsplit). */
 static float *g_vision_part = nullptr;
 static size_t g_vision_part_bytes = 0;
 /* Guards the lazily allocated operator buffer (g_vision_part): held from the

@@ -7,9 +7,10 @@
  * real GEMMs [P x K] x [K x N]; the tiled kernels (uocr_gemm_tile.hip) and the
  * attention (uocr_attn_prefill.hip) have files of their own.  Here:
  *  - the launchers, which check a GEMM and choose its kernel;
- *  - k_gemm, the general GEMM for operands that are off 16-byte pieces (the
- *    operators accept them, the engine has none): 64 x 128 output tiles, K in
- *    64-column steps (one quantisation group), activations staged in LDS as
+ *  - k_gemm, the general GEMM: for operands off 16-byte pieces (the operators
+ *    accept them, the engine has none), and where it is the faster one (K split
+ *    over blocks, some vision linears).  64 x 128 output tiles, K in 64-column
+ *    steps (one quantisation group), activations staged in LDS as
  *    fp16, each wavefront dequantising its own 32 weight rows straight into
  *    MFMA operand registers as fp16(q * scale), the reference's prefill
  *    staging (gemm_q4.metal:48-55: half(float(q) * scale)), with fp32
@@ -35,10 +36,11 @@
 #ifndef GDEPTH
 #define GDEPTH 2 /* K steps in flight per GEMM block (2, 3 and 5 measured: 2 best on the SAM shapes, equal on the prefill) */
 #endif
-/* The SwiGLU GEMMs (two weight matrices) keep one K step in flight: 16
- * fewer registers take them from 2 to 3 wavefronts per SIMD (routed gate/up
- * 66.8 -> 62.4 us, dense gate/up 62.9 -> 60.8 us); the one-matrix GEMMs run
- * 4 per SIMD either way and lose with one step (dense down 44.4 -> 48.7 us). */
+/* The SwiGLU GEMMs (two weight matrices; here only off 16-byte pieces) keep one
+ * K step in flight: 16 fewer registers take them from 2 to 3 wavefronts per SIMD
+ * (932 rows on this kernel: routed gate/up 66.8 -> 62.4 us, dense gate/up 62.9 ->
+ * 60.8); the one-matrix GEMMs run 4 per SIMD either way and lose with one step
+ * (dense down, unsplit, 44.4 -> 48.7). */
 #ifndef GDEPTH_SWIGLU
 #define GDEPTH_SWIGLU 1
 #endif
@@ -114,13 +116,14 @@ __device__ __forceinline__ void b_dequant(const u32 (&w)[BPiece<QT>::NW], u32 sc
 #define UOCR_GEMM_BLDS 1
 #endif
 
-template <int QT, int EPI, bool GROUPED, int TMR>
+template <int QT, int EPI, bool GROUPED>
 __device__ __forceinline__ void gemm_body(GemmArgs p, u32 bx, u32 by, u32 bz) {
-    constexpr int AQ4 = TMR * (TK / 8) / PB; /* activation pieces (8 halves) per thread per K step */
-    static_assert(TMR % 32 == 0 && TMR <= PB && AQ4 * PB == TMR * (TK / 8), "tile rows");
+    constexpr int AQ4 = TM * (TK / 8) / PB; /* activation pieces (8 halves) per thread per K step */
+    static_assert(TM % 32 == 0 && TM <= PB && AQ4 * PB == TM * (TK / 8), "tile rows");
     constexpr int NMAT = EPI == GE_SWIGLU ? 2 : 1;
     constexpr int GD = EPI == GE_SWIGLU ? GDEPTH_SWIGLU : GDEPTH; /* K steps in flight */
-    /* f16 with one weight matrix: the block loads each K step's raw weight
+    /* (the SAM and CLIP figures are of this kernel at shapes that the tiled
+     * kernels run now) f16 with one weight matrix: the block loads each K step's raw weight
      * tile with eight lanes per row (whole 128-byte row pieces) into LDS, and
      * each wavefront reads its 32 rows back in the MFMA operand layout; loads
      * of one row per lane touched a cache line per lane (SAM lin1 with fp16
@@ -133,8 +136,8 @@ __device__ __forceinline__ void gemm_body(GemmArgs p, u32 bx, u32 by, u32 bz) {
     constexpr u32 LDB = RB + 16u;            /* padded LDS row (bytes) */
     constexpr u32 CPR = RB / 16u;            /* 16-byte pieces per row */
     __shared__ __attribute__((aligned(16))) uint8_t bsm[BL ? 2u * TN * LDB : 16u];
-    __shared__ __attribute__((aligned(16))) h16 as[2][TMR * LDA];
-    __shared__ int32_t arow[TMR], orow[TMR];
+    __shared__ __attribute__((aligned(16))) h16 as[2][TM * LDA];
+    __shared__ int32_t arow[TM], orow[TM];
     const u32 t = threadIdx.x, lane = t & 63u, wave = t >> 6, hf = lane >> 5;
     u32 n0 = by * TN, rows = p.M, e = 0, s0 = 0;
     if (GROUPED) {
@@ -142,40 +145,33 @@ __device__ __forceinline__ void gemm_body(GemmArgs p, u32 bx, u32 by, u32 bz) {
         e = (u32)p.tile_e[bx];
         s0 = (u32)p.tile_s0[bx];
         rows = (u32)p.tile_s1[bx] - s0;
-        if (t < TMR) {
+        if (t < TM) {
             const u32 s = s0 + min(t, rows - 1u);
             arow[t] = p.a_idx[s];
             orow[t] = p.o_idx[s];
         }
     } else {
-        s0 = bx * TMR;
-        rows = min((u32)TMR, p.M - s0);
-        if (t < TMR) {
+        s0 = bx * TM;
+        rows = min((u32)TM, p.M - s0);
+        if (t < TM) {
             arow[t] = (int32_t)(s0 + min(t, rows - 1u));
             orow[t] = arow[t];
         }
     }
-    uocr_qmat W0 = p.W[0], W1 = p.W[1];
-    u32 nbase = 0;
-    if (p.nseg != 0u) {
-        const u32 sgi = n0 / p.nseg;
-        W0 = p.W[sgi];
-        nbase = sgi * p.nseg;
-    }
-    const u32 nmax = (p.nseg != 0u ? p.nseg : p.N);
+    const uocr_qmat W0 = p.W[0], W1 = p.W[1];
     const uint8_t *wp[2] = {(const uint8_t *)W0.w + (GROUPED ? e * p.w_stride : 0),
                             NMAT == 2 ? (const uint8_t *)W1.w + (GROUPED ? e * p.w_stride : 0) : nullptr};
     const h16 *sp[2] = {(const h16 *)W0.s + (GROUPED ? e * p.s_stride : 0),
                         NMAT == 2 ? (const h16 *)W1.s + (GROUPED ? e * p.s_stride : 0) : nullptr};
     /* this lane's weight row (clamped; columns past N are not stored) */
-    const u32 nrow = min(n0 - nbase + 32u * wave + (lane & 31u), nmax - 1u);
+    const u32 nrow = min(n0 + 32u * wave + (lane & 31u), p.N - 1u);
     __syncthreads();
 
-    f32x16 acc[NMAT][TMR / 32];
+    f32x16 acc[NMAT][TM / 32];
 #pragma unroll
     for (int m = 0; m < NMAT; ++m)
 #pragma unroll
-        for (int j = 0; j < TMR / 32; ++j)
+        for (int j = 0; j < TM / 32; ++j)
 #pragma unroll
             for (int i = 0; i < 16; ++i) acc[m][j][i] = 0.0f;
 
@@ -193,8 +189,8 @@ __device__ __forceinline__ void gemm_body(GemmArgs p, u32 bx, u32 by, u32 bz) {
     u32 kb[GD][NMAT][BPiece<QT>::NW], ks[GD][NMAT];
     extern __shared__ __attribute__((aligned(16))) unsigned short ssc[];
     const bool scl = QT != 1 && p.sc_lds != 0u;
-    const u32 lrow0 = n0 - nbase, nvalid = min((u32)TN, nmax - lrow0);
-    const u32 lrow = nrow - lrow0; /* this lane's row within the block's scale rows */
+    const u32 nvalid = min((u32)TN, p.N - n0);
+    const u32 lrow = nrow - n0; /* this lane's row within the block's scale rows */
     /* this thread's two activation rows, resolved once */
     const h16 *arp[AQ4];
 #pragma unroll
@@ -208,7 +204,7 @@ __device__ __forceinline__ void gemm_body(GemmArgs p, u32 bx, u32 by, u32 bz) {
 #pragma unroll
         for (int v = 0; v < BPiece<QT>::NV; ++v) {
             const u32 pidx = t + v * PB, r = pidx / CPR, c = pidx % CPR;
-            bsrc[v] = wp[0] + (size_t)min(lrow0 + r, nmax - 1u) * rowbytes + 16u * c;
+            bsrc[v] = wp[0] + (size_t)min(n0 + r, p.N - 1u) * rowbytes + 16u * c;
         }
     }
     auto issue = [&](auto D, u32 st) {
@@ -291,7 +287,7 @@ __device__ __forceinline__ void gemm_body(GemmArgs p, u32 bx, u32 by, u32 bz) {
 #pragma unroll
         for (u32 i = 0; i < 4; ++i) {
 #pragma unroll
-            for (int j = 0; j < TMR / 32; ++j) {
+            for (int j = 0; j < TM / 32; ++j) {
                 U4H8 a;
                 a.u = *(const uint4 *)(ab + (32u * j + (lane & 31u)) * LDA + b_koff<QT>(i, hf));
 #pragma unroll
@@ -303,11 +299,11 @@ __device__ __forceinline__ void gemm_body(GemmArgs p, u32 bx, u32 by, u32 bz) {
     };
     static_for<GD>([&](auto D) { issue(D, min((u32)decltype(D)::value, NS - 1u)); });
     if (scl) {
-        /* after the first steps' loads are in flight; rows past nmax are not
+        /* after the first steps' loads are in flight; rows past p.N are not
          * loaded (their lanes read the last valid row, nrow is clamped) */
 #pragma unroll
         for (int m = 0; m < NMAT; ++m) {
-            const unsigned short *src = (const unsigned short *)sp[m] + (size_t)lrow0 * NT;
+            const unsigned short *src = (const unsigned short *)sp[m] + (size_t)n0 * NT;
             unsigned short *dst = ssc + m * TN * NT;
             const u32 cnt = nvalid * NT;
             if ((((uintptr_t)src) & 15u) == 0u && cnt % 8u == 0u) {
@@ -347,7 +343,7 @@ __device__ __forceinline__ void gemm_body(GemmArgs p, u32 bx, u32 by, u32 bz) {
     }
     const u32 act = p.act;
 #pragma unroll
-    for (int j = 0; j < TMR / 32; ++j) {
+    for (int j = 0; j < TM / 32; ++j) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             const u32 r = 32u * j + 8u * (i / 4) + 4u * hf + (i % 4);
@@ -373,9 +369,9 @@ __device__ __forceinline__ void gemm_body(GemmArgs p, u32 bx, u32 by, u32 bz) {
     }
 }
 
-template <int QT, int EPI, bool GROUPED, int TMR>
+template <int QT, int EPI, bool GROUPED>
 __global__ __launch_bounds__(PB) void k_gemm(GemmArgs p) {
-    gemm_body<QT, EPI, GROUPED, TMR>(p, blockIdx.x, blockIdx.y, blockIdx.z);
+    gemm_body<QT, EPI, GROUPED>(p, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
 /* cs[64 t + d] = (cos, sin)(t * f[d]) for the P prompt tokens. */
@@ -823,21 +819,16 @@ static bool pmat_ok(uocr_qmat m) {
     return m.w != nullptr && pq_ok(m.qtype) && (m.qtype == UOCR_QT_F16 || m.s != nullptr);
 }
 
-template <int EPI, bool GROUPED, int TMR>
-static void gemm_dispatch_tm(hipStream_t st, u32 qt, const GemmArgs &a, dim3 grid, size_t shm) {
-    switch (qt) {
-        case UOCR_QT_F16: hipLaunchKernelGGL((k_gemm<1, EPI, GROUPED, TMR>), grid, dim3(PB), 0, st, a); break;
-        case UOCR_QT_Q8: hipLaunchKernelGGL((k_gemm<3, EPI, GROUPED, TMR>), grid, dim3(PB), shm, st, a); break;
-        default: hipLaunchKernelGGL((k_gemm<4, EPI, GROUPED, TMR>), grid, dim3(PB), shm, st, a); break;
-    }
-}
-
 template <int EPI, bool GROUPED>
 static void gemm_dispatch(hipStream_t st, u32 qt, GemmArgs a, dim3 grid) {
     const u32 nm = EPI == GE_SWIGLU ? 2u : 1u, nt = a.K / TK;
     a.sc_lds = qt != UOCR_QT_F16 && nm * nt <= SC_LDS_STEPS ? 1u : 0u;
     const size_t shm = a.sc_lds ? (size_t)nm * TN * nt * sizeof(unsigned short) : 0;
-    gemm_dispatch_tm<EPI, GROUPED, TM>(st, qt, a, grid, shm);
+    switch (qt) {
+        case UOCR_QT_F16: hipLaunchKernelGGL((k_gemm<1, EPI, GROUPED>), grid, dim3(PB), 0, st, a); break;
+        case UOCR_QT_Q8: hipLaunchKernelGGL((k_gemm<3, EPI, GROUPED>), grid, dim3(PB), shm, st, a); break;
+        default: hipLaunchKernelGGL((k_gemm<4, EPI, GROUPED>), grid, dim3(PB), shm, st, a); break;
+    }
 }
 
 /* Splits of K over blocks for the prompt's O projection (K = 1280) and layer 0's
@@ -926,7 +917,7 @@ extern "C" int uocr_gemm_splits_itself(int epi, const uocr_gemm_desc *d) {
 }
 
 extern "C" hipError_t uocr_launch_gemm(hipStream_t st, int epi, const uocr_gemm_desc *d) {
-    if (!gemm_desc_ok(epi, d)) return hipErrorInvalidValue;
+    if (!gemm_desc_ok(epi, d) || d->nseg != 0u) return hipErrorInvalidValue;
     const bool grouped = d->tile_e != nullptr;
     GemmArgs a = gemm_args(d);
     const dim3 grid(grouped ? d->max_tiles : (d->M + TM - 1u) / TM, (d->N + TN - 1u) / TN);
@@ -948,12 +939,8 @@ extern "C" hipError_t uocr_launch_gemm(hipStream_t st, int epi, const uocr_gemm_
     const bool fused = split && want_norm, splittable = fused || (split && epi == UOCR_GEMM_VISION && d->N % 4u == 0u && d->split % 4u == 0u);
     if (!grouped && !fused && uocr_gemm_tile_fits(epi, qt, a)) {
         const hipError_t e = uocr_gemm_tile_plain(st, epi, qt, a);
-        if (e != hipSuccess || !want_norm) return e;
-        hipLaunchKernelGGL(k_rows_rmsnorm, dim3((d->M + 3u) / 4u), dim3(PB), 0, st, (const h16 *)d->out,
-                           (const h16 *)d->norm_w, d->M, (h16 *)d->norm_out);
-        return hipGetLastError();
-    }
-    if (splittable) {
+        if (e != hipSuccess) return e;
+    } else if (splittable) {
         /* split-K: blockIdx.z takes K steps [z*kst, (z+1)*kst) into an fp32
          * partial plane of part, then one ordered reduce applies the
          * epilogue */
@@ -983,10 +970,10 @@ extern "C" hipError_t uocr_launch_gemm(hipStream_t st, int epi, const uocr_gemm_
     } else {
         if (grouped) gemm_dispatch<GE_F16, true>(st, qt, a, grid);
         else gemm_dispatch<GE_F16, false>(st, qt, a, grid);
-        if (want_norm) {
-            hipLaunchKernelGGL(k_rows_rmsnorm, dim3((d->M + 3u) / 4u), dim3(PB), 0, st, (const h16 *)d->out,
-                               (const h16 *)d->norm_w, d->M, (h16 *)d->norm_out);
-        }
+    }
+    if (want_norm) {
+        hipLaunchKernelGGL(k_rows_rmsnorm, dim3((d->M + 3u) / 4u), dim3(PB), 0, st, (const h16 *)d->out,
+                           (const h16 *)d->norm_w, d->M, (h16 *)d->norm_out);
     }
     return hipGetLastError();
 }
