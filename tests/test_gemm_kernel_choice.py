@@ -49,3 +49,13 @@ def test_bad_arguments(kernel_of):
     for args in ((2, 4, 128, 128), (Q4, 0, 128, 128), (Q4, 4, 128, 100), (Q4, 4, 128, 128, True, 3)):
         with pytest.raises(ValueError):
             kernel_of(*args)
+
+
+def test_value_tests_reach_every_kernel(kernel_of):
+    """The shapes of the value tests are on the kernels that their comments name."""
+    import test_gpu_gemm_tiles as t
+    want = ["large", "large", "mid", "mid", "mid_k4", "narrow", "narrow", "lines", "lines", "lines", "lines"]
+    for q in (F16, Q8, Q4):
+        assert [kernel_of(q, *s) for s in t.SHAPES] == want
+        for m, n, k, act, _, kernel in t.VISION_SHAPES:
+            assert kernel_of(q, m, n, k, True, act) == kernel

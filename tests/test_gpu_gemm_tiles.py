@@ -9,6 +9,8 @@ unit, 2^-11 relative, or half the subnormal spacing) plus K fp32 additions of
 products no larger than the sum of their magnitudes."""
 from __future__ import annotations
 
+import math
+
 import numpy as np
 import pytest
 
@@ -103,6 +105,98 @@ def test_vision_linear_misaligned_rows(gpu, qtype, m, n, k):
     uocr.sync()
     got = dy.download(np.float16, m * n).reshape(m, n)
     check_rows(got, x, operand_values(qtype, w, s), np.tile(bias.astype(np.float64), (m, 1)))
+
+
+def activated(x, act):
+    """(value, largest slope) of the vision activations in float64."""
+    if act == 1:
+        return x / (1 + np.exp(-1.702 * x)), 1.1
+    if act == 2:
+        return 0.5 * x * (1 + np.vectorize(math.erf)(x / math.sqrt(2))), 1.13
+    return x, 1.0
+
+
+# m, n, k, activation, split, kernel: every kernel with an epilogue of its own,
+# ragged rows and columns, K groups of 13, 13, 13 and 10 steps (mid_k4), 8 splits
+# of 5 steps and fewer in the last (general)
+VISION_SHAPES = [(2561, 2568, 128, 2, 0, "large"), (2945, 2064, 64, 1, 688, "large"), (1090, 776, 192, 1, 0, "mid"), (1300, 648, 64, 2, 216, "mid"),
+                 (780, 1032, 3136, 1, 0, "mid_k4"), (780, 1032, 3136, 0, 344, "mid_k4"), (330, 1032, 3136, 2, 0, "narrow"), (95, 200, 448, 2, 0, "lines"),
+                 (33, 72, 192, 1, 24, "lines"), (100, 256, 2368, 2, 0, "general"), (70, 264, 2368, 1, 88, "general")]
+
+
+@pytest.mark.parametrize("qtype", [1, 3, 4])
+@pytest.mark.parametrize("m,n,k,act,split,kernel", VISION_SHAPES)
+def test_vision_tile_edges(gpu, qtype, m, n, k, act, split, kernel):
+    """The bound of check_rows through the activation's slope, and 2^-21 of the
+    argument for the hardware exp2 and reciprocal and the erf polynomial (1.5e-7
+    absolute, times half the argument)."""
+    uocr = gpu
+    assert uocr.op_gemm_kernel(qtype, m, n, k, True, act) == kernel
+    rng = np.random.default_rng(m + n + k + qtype)
+    w, s = weights_for(qtype, rng, n, k)
+    x, bias = rand_f16(rng, (m, k)), rand_f16(rng, (n,))
+    of = uocr.DeviceBuffer.of
+    dw, ds, dx, db = of(w), None if s is None else of(s), of(x), of(bias)
+    width = split or n
+    outs = [of(np.full((m, width), 7, np.float16)) for _ in range(3 if split else 1)]
+    uocr.op_vision_linear(qtype, dw, ds, db, m, k, n, act, split, dx, *outs)
+    uocr.sync()
+    got = np.hstack([o.download(np.float16).reshape(m, width) for o in outs]).astype(np.float64)
+    rows = np.unique(np.concatenate([np.arange(min(m, 40)), np.arange(max(0, m - 40), m), rng.integers(0, m, 40)]))
+    wv, xd = operand_values(qtype, w, s), x[rows].astype(np.float64)
+    pre = xd @ wv.T + bias.astype(np.float64)
+    mag = np.abs(xd) @ np.abs(wv).T + np.abs(bias.astype(np.float64))
+    ref, slope = activated(pre, act)
+    bound = np.abs(ref) * 2.0**-11 + 2.0**-25 + slope * mag * (k + 1) * 2.0**-24 + (np.abs(pre) * 2.0**-21 if act else 0.0)
+    err = np.abs(got[rows] - ref)
+    assert (err <= bound).all(), (float((err / bound).max()), np.argwhere(err > bound)[:4].tolist())
+
+
+def test_vision_linear_block_split_in_a_graph(gpu):
+    """K split over blocks under capture.  The first capture needs more partials
+    than any call of this process has made the library allocate (33 MB), so it
+    holds the unsplit kernel; after an eager call, which grows the buffer, it
+    holds the split and its reduce and every replay equals the eager result."""
+    uocr = gpu
+    m, n, k, qtype = 1984, 508, 2048, 3  # 124 tiles, 8 splits; rows off 16-byte pieces
+    rng = np.random.default_rng(9)
+    w, s = weights_for(qtype, rng, n, k)
+    x, bias = rand_f16(rng, (m, k)), rand_f16(rng, (n,))
+    of = uocr.DeviceBuffer.of
+    dw, ds, dx, db, dy = of(w), of(s), of(x), of(bias), uocr.DeviceBuffer(m * n * 2)
+    rows = np.arange(0, m, 37)
+    wv, add = operand_values(qtype, w, s), np.tile(bias.astype(np.float64), (rows.size, 1))
+
+    def call():
+        uocr.op_vision_linear(qtype, dw, ds, db, m, k, n, 0, 0, dx, dy)
+
+    def result():
+        uocr.sync()
+        return dy.download(np.uint16).reshape(m, n)
+
+    def captured():
+        with uocr.Capture() as g:
+            call()
+        out = []
+        try:
+            for _ in range(3):
+                dy.zero()
+                g.replay(1)
+                out.append(result())
+        finally:
+            g.release()
+        assert all(np.array_equal(out[0], o) for o in out)
+        return out[0]
+
+    first = captured()
+    dy.zero()
+    call()
+    eager = result()
+    second = captured()
+    for got in (first, eager):
+        check_rows(got.view(np.float16)[rows], x[rows], wv, add)
+    assert np.array_equal(second, eager)
+    assert not np.array_equal(first, eager)  # another order of the sums: the first was not the split
 
 
 def routed_rows(rng, counts, P):

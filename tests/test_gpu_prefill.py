@@ -137,11 +137,11 @@ def test_batched_and_token_prefill_agree(gpu):
 
 
 def test_long_prompt_batched_and_token_prefill_agree(gpu):
-    """A 1,450-row prompt: 8,700 routed (token, expert) pairs, more than the
-    8,192 the bucket build keeps in registers, so its looped path runs; 23
-    query tiles of the split flash attention (key chunks of 7 tiles).  The
-    MFMA prefill and the per-position prefill agree on the first step's
-    winning score within the fp16 tolerance."""
+    """A 1,450-row prompt: 8,700 routed (token, expert) pairs (24 per thread of
+    the bucket build instead of 8), the Q | K | V projection with RoPE on large
+    tiles, attention with its keys split over four wavefronts.  The MFMA prefill
+    and the per-position prefill agree on the first step's winning score within
+    the fp16 tolerance."""
     uocr = gpu
     m = model(uocr, 3)
     rng = np.random.default_rng(31)
@@ -160,11 +160,11 @@ def test_long_prompt_batched_and_token_prefill_agree(gpu):
 # (4096 tokens, 768 wide: qkv 2304 split 768, lin1 3072 + GELU, lin2), the
 # CLIP-L view (257 tokens, 1024 wide: qkv split 1024, fc1 4096 + QuickGELU,
 # fc2), the projector (2048 -> 1280), the Q4 and fp16 kernels, and ragged
-# tiles (m not a multiple of 64, n not a multiple of 128).  Long-K GEMMs on
-# grids of fewer than 128 tiles split K (CLIP fc2; 37 K steps in 4 splits of
-# 10, 10, 10 and 7 in the 2368-wide case).  n = 100 with k = 192 leaves the
-# block's scale region at 300 halves, which the LDS preload copies 2 bytes at
-# a time instead of 16.
+# tiles (m not a multiple of 64, n not a multiple of 128).  The 2368-wide case
+# takes the general kernel and splits K there (37 steps in 8 splits of 5, the
+# last of 2).  n = 100 takes it too, rows not being whole 16-byte pieces; with
+# k = 192 the block's scale region is 300 halves, which the LDS preload copies
+# 2 bytes at a time instead of 16.
 VISION_CASES = [
     (3, 4096, 768, 2304, 0, 768), (3, 4096, 768, 3072, 2, 0), (3, 4096, 3072, 768, 0, 0),
     (3, 257, 1024, 3072, 0, 1024), (3, 257, 1024, 4096, 1, 0), (3, 257, 4096, 1024, 0, 0),
@@ -214,8 +214,9 @@ def test_vision_linear_rejects_bad_arguments(gpu):
 
 
 def test_vision_linear_split_k_in_a_graph(gpu, oracle):
-    """The CLIP fc2 shape (split K, partials reduced by a second kernel)
-    captured into a hipGraph: every replay equals the eager call."""
+    """The CLIP fc2 shape (K split over the wavefronts of a block) captured into
+    a hipGraph: every replay equals the eager call.  K split over blocks:
+    test_vision_linear_block_split_in_a_graph."""
     uocr = gpu
     rng = np.random.default_rng(5)
     m, k, n = 257, 4096, 1024
