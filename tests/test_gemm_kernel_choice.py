@@ -14,7 +14,8 @@ PLAIN = [
     (F16, 500, 1280, 6848, "mid_k4"), (Q4, 500, 1280, 6848, "mid_k4"), (Q4, 384, 1280, 6848, "narrow"), (F16, 2, 1280, 6848, "narrow"),
     (Q4, 932, 1280, 1280, "mid"), (Q8, 500, 1280, 1280, "mid"), (F16, 400, 1280, 1280, "mid"), (Q4, 500, 1280, 1280, "lines"),
     (Q4, 640, 1280, 1280, "mid"), (Q8, 384, 1280, 1280, "lines"), (F16, 384, 1280, 1280, "narrow"), (F16, 257, 1280, 1024, "lines"),
-    (Q4, 33, 1280, 1792, "lines"), (Q4, 70, 132, 192, "general"),
+    (Q4, 3264, 1280, 1280, "mid"), (Q4, 3265, 1280, 1280, "general"), (Q4, 4864, 1280, 6848, "general"), (Q4, 4865, 1280, 1280, "large"),
+    (Q8, 3265, 1280, 1280, "large"), (F16, 3265, 1280, 1280, "large"), (Q4, 33, 1280, 1792, "lines"), (Q4, 70, 132, 192, "general"),
 ]
 # qtype, m, n, k, act, kernel
 VISION = [
@@ -54,8 +55,8 @@ def test_bad_arguments(kernel_of):
 def test_value_tests_reach_every_kernel(kernel_of):
     """The shapes of the value tests are on the kernels that their comments name."""
     import test_gpu_gemm_tiles as t
-    want = ["large", "large", "mid", "mid", "mid_k4", "narrow", "narrow", "lines", "lines", "lines", "lines"]
+    rest = ["mid", "mid", "mid_k4", "narrow", "narrow", "lines", "lines", "lines", "lines", "large", "large"]
     for q in (F16, Q8, Q4):
-        assert [kernel_of(q, *s) for s in t.SHAPES] == want
+        assert [kernel_of(q, *s) for s in t.SHAPES] == (["general"] * 2 if q == Q4 else ["large"] * 2) + rest
         for m, n, k, act, _, kernel in t.VISION_SHAPES:
             assert kernel_of(q, m, n, k, True, act) == kernel

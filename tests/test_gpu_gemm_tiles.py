@@ -45,9 +45,10 @@ def check_rows(got, x, wv, add):
 # m x n x k: large tiles (full, ragged rows and columns, the shortest K), 64 x
 # 128 tiles with K in two groups (one step: the second group is empty; an odd
 # number of steps), K in four groups, 32 x 64 tiles with K in eight groups, and
-# K by weight lines (1 row, 1 column piece, a last line with 1, 2 or 3 groups)
+# K by weight lines (1 row, 1 column piece, a last line with 1, 2 or 3 groups);
+# the last two are the first two with a grid on which Q4 takes the large tiles too
 SHAPES = [(2561, 2048, 64), (2433, 2056, 320), (1300, 648, 64), (1090, 776, 192), (700, 1000, 4160), (130, 520, 3136),
-          (64, 1280, 3072), (1, 8, 64), (33, 72, 192), (95, 200, 448), (32, 64, 832)]
+          (64, 1280, 3072), (1, 8, 64), (33, 72, 192), (95, 200, 448), (32, 64, 832), (3073, 2048, 64), (2945, 2056, 320)]
 
 
 @pytest.mark.parametrize("qtype", [1, 3, 4])

@@ -150,9 +150,11 @@ struct GemmArgs {
     u32 nx, ny, by_row;  /* row tiles, column tiles; each XCD takes a run of row (else column) tiles */
 };
 
-/* The kernels of uocr_gemm_tile.hip: whether a plain GEMM's operands and sizes
- * fit them (16-byte aligned rows, 32-bit offsets), and its launch. */
+/* The kernels of uocr_gemm_tile.hip: whether a GEMM's operands and sizes fit
+ * them (16-byte aligned rows, 32-bit offsets), whether a plain one takes them
+ * (fits, and the general kernel is not the faster one), and its launch. */
 bool uocr_gemm_tile_fits(int epi, u32 qt, const GemmArgs &a);
+bool uocr_gemm_tile_takes(int epi, u32 qt, const GemmArgs &a);
 /* Whether a plain fp16 GEMM with fp32 output can take the router's half of uocr_gemm_tile_router. */
 bool uocr_gemm_router_fits(const GemmArgs &a);
 hipError_t uocr_gemm_tile_plain(hipStream_t st, int epi, u32 qt, const GemmArgs &a);

@@ -856,10 +856,16 @@ hipError_t plain_lines(hipStream_t st, int epi, u32 qt, const GemmArgs &a) {
  *  - with long sums on so few rows that its K splits are what fills the CUs, and,
  *    for quantised weights, between a narrow block per CU and 100 mid tiles;
  *  - with Q4 weights and an activation at up to one and a half rounds: its
- *    weights skip LDS and all its wavefronts share the epilogue.
+ *    weights skip LDS and all its wavefronts share the epilogue;
+ * and for plain Q4 GEMMs from 513 to 768 mid tiles, where three of its blocks fit
+ * a CU and large tiles leave a quarter of the CUs and more idle: 1-6% over K from
+ * 64 to 6848; above, in its second round, it is 10-25% slower from K = 256 on.
  * Measured (us): general / large / mid, K in 2 / in 4 / narrow, K in 8 / lines
  *   Q8   3500 x 1280 x 6848   123  /  97  / 118  / 128  / 200  / 229    550 mid
  *   Q8   2000 x 1280 x 6848   78.7 / 93.9 / 65.8 / 85.2 / 113  / 130    320
+ *   Q4   3584 x 1280 x 1280   23.7 / 24.4                               560
+ *   Q4   3600 x 1280 x 6848   114  / 118     (in a prompt)              570
+ *   Q4   4928 x 1280 x 1280   33.9 / 27.3                               770
  *   Q8    932 x 1280 x 6848   68.9 / 94.5 / 46.9 / 41.5                 150
  *   F16   500 x 1280 x 6848   52.3 / 92.4 / 45.6 / 39.9 / 43.1 / 74.5   320 narrow
  *   Q8    257 x 1280 x 6848   67.5 / 94.7 / 46.3 / 41.5 / 23.4 / 28.3   180
@@ -884,6 +890,7 @@ int choose(int epi, u32 qt, u32 M, u32 N, u32 K, u32 act) {
         if (K >= 2048u && (narrow < (qt == UOCR_QT_Q4 ? 128u : 100u) || (qt != UOCR_QT_F16 && narrow > 256u && mid < 100u))) return UOCR_GEMM_KERNEL_GENERAL;
         if (qt == UOCR_QT_Q4 && act != UOCR_VISION_ACT_NONE && K <= 1024u && mid > 256u && mid <= 768u) return UOCR_GEMM_KERNEL_GENERAL;
     }
+    if (epi == GE_F16 && qt == UOCR_QT_Q4 && mid > 512u && mid <= 768u) return UOCR_GEMM_KERNEL_GENERAL;
     if (mid > 512u) return UOCR_GEMM_KERNEL_LARGE;
     if (narrow <= 256u) return K >= (qt == UOCR_QT_F16 ? 1280u : 3072u) ? UOCR_GEMM_KERNEL_NARROW : UOCR_GEMM_KERNEL_LINES;
     if (qt == UOCR_QT_Q4 && K < 3072u && narrow <= 384u) return UOCR_GEMM_KERNEL_LINES;
@@ -896,10 +903,13 @@ bool uocr_gemm_tile_fits(int epi, u32 qt, const GemmArgs &a) {
     const uint64_t rowb = qt == UOCR_QT_Q4 ? a.K / 2u : (qt == UOCR_QT_Q8 ? a.K : 2ull * a.K), lim = 1ull << 32;
     uintptr_t al = (uintptr_t)a.A | (uintptr_t)a.W[0].w | (epi == GE_SWIGLU ? (uintptr_t)a.W[1].w : 0u);
     /* a plain fp32 GEMM is the router's: its sums keep their order (RouterHalf, or the general kernel) */
-    if (epi == GE_VISION && choose(epi, qt, a.M, a.N, a.K, a.act) == UOCR_GEMM_KERNEL_GENERAL) return false;
     const bool known = epi == GE_F16 || (epi == GE_F32 && a.tile_e != nullptr) || epi == GE_SWIGLU || epi == GE_VISION;
     return a.vec != 0u && known && a.nseg == 0u && al % 16u == 0u &&
            (uint64_t)a.M * a.lda * 2u < lim && (uint64_t)a.M * a.ldr * 2u < lim && a.N * rowb < lim && (!a.packed || a.N % 32u == 0u);
+}
+
+bool uocr_gemm_tile_takes(int epi, u32 qt, const GemmArgs &a) {
+    return uocr_gemm_tile_fits(epi, qt, a) && choose(epi, qt, a.M, a.N, a.K, a.act) != UOCR_GEMM_KERNEL_GENERAL;
 }
 
 bool uocr_gemm_router_fits(const GemmArgs &a) {

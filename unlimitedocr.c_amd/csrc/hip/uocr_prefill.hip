@@ -913,7 +913,7 @@ static GemmArgs gemm_args(const uocr_gemm_desc *d) {
 }
 
 extern "C" int uocr_gemm_splits_itself(int epi, const uocr_gemm_desc *d) {
-    return d->tile_e == nullptr && uocr_gemm_tile_fits(epi, d->W[0].qtype, gemm_args(d));
+    return d->tile_e == nullptr && uocr_gemm_tile_takes(epi, d->W[0].qtype, gemm_args(d));
 }
 
 extern "C" hipError_t uocr_launch_gemm(hipStream_t st, int epi, const uocr_gemm_desc *d) {
@@ -937,7 +937,7 @@ extern "C" hipError_t uocr_launch_gemm(hipStream_t st, int epi, const uocr_gemm_
     }
     if (grouped && d->tile_rows != 0u) return uocr_gemm_tile_grouped(st, epi, qt, a, d->pairs, d->tile_rows);
     const bool fused = split && want_norm, splittable = fused || (split && epi == UOCR_GEMM_VISION && d->N % 4u == 0u && d->split % 4u == 0u);
-    if (!grouped && !fused && uocr_gemm_tile_fits(epi, qt, a)) {
+    if (!grouped && !fused && uocr_gemm_tile_takes(epi, qt, a)) {
         const hipError_t e = uocr_gemm_tile_plain(st, epi, qt, a);
         if (e != hipSuccess) return e;
     } else if (splittable) {
