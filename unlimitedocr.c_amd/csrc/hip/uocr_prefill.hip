@@ -9,9 +9,9 @@
  *  - the launchers, which check a GEMM and choose its kernel;
  *  - k_gemm, the general GEMM: for operands off 16-byte pieces (the operators
  *    accept them, the engine has none), and where it is the faster one (K split
- *    over blocks, some vision linears).  64 x 128 output tiles, K in 64-column
- *    steps (one quantisation group), activations staged in LDS as
- *    fp16, each wavefront dequantising its own 32 weight rows straight into
+ *    over blocks, some vision linears and Q4 projections).  64 x 128 output
+ *    tiles, K in 64-column steps (one quantisation group), activations staged
+ *    in LDS as fp16, each wavefront dequantising its own 32 weight rows straight into
  *    MFMA operand registers as fp16(q * scale), the reference's prefill
  *    staging (gemm_q4.metal:48-55: half(float(q) * scale)), with fp32
  *    accumulation by v_mfma_f32_32x32x16_f16.  Epilogues: fp16 store with
